@@ -191,7 +191,8 @@ int rusty_hip_resident_generate(const int32_t *prompt, uint32_t n_prompt, uint32
                                 float repeat_penalty, int32_t *out_tokens, float *logits_out);
 /* forward_prefill_batch (src/model.rs:9917-10090): advances the KV cache over
  * tokens[0..n_tokens) at positions start_pos.. without computing logits, in
- * chunks (512 tokens; RUSTY_HIP_PREFILL_CHUNK, 64..2048) that run each weight matrix once per chunk on
+ * chunks (512 tokens, 1024 for a gpt-oss decoder whose attention scratch stays
+ * within 8 GB; RUSTY_HIP_PREFILL_CHUNK, 64..2048) that run each weight matrix once per chunk on
  * the matrix cores.  Needs the device embedding (set_embedding) and a model
  * that standard_prefill_batchable (:9869-9887) accepts: every projection
  * Q4_K or Q6_K, widths multiples of 256; start_pos + n_tokens <= storage_len.
@@ -207,10 +208,10 @@ int rusty_hip_resident_prefill(const int32_t *tokens, uint32_t n_tokens, uint32_
 /* Chooses the expert product of the batched gpt-oss prefill (no counterpart
  * in the reference, which prefills gpt-oss token by token): 0 (the default,
  * or environment RUSTY_HIP_EXPERT_MFMA=1 for 1) keeps every expert row the
- * reference's serial dot_mxfp4_f32_scalar sum, bit for bit; 1 runs the
- * products on the matrix cores (f32 MFMA over the exact f32 weights
- * lut * 2^(e-127) and the f32 activations), whose sums differ from the serial
- * ones in rounding only (within 1e-4 of sum |w x| per product).  Returns the
+ * reference's serial dot_mxfp4_f32_scalar sum, bit for bit; 1 adds the
+ * unrounded products (f32 MFMA over the exact f32 weights lut * 2^(e-127) and
+ * the f32 activations) at half the matrix-core work, whose sums differ from
+ * the serial ones in rounding only (within 1e-4 of sum |w x| per product).  Returns the
  * previous setting. */
 int rusty_hip_set_expert_mfma(int on);
 /* The batched expert product on DEVICE buffers (no counterpart in the
@@ -222,7 +223,7 @@ int rusty_hip_set_expert_mfma(int on);
  * row r starts at w + e * exp_stride + r * row_stride (row_stride a multiple
  * of 16 holding cols / 32 blocks of 17 bytes).  mfma = 0: the serial sums
  * (bit-exact with dot_mxfp4_f32_scalar, src/simd.rs:5886-5902); 1: the
- * matrix cores.  n_pairs <= 1024.  Waits for all device work first
+ * unrounded products.  n_pairs <= 1024.  Waits for all device work first
  * and returns once y is written; returns 0 on bad arguments. */
 int rusty_hip_mxfp4_experts(const uint8_t *w, int64_t row_stride, int64_t exp_stride, uint32_t n_exp, uint32_t rows,
                             uint32_t cols, const float *x, int64_t ldx, int x_per_pair, uint32_t top_k,

@@ -154,19 +154,8 @@ __global__ __launch_bounds__(256) void moe_combine_batch_kernel(const float *pro
     x[t * dim + i] += acc;
 }
 
-// MXFP4 expert rows for the (token, slot) pairs routed to each expert, every
-// sum dot_mxfp4_f32_scalar's running sum (as the single-token kernels).  A
-// workgroup of four waves serves one (64-row tile, expert, matrix): it lists
-// the pairs p = t k + r with sel[p] == expert, then in passes of 4 x MXE_G
-// pairs (wave w takes MXE_G of them, one running sum per pair and lane = row)
-// streams the tile's rows once per pass in 16-block chunks: coalesced direct
-// loads into a double-buffered LDS chunk (64 rows x 272 bytes, 17 loads of 1
-// KB shared among the waves), from which every lane reads its row's 17-byte
-// blocks.  A block's 32 weights are decoded once per wave and used for all
-// of its pairs; x comes through scalar loads.  y[mat] row p gets pair p's
-// sum.  grid (ceil(rows/64), n_exp, n_mats).
-#define MXE_G 8
-#define MXE_MAX_PAIRS 1024  // a token routes to an expert at most once: pairs per expert <= T
+// The routed expert product: for every (token, slot) pair p = t k + r routed
+// to expert e = sel[p], row r of e's MXFP4 matrix times the pair's activation.
 struct MxExpArgs {
     const uint8_t *w[2];  // expert tensors: expert e's row r at w + e*exp_stride + r*row_stride
     float *y[2];          // [T*k][ldy]
@@ -176,305 +165,315 @@ struct MxExpArgs {
     int64_t ldx, ldy;
     int32_t x_pair;
     const int32_t *sel;  // [n_pairs]
-    int32_t n_exp;       // the matrix-core kernel's expert count
+    int32_t n_exp;
 };
 
-__global__ __launch_bounds__(256) void gemv_mxfp4_experts_kernel(MxExpArgs A) {
-    __shared__ __align__(16) uint4 s_b[2][64 * 17];
-    __shared__ int32_t s_list[MXE_MAX_PAIRS];
-    __shared__ int32_t s_cnt[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int e = blockIdx.y, mat = blockIdx.z;
-    const int K = A.K, nb = K >> 5;
-    // the pairs routed to expert e, in pair order: each wave counts a quarter
-    // of the pairs, then writes its hits after the earlier waves'
-    const int per = (A.n_pairs + 3) / 4, pa = wave * per, pb = min(A.n_pairs, pa + per);
-    int cnt = 0;
-    for (int base = pa; base < pb; base += 64) {
-        const int p = base + lane;
-        cnt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(p < pb && A.sel[p] == e));
-    }
-    if (lane == 0) s_cnt[wave] = cnt;
-    __syncthreads();
-    int off = 0, n = 0;
-    for (int i = 0; i < 4; i++) {
-        off += i < wave ? s_cnt[i] : 0;
-        n += s_cnt[i];
-    }
-    for (int base = pa; base < pb; base += 64) {
-        const int p = base + lane;
-        const bool hit = p < pb && A.sel[p] == e;
-        const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
-        const int at = off + __builtin_popcountll(m & ((1ull << lane) - 1ull));
-        if (hit && at < MXE_MAX_PAIRS) s_list[at] = p;
-        off += __builtin_popcountll(m);
-    }
-    // the callers route every token to an expert at most once, so n <= T <=
-    // MXE_MAX_PAIRS; the bound only keeps the list inside its array
-    n = min(n, MXE_MAX_PAIRS);
-    if (n == 0) return;  // uniform over the workgroup
-    __syncthreads();
-    const uint8_t *w = A.w[mat] + (int64_t)e * A.exp_stride;
-    const int row0 = blockIdx.x * 64, row = row0 + lane;
-    const bool live = row < A.rows;
-    const int64_t stride = A.row_stride;
-    const int nch = (nb + MXF_C - 1) / MXF_C;
-    // piece f = 64 i + lane of a chunk is row f / 17, bytes 16 (f % 17); wave
-    // w issues pieces i = w, w + 4, ...
-    auto issue_chunk = [&](int c, int buf) {
-        for (int i = wave; i < 17; i += 4) {
-            const int f = 64 * i + lane, r = f / 17, p = f - 17 * r;
-            const int rr = min(row0 + r, A.rows - 1);
-            const int64_t o = min((int64_t)(MXF_C * 17 * c + 16 * p), stride - 16);
-            dma16(w + (int64_t)rr * stride + o, &s_b[buf][64 * i]);
-        }
-    };
-    for (int g0 = 0; g0 < n; g0 += 4 * MXE_G) {
-        const int q0 = g0 + wave * MXE_G;  // this wave's first pair of the pass
-        const float *xp[MXE_G];
-#pragma unroll
-        for (int i = 0; i < MXE_G; i++) {
-            // uniform, so that x arrives through scalar loads
-            const int p = __builtin_amdgcn_readfirstlane(s_list[min(q0 + i, n - 1)]);
-            xp[i] = A.x + (A.x_pair ? (int64_t)p : (int64_t)(p / A.k)) * A.ldx;
-        }
-        float sum[MXE_G];
-#pragma unroll
-        for (int i = 0; i < MXE_G; i++) sum[i] = 0.0f;
-        issue_chunk(0, 0);
-        for (int c = 0; c < nch; c++) {
-            RH_WAIT_VM(0);
-            __syncthreads();  // chunk c landed from every wave; chunk c - 1's reads are done
-            if (c + 1 < nch) issue_chunk(c + 1, (c + 1) & 1);
-            const uint8_t *rowb = (const uint8_t *)&s_b[c & 1][17 * lane];
-            for (int jj = 0; jj < MXF_C / 4; jj++) {
-#pragma unroll
-            for (int o = 0; o < 4; o++) {
-                const int j = 4 * jj + o, b = MXF_C * c + j;
-                if (b >= nb) break;  // uniform
-                // block j's 17 bytes start at byte 17 j = 68 jj + 16 o + o of
-                // the row: five dwords from the aligned 68 jj + 16 o, shifted
-                // by o bytes
-                const uint32_t *wp = (const uint32_t *)(rowb + 68 * jj + 16 * o);
-                uint32_t dw[5];
-#pragma unroll
-                for (int i = 0; i < 5; i++) dw[i] = wp[i];
-                uint32_t wd[4];
-#pragma unroll
-                for (int k4 = 0; k4 < 4; k4++) wd[k4] = o ? __builtin_amdgcn_alignbyte(dw[k4 + 1], dw[k4], o) : dw[k4];
-                const uint32_t e4 = dw[4] >> (8 * o);
-                const uint32_t ex = e4 & 0xFFu;
-                const float sc = mxfp4_scale(ex);
-                // the block's 32 weights lut * scale, exact either way
-                float wv[32];
-                if (__builtin_amdgcn_ballot_w64(ex == 0u || ex == 255u) == 0) {
-#pragma unroll
-                    for (int k4 = 0; k4 < 4; k4++)
-#pragma unroll
-                        for (int u = 0; u < 4; u++) {
-                            const fp4x2_f32 pr = fp4x2_scaled(wd[k4], sc, u);
-                            wv[8 * k4 + 2 * u] = pr.x;
-                            wv[8 * k4 + 2 * u + 1] = pr.y;
-                        }
-                } else {
-#pragma unroll
-                    for (int k4 = 0; k4 < 4; k4++)
-#pragma unroll
-                        for (int u = 0; u < 4; u++) {
-                            const uint32_t byte = (wd[k4] >> (8 * u)) & 0xFFu;
-                            wv[8 * k4 + 2 * u] = mxfp4_nibble(byte & 0xFu) * sc;
-                            wv[8 * k4 + 2 * u + 1] = mxfp4_nibble(byte >> 4) * sc;
-                        }
-                }
-#pragma unroll
-                for (int i = 0; i < MXE_G; i++) {
-                    const const_f32_ptr xb = (const_f32_ptr)xp[i] + b * 32;
-#pragma unroll
-                    for (int q = 0; q < 32; q++) sum[i] += wv[q] * xb[q];
-                }
-            }
-            }
-        }
-        __syncthreads();  // the last chunk's reads are done before the next pass restages
-#pragma unroll
-        for (int i = 0; i < MXE_G; i++)
-            if (q0 + i < n && live) A.y[mat][(int64_t)s_list[q0 + i] * A.ldy + row] = sum[i];
-    }
-}
-
-// ---- opt-in expert product on the matrix cores ------------------------------
-// The reference sums each MXFP4 row serially (dot_mxfp4_f32_scalar); the
-// matrix cores sum in their own order, so this path is not bit-exact and is
-// off unless rusty_hip_set_expert_mfma(1) selects it.  Its inputs keep the
-// reference's precision: the weights lut[n] * 2^(e-127) are exact in f32 and
-// the activations are the f32 rows; only the order of the f32 additions of
-// the K products differs (v_mfma_f32_32x32x2_f32).
-//
-// moe_expert_lists_kernel: for every expert, the pairs routed to it in pair
-// order (lists[e * cap ..]), their count, and tile0[e] = the number of
-// 32-pair tiles of the experts before e (tile0[n_exp] = all tiles).  One
-// workgroup; wave w lists experts w, w + 4, ...
-#define MXM_PAIRS 32
+// For every expert, the pairs routed to it in pair order (lists[e * cap ..]),
+// their count, and the pair tiles of all experts: tiles[0] of them, tiles[1 +
+// i] = e | (first pair / MXM_PAIRS) << 8.  Tiles of more than MXM_PAIRS / 2
+// pairs come first (they take twice the time of the others, and the last to
+// start should be the short ones), each kind in expert order.  One workgroup
+// of 16 waves, each with a contiguous sixteenth of the pairs: it counts its
+// pairs per expert (a ballot per expert and 64 pairs), then writes its hits
+// after the earlier waves'.  Pairs that name no expert are in no list.
+#define MXE_MAX_PAIRS 1024  // a token routes to an expert at most once: pairs per expert <= T
+#define MXM_PAIRS 64
 #define MXM_ROWS 128
-__global__ __launch_bounds__(256) void moe_expert_lists_kernel(const int32_t *sel, int n_pairs, int n_exp, int cap,
-                                                               int32_t *lists, int32_t *counts, int32_t *tile0) {
-    __shared__ int32_t s_cnt[64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int e = wave; e < n_exp; e += 4) {
-        int cnt = 0;
-        for (int base = 0; base < n_pairs; base += 64) {
-            const int p = base + lane;
-            const bool hit = p < n_pairs && sel[p] == e;
-            const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
-            const int at = cnt + __builtin_popcountll(m & ((1ull << lane) - 1ull));
-            if (hit && at < cap) lists[(size_t)e * cap + at] = p;
-            cnt += __builtin_popcountll(m);
-        }
-        cnt = min(cnt, cap);
-        if (lane == 0) {
-            counts[e] = cnt;
-            s_cnt[e] = cnt;
+#define MXE_MAX_TILES (8 * MXE_MAX_PAIRS / MXM_PAIRS + 64)  // top_k <= 8, n_exp <= 64
+__global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *sel, int n_pairs, int n_exp, int cap,
+                                                                 int32_t *lists, int32_t *counts, int32_t *tiles) {
+    __shared__ int32_t s_cnt[16][64], s_long[64], s_short[64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int per = ((n_pairs + 15) / 16 + 63) / 64 * 64, pa = min(n_pairs, wave * per), pb = min(n_pairs, pa + per);
+    int mine = 0;  // lane e: this wave's pairs of expert e
+    for (int base = pa; base < pb; base += 64) {
+        const int se = base + lane < pb ? sel[base + lane] : -1;
+        for (int e = 0; e < n_exp; e++) {
+            const int c = __builtin_popcountll(__builtin_amdgcn_ballot_w64(se == e));
+            mine += lane == e ? c : 0;
         }
     }
+    s_cnt[wave][lane] = mine;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
+    int off = 0, tot = 0;  // lane e: pairs of expert e in the earlier waves, in all waves
+    for (int w = 0; w < 16; w++) {
+        const int c = s_cnt[w][lane];
+        off += w < wave ? c : 0;
+        tot += c;
+    }
+    for (int base = pa; base < pb; base += 64) {
+        const int se = base + lane < pb ? sel[base + lane] : -1;
         for (int e = 0; e < n_exp; e++) {
-            tile0[e] = t;
-            t += (s_cnt[e] + MXM_PAIRS - 1) / MXM_PAIRS;
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(se == e);
+            const int at = __builtin_amdgcn_readlane(off, e) + __builtin_popcountll(m & ((1ull << lane) - 1ull));
+            if (se == e && at < cap) lists[(size_t)e * cap + at] = base + lane;
+            off += lane == e ? __builtin_popcountll(m) : 0;
         }
-        tile0[n_exp] = t;
+    }
+    if (wave == 0) {
+        tot = lane < n_exp ? min(tot, cap) : 0;
+        const int rem = tot % MXM_PAIRS, full = tot / MXM_PAIRS;
+        const int n_long = full + (rem > MXM_PAIRS / 2 ? 1 : 0), n_short = rem > 0 && rem <= MXM_PAIRS / 2 ? 1 : 0;
+        s_long[lane] = n_long;
+        s_short[lane] = n_short;
+        if (lane < n_exp) counts[lane] = tot;
+        int a = 0, b = 0, all = 0;  // earlier experts' long and short tiles, every long tile
+        for (int e = 0; e < 64; e++) {
+            const int l = s_long[e];
+            all += l;
+            a += e < lane ? l : 0;
+            b += e < lane ? s_short[e] : 0;
+        }
+        for (int i = 0; i < n_long; i++) tiles[1 + a + i] = lane | i << 8;
+        if (n_short) tiles[1 + all + b] = lane | full << 8;
+        if (lane == 63) tiles[0] = all + b + n_short;
     }
 }
 
-// y[mat] row p = expert rows times pair p's activation for one (128-row tile,
-// 32-pair tile of one expert, matrix): grid (ceil(rows / 128), an upper bound
-// of the pair tiles, n_mats); workgroups past tile0[n_exp] return.  Wave w
-// owns rows row0 + 32 w + (lane % 32); per 32-element block, 16 MFMAs
-// 32x32x2: MFMA i takes element 16 h + i (h = lane / 32) of the block from
-// both operands, A = the pair's activation (m = pair), B = the weight (n =
-// row), so lane h decodes bytes 8h..8h+7 of its row's block (element 2b + 1
-// is the high nibble of byte b).  The weights arrive in 16-block chunks of
-// 272 bytes per row by coalesced direct loads into a double-buffered LDS
-// chunk; each lane then reads its row's chunk into registers (17 reads, an
-// odd number of 16-byte units per row: conflict-free); the activations come
-// from global memory one block ahead.
-__global__ __launch_bounds__(256) void gemm_mxfp4_experts_mfma_kernel(MxExpArgs A, const int32_t *lists,
-                                                                      const int32_t *counts, const int32_t *tile0,
-                                                                      int cap) {
-    __shared__ __align__(16) uint4 s_b[2][MXM_ROWS * 17];
-    __shared__ int32_t s_pair[MXM_PAIRS];
+// y[mat] row p for one (128-row tile, 64-pair tile of one expert, matrix).
+// grid (ceil(rows / 128), an upper bound of the pair tiles, n_mats);
+// workgroups past the last tile return.  Wave w owns rows row0 + 32 w ..
+// + 31 and the tile's pairs in one or two groups of 32.
+//
+// SERIAL: dot_mxfp4_f32_scalar's running sum, sum = sum + (w x) per element in
+// order, bit for bit, on the matrix cores.  v_mfma_f32_32x32x2_f32 is a chain
+// of two fused multiply-adds in k order, each rounded (checked on the device
+// over normal, subnormal and mixed magnitudes), so a step of the chain with an
+// exact product is the reference's step.  The product of x and a weight with
+// magnitude 0.5, 1, 2 or 4 is exact; for 1.5, 3 and 6 the reference's rounded
+// w x is (w / 3) RN(3 x), an exact product again.  So an element takes both k
+// slots, (w1, x) and (w3, RN(3 x)), with w1 or w3 zero, and a zero product
+// leaves the sum as it is: the sum starts at +0 and is never -0.  Lane half h
+// = lane / 32 is k slot h: it holds w1 or w3 of row n = lane % 32 and x or
+// RN(3 x) of pair n.  Scaling by w's power of two is exact while nothing
+// leaves the normal range: a block whose |x| are 0 or in [2^-84, 2^80) and
+// whose scales are within 2^-40 .. 2^40 qualifies (products stay above 2^-126
+// and below 2^126); any other (zero, huge or non-finite values, scale bytes 0
+// and 255 among them) takes the element-by-element sums on the VALU.
+//
+// Otherwise (the opt-in product): the same chain with unrounded products,
+// element 2 i + h in k slot h of MFMA i.
+//
+// The bound is the matrix cores, 64 clocks per 32 rows x 32 pairs x element
+// (78 TFLOP/s of the reference's products), and f32 MFMAs leave the VALU
+// almost no room: beside 16x16x4 MFMAs each VALU instruction adds 2.5 to 4
+// clocks of a SIMD's 32 per MFMA.  Hence the 32x32 shape (half the operands
+// per product of 16x16; 16-pair groups, 64 rows per workgroup and the factor 3
+// in the loop took 1504 us for 1024 pairs of 11520 x 2880, 57% of the bound),
+// RN(3 x) computed once per workgroup into a plane of its own, and the code
+// lookup on four nibbles per v_perm.  Weights come from a double-buffered LDS
+// chunk of 8 blocks (rows of 136 bytes: 32 rows of a dword read are on distinct
+// banks), the activations from a double-buffered block of two planes per pair
+// (pitch 68 floats, 16-byte reads); both are loaded through registers one
+// chunk or block ahead, one barrier per block, 70 KB of LDS and two workgroups
+// per CU.  Measured: 1024 pairs of 11520 x 2880 1195 us (57 TFLOP/s, 0.72 of
+// the bound); the 4004 gate/up pairs of a 1001-token gpt-oss-20b chunk 2.68 ms
+// (49.5 TFLOP/s) where eight VALU sums per wave, x by scalar loads, took 6.92;
+// 1000 pairs over 32 experts of 2880 x 2880 (31 per expert: half-filled tiles)
+// 574 against 903 us.
+#define MXM_C 8  // weight blocks per LDS chunk
+template <bool SERIAL, int PT>
+__device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uint8_t *w, float *y, int row0, int np,
+                                                   uint2 *s_b, float *s_x, uint32_t *s_bad, const int32_t *s_pair) {
+    typedef float v4f __attribute__((ext_vector_type(4)));
     typedef float v16f __attribute__((ext_vector_type(16)));
+    constexpr int XP = 68, XN = MXM_PAIRS * XP;     // pair pitch and buffer size of s_x, in floats
+    constexpr int WP = MXM_C * 17, WN = MXM_ROWS * 17;  // row bytes and buffer size (8-byte pieces) of s_b
+    constexpr int NW = SERIAL ? 32 : 16;            // MFMAs per block and pair group
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int mat = blockIdx.z, gt = blockIdx.y;
-    const int n_exp = A.n_exp;
-    if (gt >= tile0[n_exp]) return;  // uniform
-    int e = 0;
-    while (e + 1 < n_exp && tile0[e + 1] <= gt) e++;
-    const int p0 = (gt - tile0[e]) * MXM_PAIRS;
-    const int np = min(MXM_PAIRS, counts[e] - p0);
-    if (tid < MXM_PAIRS) s_pair[tid] = lists[(size_t)e * cap + p0 + min(tid, np - 1)];
-    const int m = lane & 31, h = lane >> 5;
-    const int row0 = blockIdx.x * MXM_ROWS, row = row0 + 32 * wave + m;
-    const uint8_t *w = A.w[mat] + (int64_t)e * A.exp_stride;
-    const int64_t stride = A.row_stride;
-    const int nb = A.K >> 5, nch = (nb + MXF_C - 1) / MXF_C;
-    // piece f = 256 i + tid of a chunk: row f / 17, bytes 16 (f % 17); the
-    // 2176 pieces are 34 whole wave instructions, so a wave's instruction is
-    // either all inside the chunk or skipped
-    auto issue_chunk = [&](int c, int buf) {
+    const int n = lane & 31, h = lane >> 5;
+    const int nb = A.K >> 5;
+    // activations: thread t stages float4 t % 8 of the block for pairs t / 8 + 32 j
+    const int c4 = tid & 7, pr0 = tid >> 3;
+    const float *xr[PT];
 #pragma unroll
-        for (int i = 0; i < 9; i++) {
-            if (256 * i + 64 * wave >= MXM_ROWS * 17) continue;  // uniform
-            const int f = 256 * i + tid, r = f / 17, pc = f - 17 * r;
-            const int rr = min(row0 + r, A.rows - 1);
-            const int64_t o = min((int64_t)(MXF_C * 17 * c + 16 * pc), stride - 16);
-            dma16(w + (int64_t)rr * stride + o, &s_b[buf][256 * i + 64 * wave]);
-        }
+    for (int j = 0; j < PT; j++) {
+        const int p = s_pair[pr0 + 32 * j];
+        xr[j] = A.x + (A.x_pair ? (int64_t)p : (int64_t)(p / A.k)) * A.ldx + 4 * c4;
+    }
+    v4f xs[PT];
+    auto load_x = [&](int b) {
+#pragma unroll
+        for (int j = 0; j < PT; j++) __builtin_memcpy(&xs[j], xr[j] + 32 * b, 16);
     };
-    issue_chunk(0, 0);
-    __syncthreads();  // s_pair
-    const int pair = s_pair[m];
-    const float *xr = A.x + (A.x_pair ? (int64_t)pair : (int64_t)(pair / A.k)) * A.ldx + 16 * h;
-    float4 xa[4], xb[4];
-    auto load_x = [&](int b, float4 (&xv)[4]) {
-        const float4 *p = (const float4 *)(xr + 32 * (int64_t)min(b, nb - 1));
+    auto store_x = [&](int b) {
+        bool bad = false;
 #pragma unroll
-        for (int q = 0; q < 4; q++) xv[q] = p[q];
-    };
-    load_x(0, xa);
-    v16f acc = {};
-    for (int c = 0; c < nch; c++) {
-        RH_WAIT_VM(0);
-        __syncthreads();  // chunk c landed from every wave; every read of chunk c - 1 done
-        uint32_t wr[68];
-        {
-            const uint4 *rp = &s_b[c & 1][(32 * wave + m) * 17];
+        for (int j = 0; j < PT; j++) {
+            float *r = s_x + (b & 1) * XN + (pr0 + 32 * j) * XP;
+            const v4f v = xs[j];
+            if (SERIAL) {
+                *(v4f *)(r + 4 * c4) = v;
+                *(v4f *)(r + 32 + 4 * c4) = v * 3.0f;
 #pragma unroll
-            for (int q = 0; q < 17; q++) {
-                const uint4 v = rp[q];
-                wr[4 * q] = v.x;
-                wr[4 * q + 1] = v.y;
-                wr[4 * q + 2] = v.z;
-                wr[4 * q + 3] = v.w;
-            }
-        }
-        // block j of the chunk with its activations in cur; the next block's
-        // go to nxt (clamped past the end), then, late in the chunk, the next
-        // chunk's weights are issued: a load issued after them would wait for
-        // them too (loads retire in order), and only the next chunk's first
-        // activations are
-        auto block = [&](int j, const float4 (&cur)[4], float4 (&nxt)[4]) {
-            const int b = MXF_C * c + j;
-            if (b >= nb) return;  // uniform
-            load_x(b + 1, nxt);
-            if (j == MXF_C - 2 && c + 1 < nch) issue_chunk(c + 1, (c + 1) & 1);
-            // bytes 17 j + 8 h .. + 7 and the scale byte 17 j + 16
-            const int o0 = 17 * j, o1 = 17 * j + 8, os = 17 * j + 16;
-            const uint32_t a0 = __builtin_amdgcn_alignbyte(wr[o0 / 4 + 1], wr[o0 / 4], o0 % 4);
-            const uint32_t a1 = __builtin_amdgcn_alignbyte(wr[o0 / 4 + 2], wr[o0 / 4 + 1], o0 % 4);
-            const uint32_t c0 = __builtin_amdgcn_alignbyte(wr[o1 / 4 + 1], wr[o1 / 4], o1 % 4);
-            const uint32_t c1 = __builtin_amdgcn_alignbyte(wr[o1 / 4 + 2], wr[o1 / 4 + 1], o1 % 4);
-            const uint32_t d0 = h ? c0 : a0, d1 = h ? c1 : a1;
-            const uint32_t ex = (wr[os / 4] >> (8 * (os % 4))) & 0xFFu;
-            const float sc = mxfp4_scale(ex);
-            float wv[16];
-            if (__builtin_amdgcn_ballot_w64(ex == 0u || ex == 255u) == 0) {
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const fp4x2_f32 lo = fp4x2_scaled(d0, sc, u), hi = fp4x2_scaled(d1, sc, u);
-                    wv[2 * u] = lo.x;
-                    wv[2 * u + 1] = lo.y;
-                    wv[8 + 2 * u] = hi.x;
-                    wv[9 + 2 * u] = hi.y;
+                for (int i = 0; i < 4; i++) {
+                    const float f = fabsf(v[i]);
+                    bad |= (f < 0x1p-84f && f != 0.0f) || !(f < 0x1p80f);
                 }
             } else {
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const uint32_t b0 = (d0 >> (8 * u)) & 0xFFu, b1 = (d1 >> (8 * u)) & 0xFFu;
-                    wv[2 * u] = mxfp4_nibble(b0 & 0xFu) * sc;
-                    wv[2 * u + 1] = mxfp4_nibble(b0 >> 4) * sc;
-                    wv[8 + 2 * u] = mxfp4_nibble(b1 & 0xFu) * sc;
-                    wv[9 + 2 * u] = mxfp4_nibble(b1 >> 4) * sc;
-                }
+                *(float2 *)(r + 2 * c4) = make_float2(v[0], v[2]);
+                *(float2 *)(r + 32 + 2 * c4) = make_float2(v[1], v[3]);
             }
-            const float xs[16] = {cur[0].x, cur[0].y, cur[0].z, cur[0].w, cur[1].x, cur[1].y, cur[1].z, cur[1].w,
-                                  cur[2].x, cur[2].y, cur[2].z, cur[2].w, cur[3].x, cur[3].y, cur[3].z, cur[3].w};
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xs[i], wv[i], acc, 0, 0, 0);
-        };
-#pragma unroll
-        for (int j = 0; j < MXF_C; j += 2) {
-            block(j, xa, xb);
-            block(j + 1, xb, xa);
         }
+        if (SERIAL) {
+            const uint32_t any = __builtin_amdgcn_ballot_w64(bad) != 0 ? 1u : 0u;
+            if (lane == 0) s_bad[4 * (b & 1) + wave] = any;
+        }
+    };
+    // weights: piece f = 256 i + t of a chunk is row f / 17, bytes 8 (f % 17)
+    constexpr int NP = (WN + 255) / 256;
+    uint2 wg[NP];
+    auto load_w = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int f = min(256 * i + tid, WN - 1), r = f / 17, p = f - 17 * r;
+            const int rr = min(row0 + r, A.rows - 1);
+            const int64_t o = min((int64_t)(WP * c + 8 * p), A.row_stride - 8);
+            wg[i] = ld8(w + (int64_t)rr * A.row_stride + o);
+        }
+    };
+    auto store_w = [&](int c) {
+        uint2 *d = s_b + (c & 1) * WN;
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            if (256 * i + 256 <= WN || 256 * i + tid < WN) d[256 * i + tid] = wg[i];
+    };
+    // the weights k slot h takes of the eight magnitudes: 0.5, 1, 2 and 4, or
+    // a third of 1.5, 3 and 6
+    const uint32_t tlo = h ? 0x01000000u : 0x00020100u, thi = h ? 0x04000200u : 0x00060004u;
+    const uint8_t *rowb0 = (const uint8_t *)s_b + (32 * wave + n) * WP;
+    // block b's weights of this lane's k slot; returns whether a scale needs
+    // the element path
+    auto decode = [&](int b, float (&wv)[NW]) -> bool {
+        const int j = b & (MXM_C - 1);
+        // the block's 17 bytes from byte 17 j of the row, five aligned dwords
+        const uint32_t *wp = (const uint32_t *)(rowb0 + ((b / MXM_C) & 1) * (WN * 8) + ((17 * j) & ~3));
+        const uint32_t sb = (uint32_t)j & 3u;  // 17 j mod 4
+        uint32_t dw[5], wd[4];
+#pragma unroll
+        for (int i = 0; i < 5; i++) dw[i] = wp[i];
+#pragma unroll
+        for (int i = 0; i < 4; i++) wd[i] = __builtin_amdgcn_alignbyte(dw[i + 1], dw[i], sb);
+        const uint32_t ex = (dw[4] >> (8u * sb)) & 0xFFu;
+        const float sc = __builtin_bit_cast(float, ex << 23);  // 2^(ex - 127) where it is used: 0 < ex < 255
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            if (SERIAL) {
+                const uint32_t lo = __builtin_amdgcn_perm(thi, tlo, wd[q] & 0x07070707u);
+                const uint32_t hi = __builtin_amdgcn_perm(thi, tlo, (wd[q] >> 4) & 0x07070707u);
+                const uint32_t u = (lo | (hi << 4)) | (wd[q] & 0x88888888u);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const fp4x2_f32 p = fp4x2_scaled(u, sc, i);
+                    wv[(8 * q + 2 * i) % NW] = p.x;
+                    wv[(8 * q + 2 * i + 1) % NW] = p.y;
+                }
+            } else {
+                const uint32_t t = (wd[q] >> (4 * h)) & 0x0F0F0F0Fu, u = t | (t >> 4);
+                const fp4x2_f32 lo = fp4x2_scaled(u, sc, 0), hi = fp4x2_scaled(u, sc, 2);
+                wv[4 * q] = lo.x;
+                wv[4 * q + 1] = lo.y;
+                wv[4 * q + 2] = hi.x;
+                wv[4 * q + 3] = hi.y;
+            }
+        }
+        return SERIAL ? ex - 87u > 80u : ex - 1u > 253u;
+    };
+    v16f acc[PT];
+#pragma unroll
+    for (int g = 0; g < PT; g++) acc[g] = v16f{};
+    // block b from the LDS bytes, element by element: C element i of lane
+    // (n, h) is (pair 8 (i / 4) + 4 h + i % 4, row n)
+    auto slow_block = [&](int b) {
+        const int j = b & (MXM_C - 1);
+        const uint8_t *blk = rowb0 + ((b / MXM_C) & 1) * (WN * 8) + 17 * j;
+        const float sc = mxfp4_scale(blk[16]);
+        const float *xc = s_x + (b & 1) * XN + 4 * h * XP;
+#pragma unroll 1
+        for (int e = 0; e < 32; e++) {
+            const uint32_t byte = blk[e >> 1];
+            const float wv = mxfp4_nibble((e & 1) ? byte >> 4 : byte & 0xFu) * sc;
+            const int at = SERIAL ? e : (e & 1) * 32 + (e >> 1);
+#pragma unroll
+            for (int g = 0; g < PT; g++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    acc[g][i] += wv * xc[(32 * g + 8 * (i >> 2) + (i & 3)) * XP + at];
+        }
+    };
+    load_w(0);
+    load_x(0);
+    store_w(0);
+    store_x(0);
+    load_x(min(1, nb - 1));
+    float wcur[NW];
+    bool odd = false;
+    const float *xb0 = s_x + n * XP + 32 * h;
+    for (int b = 0; b < nb; b++) {
+        __syncthreads();  // block b is in LDS; block b - 1's reads are done
+        if (b + 1 < nb) store_x(b + 1);
+        if (b + 2 < nb) load_x(b + 2);
+        // the next weight chunk, one block before the decode ahead reads it
+        const int c = b / MXM_C, j = b & (MXM_C - 1);
+        if (MXM_C * (c + 1) < nb) {
+            if (j == 1) load_w(c + 1);
+            if (j == MXM_C - 2) store_w(c + 1);
+        }
+        if (b == 0) odd = __builtin_amdgcn_ballot_w64(decode(0, wcur)) != 0;
+        uint32_t xbad = 0;
+        if (SERIAL) {
+            const uint4 b4 = *(const uint4 *)(s_bad + 4 * (b & 1));
+            xbad = __builtin_amdgcn_readfirstlane(b4.x | b4.y | b4.z | b4.w);
+        }
+        if (odd || xbad != 0) {
+            slow_block(b);
+        } else {
+            const float *xc = xb0 + (b & 1) * XN;
+            v4f xv[NW / 4][PT];
+#pragma unroll
+            for (int q = 0; q < NW / 4; q++)
+#pragma unroll
+                for (int g = 0; g < PT; g++) xv[q][g] = *(const v4f *)(xc + 32 * g * XP + 4 * q);
+#pragma unroll
+            for (int i = 0; i < NW; i++)
+#pragma unroll
+                for (int g = 0; g < PT; g++)
+                    acc[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[i >> 2][g][i & 3], wcur[i], acc[g], 0, 0, 0);
+        }
+        odd = __builtin_amdgcn_ballot_w64(decode(min(b + 1, nb - 1), wcur)) != 0;
     }
+    const int row = row0 + 32 * wave + n;
     if (row >= A.rows) return;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int mi = 8 * (i >> 2) + 4 * h + (i & 3);
-        if (mi < np) A.y[mat][(int64_t)s_pair[mi] * A.ldy + row] = acc[i];
-    }
+    for (int g = 0; g < PT; g++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int p = 32 * g + 8 * (i >> 2) + 4 * h + (i & 3);
+            if (p < np) y[(int64_t)s_pair[p] * A.ldy + row] = acc[g][i];
+        }
+}
+
+template <bool SERIAL>
+__global__ __launch_bounds__(256, 2) void gemm_mxfp4_experts_kernel(MxExpArgs A, const int32_t *lists,
+                                                                    const int32_t *counts, const int32_t *tiles,
+                                                                    int cap) {
+    __shared__ __align__(16) uint2 s_b[2 * MXM_ROWS * 17];
+    __shared__ __align__(16) float s_x[2 * MXM_PAIRS * 68];
+    __shared__ __align__(16) uint32_t s_bad[8];
+    __shared__ int32_t s_pair[MXM_PAIRS];
+    const int mat = blockIdx.z;
+    if ((int)blockIdx.y >= tiles[0]) return;  // uniform
+    const int tile = tiles[1 + blockIdx.y], e = tile & 0xFF;
+    const int p0 = (tile >> 8) * MXM_PAIRS, np = min(MXM_PAIRS, counts[e] - p0);
+    if (threadIdx.x < MXM_PAIRS) s_pair[threadIdx.x] = lists[(size_t)e * cap + p0 + min((int)threadIdx.x, np - 1)];
+    __syncthreads();
+    const uint8_t *w = A.w[mat] + (int64_t)e * A.exp_stride;
+    float *y = A.y[mat];
+    const int row0 = blockIdx.x * MXM_ROWS;
+    if (np > 32)
+        mxfp4_experts_tile<SERIAL, 2>(A, w, y, row0, np, s_b, s_x, s_bad, s_pair);
+    else
+        mxfp4_experts_tile<SERIAL, 1>(A, w, y, row0, np, s_b, s_x, s_bad, s_pair);
 }
 
 // K/V rows between a ring cache and the linear buffer of a batched ring

@@ -2146,7 +2146,7 @@ struct Resident {
     int32_t *psel = nullptr;
     // the matrix-core expert product's per-expert pair lists, counts and
     // tile offsets (rusty_hip_set_expert_mfma)
-    int32_t *plists = nullptr, *pcounts = nullptr, *ptile0 = nullptr;
+    int32_t *plists = nullptr, *pcounts = nullptr, *ptiles = nullptr;
     std::map<std::pair<int, uint32_t>, hipGraphExec_t> graphs;  // by (mode, penalty bits)
     std::vector<void *> allocs;
     std::vector<std::pair<const void *, DevW>> wown;  // weight copies owned by the decoder
@@ -2623,15 +2623,18 @@ static int r_run(int mode, float penalty) {
 // result exactly.  Every value written is bit-identical to decoding the
 // tokens one by one.
 // Tokens per chunk: RUSTY_HIP_PREFILL_CHUNK (64..2048), else 512 (a sweep
-// over 256/512/1024 on a 2048-token prompt put 512 first, by 2-4%).
-static int pf_chunk() {
+// over 256/512/1024 on a 2048-token prompt put 512 first, by 2-4%).  A gpt-oss
+// chunk is 1024 tokens where its attention scratch (moe_scratch bytes per
+// token; 0 for other models) stays within 8 GB: the experts' 64-pair tiles
+// fill up (32 experts, top 4: 128 pairs per expert instead of 64).
+static int pf_chunk(size_t moe_scratch) {
     static int v = -1;
     if (v < 0) {
         const char *e = getenv("RUSTY_HIP_PREFILL_CHUNK");
-        v = e ? atoi(e) : 512;
-        v = std::max(64, std::min(2048, v));
+        v = e ? std::max(64, std::min(2048, atoi(e))) : 0;
     }
-    return v;
+    if (v) return v;
+    return moe_scratch && moe_scratch * 1024 <= ((size_t)8 << 30) ? 1024 : 512;
 }
 
 static bool r_prefill_enabled() {
@@ -2656,11 +2659,11 @@ static bool r_prefill_batchable() {
 
 static int r_prefill_alloc() {
     if (R.pf_cap) return 1;
-    const size_t C = (size_t)pf_chunk();
+    const size_t ex = exact_scratch_floats((int)R.n_kv, (int)(R.n_heads / R.n_kv), R.ex_cap);
+    const size_t C = (size_t)pf_chunk(R.moe ? ex * 4 : 0);
     const size_t qd = (size_t)R.n_heads * R.hd, kd = (size_t)R.n_kv * R.hd, vdim = (size_t)R.n_kv * R.vd;
     const size_t attn_cols = (size_t)R.n_heads * R.vd;
     const size_t kmax = std::max<size_t>(std::max<size_t>(R.dim, attn_cols), R.hidden);
-    const size_t ex = exact_scratch_floats((int)R.n_kv, (int)(R.n_heads / R.n_kv), R.ex_cap);
     if (!r_alloc((void **)&R.px, C * R.dim * 4) || !r_alloc((void **)&R.pq, C * qd * 4) ||
         !r_alloc((void **)&R.pk, C * kd * 4) || !r_alloc((void **)&R.pv, C * vdim * 4) ||
         !r_alloc((void **)&R.pattn, C * attn_cols * 4) || !r_alloc((void **)&R.ptg, C * R.hidden * 4) ||
@@ -2811,15 +2814,15 @@ static int r_prefill_moe_alloc() {
         !r_alloc((void **)&R.pprob, C * k * 4) || !r_alloc((void **)&R.pgate, C * k * hid * 4) ||
         !r_alloc((void **)&R.pup, C * k * hid * 4) || !r_alloc((void **)&R.pproj, C * k * R.dim * 4) ||
         !r_alloc((void **)&R.pxn, C * R.dim * 4) || !r_alloc((void **)&R.plists, (size_t)64 * MXE_MAX_PAIRS * 4) ||
-        !r_alloc((void **)&R.pcounts, 64 * 4) || !r_alloc((void **)&R.ptile0, 65 * 4))
+        !r_alloc((void **)&R.pcounts, 64 * 4) || !r_alloc((void **)&R.ptiles, (1 + MXE_MAX_TILES) * 4))
         return 0;
     return 1;
 }
 
-// The expert product of the batched gpt-oss prefill: the reference's serial
-// row sums (gemv_mxfp4_experts_kernel, bit-exact; the default) or, when
-// rusty_hip_set_expert_mfma(1) chose it, the matrix cores (the pair lists
-// first, then gemm_mxfp4_experts_mfma_kernel).  lists/counts/tile0: the list
+// The expert product of the batched gpt-oss prefill on the matrix cores (the
+// pair lists first, then gemm_mxfp4_experts_kernel): the reference's serial
+// row sums (bit-exact; the default) or, when rusty_hip_set_expert_mfma(1)
+// chose it, sums of unrounded products.  lists/counts/tiles: the list
 // buffers; with lists_ready the lists of this sel are already built.
 static int g_expert_mfma = -1;
 static bool expert_mfma_on() {
@@ -2829,33 +2832,30 @@ static bool expert_mfma_on() {
     }
     return g_expert_mfma == 1;
 }
-static int experts_enqueue(MxExpArgs A, int n_mats, bool mfma, int32_t *lists, int32_t *counts, int32_t *tile0,
+static int experts_enqueue(MxExpArgs A, int n_mats, bool mfma, int32_t *lists, int32_t *counts, int32_t *tiles,
                            bool lists_ready, const char *name, hipStream_t s) {
     if (A.n_exp < 1 || A.n_exp > 64 || A.K % 32 != 0 || A.n_pairs <= 0 || A.rows <= 0 || n_mats < 1 || n_mats > 2)
         return 0;
-    if (!mfma) {
-        if (A.n_pairs > MXE_MAX_PAIRS * A.k) return 0;
-        ProfScope ps(name, s);
-        rh_launch(gemv_mxfp4_experts_kernel, dim3((unsigned)((A.rows + 63) / 64), (unsigned)A.n_exp, (unsigned)n_mats),
-                  dim3(256), 0, s, A);
-        RH_LAUNCH_OK();
-        return 1;
-    }
-    // the activation rows are read as 16-byte pieces
-    if (A.ldx % 4 != 0 || ((uintptr_t)A.x & 15) != 0 || A.row_stride % 16 != 0) return 0;
+    // every expert's list holds at most MXE_MAX_PAIRS pairs
+    if (A.n_pairs > MXE_MAX_PAIRS * A.k || A.row_stride % 16 != 0) return 0;
+    // (the opt-in product refuses activations off 16-byte rows, as it always has)
+    if (mfma && (A.ldx % 4 != 0 || ((uintptr_t)A.x & 15) != 0)) return 0;
     if (!lists_ready) {
         ProfScope ps("moe_expert_lists", s);
-        rh_launch(moe_expert_lists_kernel, dim3(1), dim3(256), 0, s, A.sel, A.n_pairs, A.n_exp, MXE_MAX_PAIRS, lists,
-                  counts, tile0);
+        rh_launch(moe_expert_lists_kernel, dim3(1), dim3(1024), 0, s, A.sel, A.n_pairs, A.n_exp, MXE_MAX_PAIRS, lists,
+                  counts, tiles);
         RH_LAUNCH_OK();
     }
-    // at most ceil(n_pairs / 32) + n_exp pair tiles in all
-    const unsigned tiles = (unsigned)((A.n_pairs + MXM_PAIRS - 1) / MXM_PAIRS + A.n_exp);
+    // at most floor(n_pairs / 64) full pair tiles and one partial tile per expert
+    const unsigned n_tiles = (unsigned)(A.n_pairs / MXM_PAIRS + std::min(A.n_exp, A.n_pairs));
+    const dim3 grid((unsigned)((A.rows + MXM_ROWS - 1) / MXM_ROWS), n_tiles, (unsigned)n_mats);
     ProfScope ps(name, s);
-    rh_launch(gemm_mxfp4_experts_mfma_kernel, dim3((unsigned)((A.rows + MXM_ROWS - 1) / MXM_ROWS), tiles,
-                                                   (unsigned)n_mats),
-              dim3(256), 0, s, A, (const int32_t *)lists, (const int32_t *)counts, (const int32_t *)tile0,
-              (int)MXE_MAX_PAIRS);
+    if (mfma)
+        rh_launch(gemm_mxfp4_experts_kernel<false>, grid, dim3(256), 0, s, A, (const int32_t *)lists,
+                  (const int32_t *)counts, (const int32_t *)tiles, (int)MXE_MAX_PAIRS);
+    else
+        rh_launch(gemm_mxfp4_experts_kernel<true>, grid, dim3(256), 0, s, A, (const int32_t *)lists,
+                  (const int32_t *)counts, (const int32_t *)tiles, (int)MXE_MAX_PAIRS);
     RH_LAUNCH_OK();
     return 1;
 }
@@ -3058,7 +3058,7 @@ static int r_prefill_chunk_moe(const int32_t *tok, int T, int pos0, hipStream_t 
             A.sel = R.psel;
             A.n_exp = M.n_exp;
             if (M.up.stride != M.gate.stride) return 0;
-            if (!experts_enqueue(A, 2, mfma, R.plists, R.pcounts, R.ptile0, false, "pf_mxfp4_gate_up", s)) return 0;
+            if (!experts_enqueue(A, 2, mfma, R.plists, R.pcounts, R.ptiles, false, "pf_mxfp4_gate_up", s)) return 0;
         }
         {
             ProfScope ps("moe_swiglu_batch", s);
@@ -3083,7 +3083,7 @@ static int r_prefill_chunk_moe(const int32_t *tok, int T, int pos0, hipStream_t 
             A.x_pair = 1;
             A.sel = R.psel;
             A.n_exp = M.n_exp;
-            if (!experts_enqueue(A, 1, mfma, R.plists, R.pcounts, R.ptile0, true, "pf_mxfp4_down", s)) return 0;
+            if (!experts_enqueue(A, 1, mfma, R.plists, R.pcounts, R.ptiles, true, "pf_mxfp4_down", s)) return 0;
         }
         {
             ProfScope ps("moe_combine_batch", s);
@@ -3473,7 +3473,7 @@ int rusty_hip_mxfp4_experts(const uint8_t *w, int64_t row_stride, int64_t exp_st
     static int32_t *lists[64] = {};  // per device: pair lists, counts, tile offsets
     if (g.dev < 0 || g.dev >= 64) return 0;
     int32_t *&L = lists[g.dev];
-    if (mfma && !L && hipMalloc((void **)&L, ((size_t)64 * MXE_MAX_PAIRS + 64 + 65) * 4) != hipSuccess) {
+    if (!L && hipMalloc((void **)&L, ((size_t)64 * MXE_MAX_PAIRS + 64 + 1 + MXE_MAX_TILES) * 4) != hipSuccess) {
         L = nullptr;
         return 0;
     }
@@ -3494,7 +3494,7 @@ int rusty_hip_mxfp4_experts(const uint8_t *w, int64_t row_stride, int64_t exp_st
     A.sel = sel;
     A.n_exp = (int32_t)n_exp;
     RH_CHECK(hipDeviceSynchronize());  // the caller's writes of w, x and sel are complete
-    int32_t *lp = L, *cp = L ? L + (size_t)64 * MXE_MAX_PAIRS : nullptr, *tp = cp ? cp + 64 : nullptr;
+    int32_t *lp = L, *cp = L + (size_t)64 * MXE_MAX_PAIRS, *tp = cp + 64;
     if (!experts_enqueue(A, 1, mfma != 0, lp, cp, tp, false, mfma ? "mxfp4_experts_mfma" : "mxfp4_experts", g.s))
         return 0;
     RH_CHECK(hipStreamSynchronize(g.s));
