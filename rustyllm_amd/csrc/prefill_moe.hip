@@ -128,6 +128,245 @@ __global__ __launch_bounds__(256) void gemv_q8_0_batch_kernel(Q80BatchArgs A) {
     }
 }
 
+// ---- Q8_0 products of a token batch on the matrix cores ----------------------
+// y[t][r] for up to three matrices that share their activations (the q/k/v
+// projections in one launch: k and v alone would leave half of the CUs idle);
+// each (row, token) is exactly the single-token kernel's value.  A workgroup
+// is 64 rows by 64 tokens, wave (wr, wt) of it 32 rows by 32 tokens with eight
+// accumulators per output, one per AVX2 lane j.  Both operands of a chunk of
+// two 32-element blocks are staged in LDS in the form the MFMAs take them
+// (double-buffered, loaded through registers a chunk ahead; one barrier per
+// chunk), so a weight is decoded once per 64 tokens.
+struct Q80GemmArgs {
+    Q80BatchArgs m[3];  // epi, x / qs / dx / ldx, K and T are the same in all
+    int32_t tiles[3];   // 64-row tiles up to and including matrix i
+};
+#define Q8G_P 68  // row pitch in LDS, floats: 16-byte reads of 8 rows start on distinct banks
+
+__device__ __forceinline__ Q80BatchArgs q80_gemm_pick(const Q80GemmArgs &G, int &row0) {
+    const int bx = blockIdx.x;
+    const int i = bx < G.tiles[0] ? 0 : bx < G.tiles[1] ? 1 : 2;
+    row0 = 64 * (bx - (i == 0 ? 0 : i == 1 ? G.tiles[0] : G.tiles[1]));
+    // member by member: a copy of a run-time element would go through scratch
+    Q80BatchArgs A = G.m[0];
+    A.w = i == 0 ? A.w : i == 1 ? G.m[1].w : G.m[2].w;
+    A.row_stride = i == 0 ? A.row_stride : i == 1 ? G.m[1].row_stride : G.m[2].row_stride;
+    A.rows = i == 0 ? A.rows : i == 1 ? G.m[1].rows : G.m[2].rows;
+    A.bias = i == 0 ? A.bias : i == 1 ? G.m[1].bias : G.m[2].bias;
+    A.y = i == 0 ? A.y : i == 1 ? G.m[1].y : G.m[2].y;
+    A.ldy = i == 0 ? A.ldy : i == 1 ? G.m[1].ldy : G.m[2].ldy;
+    return A;
+}
+
+typedef float q8_v4f __attribute__((ext_vector_type(4)));
+typedef float q8_v16f __attribute__((ext_vector_type(16)));
+
+// hsum_avx of the eight accumulators, bias, store or add.  C element i of lane
+// (n, h) is (token 8 (i / 4) + 4 h + i % 4, row n).
+__device__ __forceinline__ void q80_gemm_store(const Q80BatchArgs &A, const q8_v16f (&acc)[8], int row, int t0, int h) {
+    if (row >= A.rows) return;
+    const float bias = A.bias ? A.bias[row] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int t = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
+        if (t >= A.T) continue;
+        float v = ((acc[0][i] + acc[4][i]) + (acc[1][i] + acc[5][i])) + ((acc[2][i] + acc[6][i]) + (acc[3][i] + acc[7][i]));
+        if (A.bias) v += bias;
+        float *y = A.y + (int64_t)t * A.ldy + row;
+        if (A.epi == EPI_ADD)
+            *y += v;
+        else
+            *y = v;
+    }
+}
+
+// f32 activations (K % 256 != 0): acc_j = fma(d q, x, acc_j) over the elements
+// e = j (mod 8) in order.  v_mfma_f32_32x32x2_f32 is two such steps in k order
+// (gemm_mxfp4_experts_kernel), so chain j takes elements 16 u + j and 16 u + 8
+// + j in MFMA u: lane half h holds elements 8 h .. 8 h + 7 of every 16.  d q is
+// exact in f32.  Bound by the matrix cores, 64 clocks per 32 x 32 x 2 products
+// (157 TFLOP/s).  Measured: the q, k and v products of gpt-oss-20b (5120 x
+// 2880, 1001 tokens) 300 us (98 TFLOP/s), 2253 with gemv_q8_0_batch_kernel.
+__global__ __launch_bounds__(256, 2) void gemm_q8_0_f32_kernel(Q80GemmArgs G) {
+    __shared__ __align__(16) float s_x[2][64 * Q8G_P], s_w[2][64 * Q8G_P];
+    int row0;
+    const Q80BatchArgs A = q80_gemm_pick(G, row0);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, h = lane >> 5, wr = wave & 1, wt = wave >> 1, t0 = blockIdx.y * 64;
+    const int K = A.K, nb = K >> 5, nc = (nb + 1) / 2;
+    // thread t stages float4 t % 16 of the chunk for tokens t / 16 + 16 j, and
+    // quants 8 (t % 4) .. + 7 of row t / 4 of both blocks
+    const int c4 = tid & 15, part = tid & 3;
+    const float *xr[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) xr[j] = A.x + (int64_t)min(t0 + (tid >> 4) + 16 * j, A.T - 1) * K + 4 * c4;
+    const uint8_t *wr0 = A.w + (int64_t)min(row0 + (tid >> 2), A.rows - 1) * A.row_stride;
+    q8_v4f xs[4];
+    uint2 wq[2];
+    uint16_t wd[2];
+    auto load = [&](int c) {
+        const bool in = 64 * c + 4 * c4 < K;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            xs[j] = q8_v4f{0.f, 0.f, 0.f, 0.f};
+            if (in) xs[j] = *(const q8_v4f *)(xr[j] + 64 * c);
+        }
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            const uint8_t *blk = wr0 + (int64_t)min(2 * c + o, nb - 1) * 34;
+            wd[o] = ld2(blk);
+            wq[o] = ld8(blk + 2 + 8 * part);
+        }
+    };
+    auto store = [&](int c) {
+        float *dx = s_x[c & 1] + (tid >> 4) * Q8G_P + 4 * c4;
+#pragma unroll
+        for (int j = 0; j < 4; j++) *(q8_v4f *)(dx + 16 * j * Q8G_P) = xs[j];
+        float *dw = s_w[c & 1] + (tid >> 2) * Q8G_P + 8 * part;
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            const float d = h2f(wd[o]);
+            q8_v4f a, b;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                a[i] = d * (float)(int8_t)(wq[o].x >> (8 * i));
+                b[i] = d * (float)(int8_t)(wq[o].y >> (8 * i));
+            }
+            *(q8_v4f *)(dw + 32 * o) = a;
+            *(q8_v4f *)(dw + 32 * o + 4) = b;
+        }
+    };
+    q8_v16f acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) acc[j] = q8_v16f{};
+    load(0);
+    store(0);
+    load(min(1, nc - 1));
+    for (int c = 0; c < nc; c++) {
+        __syncthreads();  // chunk c is in LDS; chunk c - 1's reads are done
+        if (c + 1 < nc) store(c + 1);
+        if (c + 2 < nc) load(c + 2);
+        const float *xa = s_x[c & 1] + (32 * wt + n) * Q8G_P + 8 * h;
+        const float *wa = s_w[c & 1] + (32 * wr + n) * Q8G_P + 8 * h;
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            if (2 * c + o >= nb) break;  // uniform
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                q8_v4f a[2], b[2];
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    a[q] = *(const q8_v4f *)(xa + 32 * o + 16 * u + 4 * q);
+                    b[q] = *(const q8_v4f *)(wa + 32 * o + 16 * u + 4 * q);
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j >> 2][j & 3], b[j >> 2][j & 3], acc[j], 0, 0, 0);
+            }
+        }
+    }
+    q80_gemm_store(A, acc, row0 + 32 * wr + n, t0 + 32 * wt, h);
+}
+
+// Q8_K activations (K % 256 == 0): acc_j = fma(dx d, s_j, acc_j) per 32-element
+// block, s_j the exact dot of bytes 4 j .. 4 j + 3.  v_mfma_f32_32x32x4_2b_f16
+// gives two of the eight s_j at once, as f32 with no conversion: quants are
+// exact in f16 and |s_j| <= 2^16; lane half h holds chain j = 2 u + h of MFMA
+// u.  Bound by the VALU's 144 multiplies and fused adds per 32 x 32 outputs
+// and block (the matrix cores' 4 x 64 clocks run beside them).  Measured: wo
+// of gpt-oss-20b (2880 x 4096, 1001 tokens) 212 us, 975 with
+// gemv_q8_0_batch_kernel.
+typedef _Float16 q8_v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 q8_v2h __attribute__((ext_vector_type(2)));
+typedef float q8_v32f __attribute__((ext_vector_type(32)));
+#define Q8G_HP 72  // row pitch of the f16 operands in LDS, halves (144 bytes)
+
+// four signed bytes as f16: 1024 + (q + 128) by its bit pattern, minus 1152
+__device__ __forceinline__ q8_v4h i8x4_to_f16(uint32_t q) {
+    const uint32_t u = q ^ 0x80808080u;
+    const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);
+    const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
+    const q8_v2h off = {(_Float16)1152.0f, (_Float16)1152.0f};
+    const q8_v2h a = __builtin_bit_cast(q8_v2h, lo) - off, b = __builtin_bit_cast(q8_v2h, hi) - off;
+    return q8_v4h{a[0], a[1], b[0], b[1]};
+}
+
+__global__ __launch_bounds__(256, 2) void gemm_q8_0_q8k_kernel(Q80GemmArgs G) {
+    __shared__ __align__(16) _Float16 s_x[2][64 * Q8G_HP], s_w[2][64 * Q8G_HP];
+    __shared__ float s_d[2][2][64];
+    int row0;
+    const Q80BatchArgs A = q80_gemm_pick(G, row0);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, h = lane >> 5, wr = wave & 1, wt = wave >> 1, t0 = blockIdx.y * 64;
+    const int K = A.K, nc = K >> 6;
+    // thread t stages quants 8 (t % 4) .. + 7 of both blocks of token / row t / 4:
+    // the first four are chain 2 (t % 4), the others the next
+    const int part = tid & 3, r = tid >> 2;
+    const int8_t *xr = A.qs + (int64_t)min(t0 + r, A.T - 1) * K + 8 * part;
+    const uint8_t *wr0 = A.w + (int64_t)min(row0 + r, A.rows - 1) * A.row_stride;
+    uint2 xq[2], wq[2];
+    uint16_t wd[2];
+    auto load = [&](int c) {
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            xq[o] = *(const uint2 *)(xr + 64 * c + 32 * o);
+            const uint8_t *blk = wr0 + (int64_t)(2 * c + o) * 34;
+            wd[o] = ld2(blk);
+            wq[o] = ld8(blk + 2 + 8 * part);
+        }
+    };
+    // LDS row: [block][h][u][4 halves]
+    auto store = [&](int c) {
+        _Float16 *dx = s_x[c & 1] + r * Q8G_HP + 4 * part, *dw = s_w[c & 1] + r * Q8G_HP + 4 * part;
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            *(q8_v4h *)(dx + 32 * o) = i8x4_to_f16(xq[o].x);
+            *(q8_v4h *)(dx + 32 * o + 16) = i8x4_to_f16(xq[o].y);
+            *(q8_v4h *)(dw + 32 * o) = i8x4_to_f16(wq[o].x);
+            *(q8_v4h *)(dw + 32 * o + 16) = i8x4_to_f16(wq[o].y);
+            if (part == 0) s_d[c & 1][o][r] = h2f(wd[o]);
+        }
+    };
+    q8_v16f acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) acc[j] = q8_v16f{};
+    q8_v4f dt[4];  // the scales of the lane's 16 tokens for the 256-element block in hand
+    load(0);
+    store(0);
+    load(min(1, nc - 1));
+    for (int c = 0; c < nc; c++) {
+        __syncthreads();  // chunk c is in LDS; chunk c - 1's reads are done
+        if ((c & 3) == 0) {
+            // ldx is a multiple of 64 >= T: the tile's 64 scales exist
+            const float *p = A.dx + (int64_t)(c >> 2) * A.ldx + t0 + 32 * wt + 4 * h;
+#pragma unroll
+            for (int q = 0; q < 4; q++) dt[q] = *(const q8_v4f *)(p + 8 * q);
+        }
+        if (c + 1 < nc) store(c + 1);
+        if (c + 2 < nc) load(c + 2);
+        const _Float16 *xa = s_x[c & 1] + (32 * wt + n) * Q8G_HP + 16 * h;
+        const _Float16 *wa = s_w[c & 1] + (32 * wr + n) * Q8G_HP + 16 * h;
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            const float d = s_d[c & 1][o][32 * wr + n];
+            float sc[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) sc[i] = dt[i >> 2][i & 3] * d;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const q8_v4h a = *(const q8_v4h *)(xa + 32 * o + 4 * u), b = *(const q8_v4h *)(wa + 32 * o + 4 * u);
+                const q8_v32f s = __builtin_amdgcn_mfma_f32_32x32x4f16(a, b, q8_v32f{}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    acc[2 * u][i] = fmaf(sc[i], s[i], acc[2 * u][i]);
+                    acc[2 * u + 1][i] = fmaf(sc[i], s[16 + i], acc[2 * u + 1][i]);
+                }
+            }
+        }
+    }
+    q80_gemm_store(A, acc, row0 + 32 * wr + n, t0 + 32 * wt, h);
+}
+
 // Router selection of T tokens (moe_topk_kernel per token): logits [T][ldl],
 // sel / prob [T][k].  grid T.
 __global__ __launch_bounds__(64) void moe_topk_batch_kernel(const float *logits, int ldl, int n, int k, int32_t *sel,

@@ -2860,48 +2860,89 @@ static int experts_enqueue(MxExpArgs A, int n_mats, bool mfma, int32_t *lists, i
     return 1;
 }
 
-// y[t][r] (=, or += with EPI_ADD) Q8_0 row r of W times token t (+ bias):
-// f32 activations x [T][K] or the batched Q8_K in bq, as cat_of picks for K.
-static int q80_batch_enqueue(const DevW &W, int rows, int K, int T, const float *x, const BatchXq *bq,
-                             const float *bias, float *y, int ldy, int epi, const char *name, hipStream_t s) {
-    if (W.fmt != 8 || T <= 0) return 0;
-    Q80BatchArgs A;
-    memset(&A, 0, sizeof(A));
-    A.w = W.p;
-    A.row_stride = W.stride;
-    A.rows = rows;
-    A.K = K;
-    A.T = T;
-    A.epi = epi;
-    A.bias = bias;
-    A.y = y;
-    A.ldy = ldy;
+// Whether a Q8_0 batch of n matrices (tiles 64-row tiles in all) goes to the
+// matrix-core kernels.  Their shortest launch takes K's whole loop, 75 us with
+// f32 activations (K = 2880) and 104 with int8 ones (K = 4096); the per-row
+// kernel's take about 24 us per launch plus 0.033 us per tile and token (f32),
+// or 45 plus 0.02 (int8).  Measured, matrix cores against per-row kernel, us:
+// q/k/v in one launch against three (80 tiles): 4 tokens 74 : 77, 33 tokens
+// 77 : 148, 1001 tokens 300 : 2253; router (1 tile) 1001 tokens 77 : 25; wo
+// (int8, 45 tiles): 33 tokens 106 : 63, 65 tokens 104 : 86, 129 tokens 105 :
+// 169, 1001 tokens 212 : 975.
+static bool q80_gemm_pays(int cat, int n, int64_t tiles, int64_t T) {
+    if (cat == CAT_F32) return tiles * T >= (n == 3 ? 256 : n == 2 ? 900 : 1536);
+    return tiles * T >= 3584;
+}
+
+// y[t][r] (=, or += with EPI_ADD) Q8_0 row r of W times token t (+ bias) for
+// n <= 3 matrices of the same K: f32 activations x [T][K] or the batched Q8_K
+// in bq, as cat_of picks for K.
+struct Q80Mat {
+    const DevW *w;
+    int rows;
+    const float *bias;
+    float *y;
+    int ldy;
+};
+static int q80_batch_enqueue(const Q80Mat *ms, int n, int K, int T, const float *x, const BatchXq *bq, int epi,
+                             const char *name, hipStream_t s) {
     const int cat = cat_of(8, K);
-    ProfScope ps(name, s);
-    const dim3 rg((unsigned)((rows + 31) / 32));
-    if (cat == CAT_F32) {
-        if (!x || K % 4 != 0) return 0;
+    if (n < 1 || n > 3 || T <= 0 || (cat != CAT_F32 && cat != CAT_Q8I)) return 0;
+    if (cat == CAT_F32 ? (!x || K % 4 != 0) : !bq) return 0;
+    Q80GemmArgs G;
+    memset(&G, 0, sizeof(G));
+    int tiles = 0;
+    for (int i = 0; i < n; i++) {
+        if (ms[i].w->fmt != 8) return 0;
+        Q80BatchArgs &A = G.m[i];
+        A.w = ms[i].w->p;
+        A.row_stride = ms[i].w->stride;
+        A.rows = ms[i].rows;
+        A.K = K;
+        A.T = T;
+        A.epi = epi;
+        A.bias = ms[i].bias;
+        A.y = ms[i].y;
+        A.ldy = ms[i].ldy;
         A.x = x;
-        if (K <= 4096)
-            rh_launch((gemv_q8_0_batch_kernel<true, 4>), dim3(rg.x, (unsigned)((T + 3) / 4)), dim3(256),
-                      (size_t)4 * K * 4, s, A);
-        else
-            rh_launch((gemv_q8_0_batch_kernel<true, 1>), dim3(rg.x, (unsigned)T), dim3(256), (size_t)K * 4, s, A);
-    } else if (cat == CAT_Q8I) {
-        if (!bq) return 0;
-        A.qs = bq->qs;
-        A.dx = bq->dx;
-        A.ldx = bq->ldx;
-        if (K <= 8192)
-            rh_launch((gemv_q8_0_batch_kernel<false, 8>), dim3(rg.x, (unsigned)((T + 7) / 8)), dim3(256),
-                      (size_t)8 * K + 8 * (K / 256) * 4, s, A);
-        else
-            rh_launch((gemv_q8_0_batch_kernel<false, 2>), dim3(rg.x, (unsigned)((T + 1) / 2)), dim3(256),
-                      (size_t)2 * K + 2 * (K / 256) * 4, s, A);
-    } else {
-        return 0;
+        if (bq) {
+            A.qs = bq->qs;
+            A.dx = bq->dx;
+            A.ldx = bq->ldx;
+        }
+        tiles += (A.rows + 63) / 64;
+        G.tiles[i] = tiles;
     }
-    RH_LAUNCH_OK();
+    for (int i = n; i < 3; i++) G.tiles[i] = tiles;
+    ProfScope ps(name, s);
+    if (q80_gemm_pays(cat, n, tiles, T)) {
+        const dim3 grid((unsigned)tiles, (unsigned)((T + 63) / 64));
+        if (cat == CAT_F32)
+            rh_launch(gemm_q8_0_f32_kernel, grid, dim3(256), 0, s, G);
+        else
+            rh_launch(gemm_q8_0_q8k_kernel, grid, dim3(256), 0, s, G);
+        RH_LAUNCH_OK();
+        return 1;
+    }
+    for (int i = 0; i < n; i++) {
+        const Q80BatchArgs &A = G.m[i];
+        const unsigned rg = (unsigned)((A.rows + 31) / 32);
+        if (cat == CAT_F32) {
+            if (K <= 4096)
+                rh_launch((gemv_q8_0_batch_kernel<true, 4>), dim3(rg, (unsigned)((T + 3) / 4)), dim3(256),
+                          (size_t)4 * K * 4, s, A);
+            else
+                rh_launch((gemv_q8_0_batch_kernel<true, 1>), dim3(rg, (unsigned)T), dim3(256), (size_t)K * 4, s, A);
+        } else {
+            if (K <= 8192)
+                rh_launch((gemv_q8_0_batch_kernel<false, 8>), dim3(rg, (unsigned)((T + 7) / 8)), dim3(256),
+                          (size_t)8 * K + 8 * (K / 256) * 4, s, A);
+            else
+                rh_launch((gemv_q8_0_batch_kernel<false, 2>), dim3(rg, (unsigned)((T + 1) / 2)), dim3(256),
+                          (size_t)2 * K + 2 * (K / 256) * 4, s, A);
+        }
+        RH_LAUNCH_OK();
+    }
     return 1;
 }
 
@@ -2954,10 +2995,10 @@ static int r_prefill_chunk_moe(const int32_t *tok, int T, int pos0, hipStream_t 
         RLayer &Ly = R.L[l];
         const MoeDev &M = Ly.moe;
         if (!r_norm_batch_moe(Ly.attn_norm, T, bd, s)) return 0;
-        if (!q80_batch_enqueue(Ly.w[0], qd, dim, T, R.pxn, &bd, Ly.bias[0], R.pq, qd, EPI_STORE, "pf_q80_q", s) ||
-            !q80_batch_enqueue(Ly.w[1], kd, dim, T, R.pxn, &bd, Ly.bias[1], R.pk, kd, EPI_STORE, "pf_q80_k", s) ||
-            !q80_batch_enqueue(Ly.w[2], vdim, dim, T, R.pxn, &bd, Ly.bias[2], R.pv, vdim, EPI_STORE, "pf_q80_v", s))
-            return 0;
+        const Q80Mat qkv[3] = {{&Ly.w[0], qd, Ly.bias[0], R.pq, qd},
+                               {&Ly.w[1], kd, Ly.bias[1], R.pk, kd},
+                               {&Ly.w[2], vdim, Ly.bias[2], R.pv, vdim}};
+        if (!q80_batch_enqueue(qkv, 3, dim, T, R.pxn, &bd, EPI_STORE, "pf_q80_qkv", s)) return 0;
         if (!kv_ring_copy(Ly, P0, npre, 0, 0, s)) return 0;
         {
             RopeArgs A;
@@ -3023,15 +3064,14 @@ static int r_prefill_chunk_moe(const int32_t *tok, int T, int pos0, hipStream_t 
         }
         if (!kv_ring_copy(Ly, last0, pos0 + T - last0, last0 - P0, 1, s)) return 0;
         // x += wo attn + bo (src/model.rs:6837-6840)
-        if (!q80_batch_enqueue(Ly.w[3], dim, attn_cols, T, nullptr, &ba, Ly.bo, R.px, dim, EPI_ADD, "pf_q80_o", s))
-            return 0;
+        const Q80Mat wo = {&Ly.w[3], dim, Ly.bo, R.px, dim};
+        if (!q80_batch_enqueue(&wo, 1, attn_cols, T, nullptr, &ba, EPI_ADD, "pf_q80_o", s)) return 0;
         // xn2 = rms_norm(x, post_attn_norm); x += moe(xn2) (src/model.rs:6846-6898)
         if (!r_norm_batch_moe(Ly.ffn_norm, T, bd, s)) return 0;
         const int k = M.k, hid = M.hidden, np = T * k;
         const bool mfma = expert_mfma_on();
-        if (!q80_batch_enqueue(M.router, M.n_exp, dim, T, R.pxn, &bd, M.router_bias, R.plog, 64, EPI_STORE,
-                               "pf_router", s))
-            return 0;
+        const Q80Mat router = {&M.router, M.n_exp, M.router_bias, R.plog, 64};
+        if (!q80_batch_enqueue(&router, 1, dim, T, R.pxn, &bd, EPI_STORE, "pf_router", s)) return 0;
         {
             ProfScope ps("moe_topk_batch", s);
             rh_launch(moe_topk_batch_kernel, dim3((unsigned)T), dim3(64), 0, s, (const float *)R.plog, 64, M.n_exp, k,
