@@ -15,13 +15,12 @@
 //   Q4_K: two x32 MFMAs per 32-element sub-block on the nibbles times the
 //         two base-8 digits of the sub-block scale, accumulated over the
 //         block, so isum = sum_j sc_j * C_j (C_j = sum q x) exactly; imin =
-//         sum_j m_j * bsums_j = sum_e m_j(e) * x_e is one more MFMA per
-//         sub-block with m_j as the B operand; value = dx * (d*isum -
-//         dmin*imin).
+//         sum_j m_j * bsums_j is one f16 MFMA per block on the sums of 16
+//         quants; value = dx * (d*isum - dmin*imin).
 //   Q6_K: one x16 MFMA per 16-element scale group on q - 32 as signed
 //         bytes, isum += sc_g * C_g; value = (dx*d) * isum.
-// Rows and tokens past the ends read clamped (in-bounds) data and are not
-// stored.
+// Rows and tokens past the ends read clamped (in-bounds) data or zeros and
+// are not stored.
 #pragma once
 #include "common.hpp"
 #include "gemv.hip"
@@ -31,17 +30,23 @@ namespace rh {
 typedef int rh_v4i __attribute__((ext_vector_type(4)));
 typedef int rh_v16i __attribute__((ext_vector_type(16)));
 
-struct GemmArgs {
+struct GemmOut {
     const uint8_t *w;
     int64_t row_stride;
-    int32_t rows, K, T;
+    float *y;
+    const float *bias;  // [rows] or null
+    int32_t rows;
+    int32_t ldy;        // y[t * ldy + r]
+    int32_t tiles;      // 128-row tiles up to and including this matrix
+};
+struct GemmArgs {
+    GemmOut m[2];       // (m[1] in two-matrix Q4_K launches)
+    int32_t K, T;
     int32_t epi;        // EPI_STORE or EPI_ADD
     const int8_t *xq;   // [T][K] Q8_K quants, token-major
     const float *dx;    // [K/256][ldx] Q8_K scales, token-minor
-    int32_t ldx;        // >= T, a multiple of 4
-    int32_t ldy;        // y[t * ldy + r]
-    float *y;
-    const float *bias;  // [rows] or null
+    const _Float16 *hs; // [K/256][ldx][16] sums of 16 quants
+    int32_t ldx;        // >= T, a multiple of 64
 };
 
 // Q6_K bytes q (0..63, four per dword) as signed q - 32: (q + 0x60) ^ 0x80
@@ -49,9 +54,6 @@ struct GemmArgs {
 // and one xor per dword; a copy of bit 5 into bits 6 and 7 compiled to a
 // quarter-rate multiply by 6).
 __device__ __forceinline__ uint32_t q6_signed4(uint32_t q) { return (q + 0x60606060u) ^ 0x80808080u; }
-
-// Byte m (< 256) in all four bytes of a dword (one v_perm_b32).
-__device__ __forceinline__ int bcast_byte(int m) { return (int)__builtin_amdgcn_perm(0u, (uint32_t)m, 0u); }
 
 // One block of the lane's weight row, as the lane's MFMA B operands need it
 // (lane half h = lane / 32 takes k = 16h.. of each 32-element Q4_K sub-block,
@@ -92,8 +94,6 @@ __device__ __forceinline__ void gemm_w_load(GemmW<F_Q6_K> &W, const uint8_t *blk
 // touches start 4 banks apart.
 #define GEMM_XS 272
 
-// Integer sums of block b for the wave's 32 rows x 32*NT tokens: isum (and
-// for Q4_K imin) per C element, from the activation tile xs.
 typedef unsigned short rh_u16x2 __attribute__((ext_vector_type(2)));
 
 // Each byte of the four dwords of x (nibbles, < 16) times s (< 8): one packed
@@ -110,60 +110,12 @@ __device__ __forceinline__ rh_v4i bytes_times(const rh_v4i &x, int s) {
     return r;
 }
 
-// Q4_K: the sub-block scale (6 bits) enters the B operand as two digits, sc
-// = 8 * (sc >> 3) + (sc & 7), each digit times a nibble fitting a signed
-// byte, so that the MFMAs accumulate the whole block: isum = 8 * hi + lo =
-// sum_j sc_j * C_j exactly (the same integer as one MFMA per sub-block scaled
-// afterwards, with no per-sub-block multiply-add on the vector ALU).
-template <int NT>
-__device__ __forceinline__ void gemm_block_ints(const GemmW<F_Q4_K> &W, const int8_t *xs, int lane,
-                                                int (&isum)[NT][16], rh_v16i (&imin)[NT]) {
-    const int half = lane >> 5, n = lane & 31;
-    rh_v16i ahi[NT], alo[NT];
-#pragma unroll
-    for (int tt = 0; tt < NT; tt++) {
-        imin[tt] = rh_v16i{};
-        ahi[tt] = rh_v16i{};
-        alo[tt] = rh_v16i{};
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        int sc0, m0, sc1, m1;
-        scale_min_k4(2 * q, W.hdr.y, W.hdr.z, W.hdr.w, sc0, m0);
-        scale_min_k4(2 * q + 1, W.hdr.y, W.hdr.z, W.hdr.w, sc1, m1);
-        const uint4 qs = W.qs[q];
-        const rh_v4i blo = {(int)(qs.x & 0x0F0F0F0Fu), (int)(qs.y & 0x0F0F0F0Fu), (int)(qs.z & 0x0F0F0F0Fu),
-                            (int)(qs.w & 0x0F0F0F0Fu)};
-        const rh_v4i bhi = {(int)((qs.x >> 4) & 0x0F0F0F0Fu), (int)((qs.y >> 4) & 0x0F0F0F0Fu),
-                            (int)((qs.z >> 4) & 0x0F0F0F0Fu), (int)((qs.w >> 4) & 0x0F0F0F0Fu)};
-        const rh_v4i l8 = bytes_times(blo, sc0 >> 3), l1 = bytes_times(blo, sc0 & 7);
-        const rh_v4i h8 = bytes_times(bhi, sc1 >> 3), h1 = bytes_times(bhi, sc1 & 7);
-        const int mb0 = bcast_byte(m0), mb1 = bcast_byte(m1);
-        const rh_v4i bm0 = {mb0, mb0, mb0, mb0}, bm1 = {mb1, mb1, mb1, mb1};
-#pragma unroll
-        for (int tt = 0; tt < NT; tt++) {
-            const int8_t *xr = xs + (32 * tt + n) * GEMM_XS + 64 * q + 16 * half;
-            const rh_v4i a0 = *(const rh_v4i *)xr;
-            const rh_v4i a1 = *(const rh_v4i *)(xr + 32);
-            ahi[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, l8, ahi[tt], 0, 0, 0);
-            alo[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, l1, alo[tt], 0, 0, 0);
-            imin[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, bm0, imin[tt], 0, 0, 0);
-            ahi[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, h8, ahi[tt], 0, 0, 0);
-            alo[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, h1, alo[tt], 0, 0, 0);
-            imin[tt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, bm1, imin[tt], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int tt = 0; tt < NT; tt++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) isum[tt][i] = (ahi[tt][i] << 3) + alo[tt][i];
-}
-
+// Integer sums of a block for the wave's 32 rows x 32*NT tokens: isum per C
+// element, from the activation tile xs.
 template <int NT>
 __device__ __forceinline__ void gemm_block_ints(const GemmW<F_Q6_K> &W, const int8_t *xs, int lane,
-                                                int (&isum)[NT][16], rh_v16i (&imin)[NT]) {
+                                                int (&isum)[NT][16]) {
     const int half = lane >> 5, n = lane & 31;
-    (void)imin;
 #pragma unroll
     for (int tt = 0; tt < NT; tt++)
 #pragma unroll
@@ -200,132 +152,217 @@ __device__ __forceinline__ void gemm_block_ints(const GemmW<F_Q6_K> &W, const in
         }
 }
 
-// Workgroup: 4 waves x 32 weight rows, 32*NT tokens.  Per block: the next
-// block's weights (registers) and activation tile (registers, then the other
-// LDS buffer) are loaded while this block's MFMAs and combine run; one
-// barrier per block.  Waves past the last row compute clamped rows and store
-// nothing, so every wave reaches every barrier.
-template <int FMT, int NT>
-__global__ __launch_bounds__(256) void gemm_kq_mfma_kernel(GemmArgs A) {
-    extern __shared__ __align__(16) int8_t s_xs[];  // [2][32*NT][GEMM_XS]
-    constexpr int TOK = 32 * NT;
-    constexpr int NLD = TOK * 16 / 256;  // 16-byte activation pieces per thread per block
+// Q4_K products: a workgroup is 128 weight rows (a wave 32) by 32 NT tokens.
+//
+// The sub-block scale (6 bits) enters the B operand as two digits, sc = 8 (sc
+// >> 3) + (sc & 7), each digit times a nibble fitting a signed byte, so the
+// MFMAs accumulate the whole block: isum = 8 hi + lo = sum_j sc_j C_j exactly.
+// The minimums' sum imin = sum_j m_j (sum of sub-block j) is one 32x32x16 f16
+// MFMA on the sums of 16 quants that the quantizers leave: |sum| <= 2048 and
+// m <= 63 are exact in f16 and every partial sum is an integer below 2^22, so
+// the f32 result is the integer (exactness of such sums checked on the
+// device), and it arrives as the float the combine wants.
+//
+// Per 32 x 32 outputs and block the VALU does the reference's combine, 7
+// operations on 16 elements, which nothing can fold, and the wave decodes its
+// 32 rows once, about 150 instructions, for its NT token tiles: the digits stay
+// in 64 registers.  The activation tile (quants, sums, scales) is double-buffered in
+// LDS and shared by the four waves; the next block's comes through registers, a
+// few 16-byte pieces per token tile a block ahead (loaded at the tile they are
+// stored after, the 28672 x 4096 product took 176 us instead of 160), and its
+// weights straight after the digits are made.  One barrier per block.
+//
+// Bound by the VALU: 200 instructions per 32 x 32 outputs and block with NT =
+// 2 (390 with a minimum MFMA per sub-block and one token tile), about 60% busy;
+// the waits are the barrier and the start of each tile.  Gate and up of an
+// 8B-class model, 28672 x 4096, 512 tokens in one launch: 161 us (747 TOP/s);
+// two launches of the one-tile kernel before, 244.  Measured and dropped: four
+// token tiles (spills at two waves per SIMD: 189 us); each row tile's token
+// tiles on one XCD (160).
+typedef _Float16 rh_v8h __attribute__((ext_vector_type(8)));
+typedef float rh_v16f __attribute__((ext_vector_type(16)));
+typedef float rh_v4f __attribute__((ext_vector_type(4)));
+
+// One block of the lane's Q4_K row as MFMA B operands: per 64 weights the low
+// nibbles times the high and low scale digit, then the high nibbles likewise;
+// the minimums of this lane half's eight groups of 16 (sub-blocks 4 half .. +
+// 3, each twice); d and dmin.
+struct Q4kOps {
+    rh_v4i dig[4][4];
+    rh_v8h bm;
+    float d, dmin;
+};
+__device__ __forceinline__ void q4k_decode(Q4kOps &O, const GemmW<F_Q4_K> &W, int half) {
+    const uint4 hdr = W.hdr;
+    O.d = h2f((uint16_t)hdr.x);
+    O.dmin = h2f((uint16_t)(hdr.x >> 16));
+    // scales and minimums of the eight sub-blocks, one per byte
+    const uint32_t sc03 = hdr.y & 0x3F3F3F3Fu, sc47 = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
+    const uint32_t mn = half ? ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u) : hdr.z & 0x3F3F3F3Fu;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint32_t sw = q < 2 ? sc03 : sc47;
+        const int s0 = (sw >> (16 * (q & 1))) & 0xFF, s1 = (sw >> (16 * (q & 1) + 8)) & 0xFF;
+        const uint32_t w4[4] = {W.qs[q].x, W.qs[q].y, W.qs[q].z, W.qs[q].w};
+        rh_v4i lo, hi;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            lo[i] = (int)(w4[i] & 0x0F0F0F0Fu);
+            hi[i] = (int)((w4[i] >> 4) & 0x0F0F0F0Fu);
+        }
+        O.dig[q][0] = bytes_times(lo, s0 >> 3);
+        O.dig[q][1] = bytes_times(lo, s0 & 7);
+        O.dig[q][2] = bytes_times(hi, s1 >> 3);
+        O.dig[q][3] = bytes_times(hi, s1 & 7);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const _Float16 m = (_Float16)(float)((mn >> (8 * i)) & 0xFF);
+        O.bm[2 * i] = m;
+        O.bm[2 * i + 1] = m;
+    }
+}
+
+// The block's values dx (d isum - dmin imin) of 32 rows x 32 tokens: xr the
+// lane's token row of the LDS tile (+ 16 half), hs its sums, dv(g) the scales
+// of tokens 8 g + 4 half ..; out(i, value) takes C element i's.
+template <class Dv, class Out>
+__device__ __forceinline__ void q4k_tile(const Q4kOps &O, const int8_t *xr, rh_v8h hs, Dv dv, Out out) {
+    rh_v16i hi = {}, lo = {};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const rh_v4i a0 = *(const rh_v4i *)(xr + 64 * q), a1 = *(const rh_v4i *)(xr + 64 * q + 32);
+        hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, O.dig[q][0], hi, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, O.dig[q][1], lo, 0, 0, 0);
+        hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, O.dig[q][2], hi, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, O.dig[q][3], lo, 0, 0, 0);
+    }
+    const rh_v16f im = __builtin_amdgcn_mfma_f32_32x32x16_f16(hs, O.bm, rh_v16f{}, 0, 0, 0);
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const rh_v4f dx = dv(g);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int i = 4 * g + r;
+            const float t1 = O.d * (float)((hi[i] << 3) + lo[i]);
+            const float t2 = O.dmin * im[i];
+            out(i, dx[r] * (t1 - t2));
+        }
+    }
+}
+
+constexpr int gemm_q4k_buf(int nt) { return 32 * nt * (GEMM_XS + 32 + 4); }
+constexpr int gemm_q4k_lds(int nt) { return 2 * gemm_q4k_buf(nt); }
+
+template <int NT>
+__global__ __launch_bounds__(256, 2) void gemm_q4k_mfma_kernel(GemmArgs A) {
+    extern __shared__ __align__(16) int8_t s_xt[];  // [2]: quants [TOK][GEMM_XS], sums [TOK][16] f16, scales [TOK]
+    constexpr int TOK = 32 * NT, HS0 = TOK * GEMM_XS, DX0 = HS0 + TOK * 32, BUF = gemm_q4k_buf(NT);
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r0 = (blockIdx.x * 4 + wave) * 32;
-    const int t0 = blockIdx.y * TOK;
-    const int row = min(r0 + n, A.rows - 1);
-    const uint8_t *wr = A.w + (int64_t)row * A.row_stride;
+    const int bx = blockIdx.x, by = blockIdx.y;
+    const bool m1 = bx >= A.m[0].tiles;
+    const int rows = m1 ? A.m[1].rows : A.m[0].rows;
+    const int r0 = (bx - (m1 ? A.m[0].tiles : 0)) * 128 + 32 * wave;
+    const int t0 = by * TOK;
+    const uint8_t *wr = (m1 ? A.m[1].w : A.m[0].w) +
+                        (int64_t)min(r0 + n, rows - 1) * (m1 ? A.m[1].row_stride : A.m[0].row_stride);
     const int nb = A.K >> 8;
-    constexpr int BB = FMT == F_Q4_K ? 144 : 210;
-    // activation pieces: thread -> (token, 16-byte part)
-    const int8_t *xsrc[NLD];
-    int xdst[NLD];
+    // activation pieces: piece j of thread t is part t % 16 of token t / 16 + 16 j;
+    // tokens past the batch read zeros (their outputs are not stored)
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(A.xq + (int64_t)t0 * A.K), (short)0, (int)min((int64_t)(A.T - t0), (int64_t)TOK) * A.K, 0x00020000);
+    const int xoff = (tid >> 4) * A.K + 16 * (tid & 15), xdst = (tid >> 4) * GEMM_XS + 16 * (tid & 15);
+    const int ht = min(t0 + min(tid, 2 * TOK - 1) / 2, A.T - 1), dt = min(t0 + min(tid, TOK - 1), A.T - 1);
+    auto load_x = [&](int b, int j) {
+        return __builtin_amdgcn_raw_buffer_load_b128(xres, xoff, 16 * j * A.K + 256 * b, 0);
+    };
+    typedef decltype(__builtin_amdgcn_raw_buffer_load_b128(xres, 0, 0, 0)) piece_t;
+    GemmW<F_Q4_K> W;
+    auto load_w = [&](int b) { gemm_w_load(W, wr + (int64_t)b * 144, half); };
+    rh_v4i hsr;
+    float dxr = 0.0f;
+    auto load_hd = [&](int b) {
+        if (tid < 2 * TOK) hsr = *(const rh_v4i *)(A.hs + ((int64_t)b * A.ldx + ht) * 16 + 8 * (tid & 1));
+        if (tid < TOK) dxr = A.dx[(int64_t)b * A.ldx + dt];
+    };
+    auto store_hd = [&](int8_t *buf) {
+        if (tid < 2 * TOK) *(rh_v4i *)(buf + HS0 + 16 * tid) = hsr;
+        if (tid < TOK) *(float *)(buf + DX0 + 4 * tid) = dxr;
+    };
+    piece_t st[2 * NT];
+    load_w(0);
+    load_hd(0);
 #pragma unroll
-    for (int j = 0; j < NLD; j++) {
-        const int p = tid + 256 * j, tok = p >> 4, part = p & 15;
-        xsrc[j] = A.xq + (int64_t)min(t0 + tok, A.T - 1) * A.K + 16 * part;
-        xdst[j] = tok * GEMM_XS + 16 * part;
-    }
-    GemmW<FMT> W;
-    gemm_w_load(W, wr, half);
-    {
-        uint4 st[NLD];
+    for (int j = 0; j < 2 * NT; j++) st[j] = load_x(0, j);
 #pragma unroll
-        for (int j = 0; j < NLD; j++) st[j] = *(const uint4 *)xsrc[j];
+    for (int j = 0; j < 2 * NT; j++) *(piece_t *)(s_xt + xdst + 16 * j * GEMM_XS) = st[j];
+    store_hd(s_xt);
+    load_hd(min(1, nb - 1));
 #pragma unroll
-        for (int j = 0; j < NLD; j++) *(uint4 *)(s_xs + xdst[j]) = st[j];
-    }
-    __syncthreads();
+    for (int j = 0; j < 2 * NT; j++) st[j] = load_x(min(1, nb - 1), j);
     float acc[NT][16];
 #pragma unroll
     for (int tt = 0; tt < NT; tt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[tt][i] = 0.0f;
-
+    __syncthreads();
     for (int b = 0; b < nb; b++) {
-        const bool more = b + 1 < nb;
-        const int bn = more ? b + 1 : b;
-        GemmW<FMT> Wn;
-        gemm_w_load(Wn, wr + (int64_t)bn * BB, half);
-        uint4 st[NLD];
+        const int8_t *cur = s_xt + (b & 1) * BUF;
+        int8_t *nxt = s_xt + ((b + 1) & 1) * BUF;
+        const int bn = min(b + 1, nb - 1);  // (the last block stages itself again, unread)
+        Q4kOps O;
+        q4k_decode(O, W, half);
+        load_w(bn);
+        // the next block's activations, loaded a block ago, then the one after
+        store_hd(nxt);
 #pragma unroll
-        for (int j = 0; j < NLD; j++) st[j] = *(const uint4 *)(xsrc[j] + 256 * bn);
-        // this block's activation scales, four consecutive tokens per load:
-        // token of C element i = 8*(i/4) + 4*half + i%4
-        float4 dv[NT][4];
+        for (int j = 0; j < 2 * NT; j++) *(piece_t *)(nxt + xdst + 16 * j * GEMM_XS) = st[j];
+        const int b2 = min(b + 2, nb - 1);
+        load_hd(b2);
 #pragma unroll
-        for (int tt = 0; tt < NT; tt++)
+        for (int j = 0; j < 2 * NT; j++) st[j] = load_x(b2, j);
 #pragma unroll
-            for (int g4 = 0; g4 < 4; g4++)
-                dv[tt][g4] = *(const float4 *)(A.dx + (int64_t)b * A.ldx + t0 + 32 * tt + 4 * half + 8 * g4);
-        int isum[NT][16];
-        rh_v16i imin[NT];
-        gemm_block_ints<NT>(W, s_xs + (b & 1) * TOK * GEMM_XS, lane, isum, imin);
-        float d, dmin = 0.0f;
-        if constexpr (FMT == F_Q4_K) {
-            d = h2f(W.hdr.x & 0xFFFF);
-            dmin = h2f(W.hdr.x >> 16);
-        } else {
-            d = h2f(W.d & 0xFFFF);
-        }
-        // the reference's per-block combine, accumulated in block order
-#pragma unroll
-        for (int tt = 0; tt < NT; tt++)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; g4++) {
-                const float dxs[4] = {dv[tt][g4].x, dv[tt][g4].y, dv[tt][g4].z, dv[tt][g4].w};
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int i = 4 * g4 + r;
-                    float v;
-                    if constexpr (FMT == F_Q4_K) {
-                        const float t1 = d * (float)isum[tt][i];
-                        const float t2 = dmin * (float)imin[tt][i];
-                        v = dxs[r] * (t1 - t2);
-                    } else {
-                        v = (dxs[r] * d) * (float)isum[tt][i];
-                    }
-                    acc[tt][i] += v;
-                }
-            }
-        if (more) {
-#pragma unroll
-            for (int j = 0; j < NLD; j++) *(uint4 *)(s_xs + ((b + 1) & 1) * TOK * GEMM_XS + xdst[j]) = st[j];
+        for (int tt = 0; tt < NT; tt++) {
+            // the reference's per-block combine, accumulated in block order
+            q4k_tile(
+                O, cur + (32 * tt + n) * GEMM_XS + 16 * half,
+                *(const rh_v8h *)(cur + HS0 + (32 * tt + n) * 32 + 16 * half),
+                [&](int g) { return *(const rh_v4f *)(cur + DX0 + 4 * (32 * tt + 8 * g + 4 * half)); },
+                [&](int i, float v) { acc[tt][i] += v; });
         }
         __syncthreads();
-        W = Wn;
     }
-    if (r0 + n >= A.rows) return;
-    const float bias = A.bias ? A.bias[r0 + n] : 0.0f;
+    if (r0 + n >= rows) return;
+    const float *bp = m1 ? A.m[1].bias : A.m[0].bias;
+    const float bias = bp ? bp[r0 + n] : 0.0f;
+    const int ldy = m1 ? A.m[1].ldy : A.m[0].ldy;
+    float *y = (m1 ? A.m[1].y : A.m[0].y) + r0 + n;
 #pragma unroll
     for (int tt = 0; tt < NT; tt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * half + (i & 3);
             if (t >= A.T) continue;
-            float *yp = A.y + (int64_t)t * A.ldy + r0 + n;
             float v = acc[tt][i];
-            if (A.bias) v = v + bias;
+            if (bp) v = v + bias;
             if (A.epi == EPI_ADD)
-                *yp += v;
+                y[(int64_t)t * ldy] += v;
             else
-                *yp = v;
+                y[(int64_t)t * ldy] = v;
         }
 }
 
 // The same products with the blocks of K split over the workgroup's four
-// waves, for launches with too few (row tile, token tile) pairs to fill the
-// chip (the q/k/v/o projections, the long-K down projection): one workgroup
-// per 32 weight rows x 32 tokens, wave w computing blocks w, w+4, w+8, ...
-// Each wave stages its own block's activations in its own LDS tile, computes
-// the block's per-output value exactly as gemm_kq_mfma_kernel does, and
-// leaves the 16 values of each lane in LDS; after a barrier, wave w adds the
-// round's values of C elements 4w..4w+3 to its accumulators in block order
-// (a barrier before the next round's values are written keeps them until
-// every wave has read these).  Every output is therefore the same sum of
-// the same per-block values in the same order: bit-identical to the
-// one-wave-per-row-tile kernel.
+// waves, for Q6_K and for Q4_K launches with too few (row tile, token tile)
+// pairs to fill the chip: one workgroup per 32 weight rows x 32 tokens, wave w
+// computing blocks w, w+4, w+8, ...  Each wave stages its own block's
+// activations in its own LDS tile, computes the block's per-output value
+// exactly as the unsplit kernel does, and leaves the 16 values of each lane in
+// LDS; after a barrier, wave w adds the round's values of C elements 4w..4w+3
+// to its accumulators in block order (a barrier before the next round's values
+// are written keeps them until every wave has read these).  Every output is
+// therefore the same sum of the same per-block values in the same order.
 template <int FMT>
 __global__ __launch_bounds__(256) void gemm_kq_mfma_ks_kernel(GemmArgs A) {
     __shared__ __align__(16) int8_t s_xs[4][32 * GEMM_XS];  // per wave: 32 token rows of one block
@@ -333,8 +370,8 @@ __global__ __launch_bounds__(256) void gemm_kq_mfma_ks_kernel(GemmArgs A) {
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r0 = blockIdx.x * 32, t0 = blockIdx.y * 32;
-    const int row = min(r0 + n, A.rows - 1);
-    const uint8_t *wr = A.w + (int64_t)row * A.row_stride;
+    const int row = min(r0 + n, A.m[0].rows - 1);
+    const uint8_t *wr = A.m[0].w + (int64_t)row * A.m[0].row_stride;
     const int nb = A.K >> 8, rounds = (nb + 3) >> 2;
     constexpr int BB = FMT == F_Q4_K ? 144 : 210;
     // activation pieces of the wave's block: lane -> (token, 16-byte part),
@@ -363,38 +400,30 @@ __global__ __launch_bounds__(256) void gemm_kq_mfma_ks_kernel(GemmArgs A) {
         b = 4 * it + wave;
         const bool have = b < nb;
         const int bn = min(b + 4, nb - 1);  // the wave's next block (clamped; unused past the end)
+        // this block's scales and sums before the next block's weights: loads
+        // retire in order, and only the former are needed now (rows up to ldx, a
+        // multiple of 64, exist; a wave past the last block reads the last one)
+        const int bc = min(b, nb - 1);
+        rh_v4f dv[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++) dv[g] = *(const rh_v4f *)(A.dx + (int64_t)bc * A.ldx + t0 + 4 * half + 8 * g);
+        rh_v8h hs;
+        if constexpr (FMT == F_Q4_K) hs = *(const rh_v8h *)(A.hs + ((int64_t)bc * A.ldx + t0 + n) * 16 + 8 * half);
         GemmW<FMT> Wn;
         gemm_w_load(Wn, wr + (int64_t)bn * BB, half);
         float v[16] = {};
         if (have) {
-            float4 dv[4];
-#pragma unroll
-            for (int g4 = 0; g4 < 4; g4++)
-                dv[g4] = *(const float4 *)(A.dx + (int64_t)b * A.ldx + t0 + 4 * half + 8 * g4);
-            int isum[1][16];
-            rh_v16i imin[1];
-            gemm_block_ints<1>(W, xs, lane, isum, imin);
-            float d, dmin = 0.0f;
             if constexpr (FMT == F_Q4_K) {
-                d = h2f(W.hdr.x & 0xFFFF);
-                dmin = h2f(W.hdr.x >> 16);
+                Q4kOps O;
+                q4k_decode(O, W, half);
+                q4k_tile(O, xs + n * GEMM_XS + 16 * half, hs, [&](int g) { return dv[g]; },
+                         [&](int i, float val) { v[i] = val; });
             } else {
-                d = h2f(W.d & 0xFFFF);
-            }
+                int isum[1][16];
+                gemm_block_ints<1>(W, xs, lane, isum);
+                const float d = h2f(W.d & 0xFFFF);
 #pragma unroll
-            for (int g4 = 0; g4 < 4; g4++) {
-                const float dxs[4] = {dv[g4].x, dv[g4].y, dv[g4].z, dv[g4].w};
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int i = 4 * g4 + r;
-                    if constexpr (FMT == F_Q4_K) {
-                        const float t1 = d * (float)isum[0][i];
-                        const float t2 = dmin * (float)imin[0][i];
-                        v[i] = dxs[r] * (t1 - t2);
-                    } else {
-                        v[i] = (dxs[r] * d) * (float)isum[0][i];
-                    }
-                }
+                for (int i = 0; i < 16; i++) v[i] = (dv[i >> 2][i & 3] * d) * (float)isum[0][i];
             }
         }
         // the next block's activations, in flight over the barrier (issued
@@ -421,16 +450,16 @@ __global__ __launch_bounds__(256) void gemm_kq_mfma_ks_kernel(GemmArgs A) {
         }
         W = Wn;
     }
-    if (r0 + n >= A.rows) return;
-    const float bias = A.bias ? A.bias[r0 + n] : 0.0f;
+    if (r0 + n >= A.m[0].rows) return;
+    const float bias = A.m[0].bias ? A.m[0].bias[r0 + n] : 0.0f;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const int i = 4 * wave + e;
         const int t = t0 + 8 * (i >> 2) + 4 * half + (i & 3);
         if (t >= A.T) continue;
-        float *yp = A.y + (int64_t)t * A.ldy + r0 + n;
+        float *yp = A.m[0].y + (int64_t)t * A.m[0].ldy + r0 + n;
         float v = acc[e];
-        if (A.bias) v = v + bias;
+        if (A.m[0].bias) v = v + bias;
         if (A.epi == EPI_ADD)
             *yp += v;
         else

@@ -2,7 +2,9 @@
 // src/model.rs:9917-10090) for T tokens in one launch, token = blockIdx.y.
 // Each is the decode step's arithmetic applied to every token row, and each
 // ends in the Q8_K quantization the next batched product reads:
-//   quants [T][K] (token-major) and scales [K/256][ldx] (token-minor).
+//   quants [T][K] (token-major), scales [K/256][ldx] (token-minor) and the
+//   sums of every 16 quants as f16 [K/256][ldx][16] (exact: |sum| <= 2048),
+//   the Q4_K product's operand for the block minimums.
 #pragma once
 #include "attention_exact.hip"
 #include "common.hpp"
@@ -15,22 +17,24 @@ namespace rh {
 // (quantize_row_q8k, src/simd.rs:5013-5101; same arithmetic as
 // q8k_block_store).
 __device__ __forceinline__ void q8k_batch_store(float v, int b, int t, int K, int8_t *qs, float *dx, int ldx,
-                                                float *red) {
+                                                _Float16 *hs, float *red) {
     const float amax = block_max_256(fabsf(v), red);
     const float id = amax > 0.0f ? 127.0f / amax : 0.0f;
     int q = (int)__builtin_rintf(v * id);
     q = max(-128, min(127, q));
     qs[(int64_t)t * K + b * 256 + threadIdx.x] = (int8_t)q;
     if (threadIdx.x == 0) dx[(int64_t)b * ldx + t] = amax * (1.0f / 127.0f);
+    const int sum = row_sum16_i(q);
+    if ((threadIdx.x & 15) == 0) hs[((int64_t)b * ldx + t) * 16 + (threadIdx.x >> 4)] = (_Float16)(float)sum;
 }
 
 // x [T][ldxf] -> Q8_K.  grid (K/256, T).
 __global__ __launch_bounds__(256) void quantize_q8k_batch_kernel(const float *x, int K, int ldxf, int8_t *qs,
-                                                                 float *dx, int ldx) {
+                                                                 float *dx, int ldx, _Float16 *hs) {
     __shared__ float red[4];
     const int b = blockIdx.x, t = blockIdx.y;
     const float v = x[(int64_t)t * ldxf + b * 256 + threadIdx.x];
-    q8k_batch_store(v, b, t, K, qs, dx, ldx, red);
+    q8k_batch_store(v, b, t, K, qs, dx, ldx, hs, red);
 }
 
 // rms_norm_slice_into (src/model.rs:9889-9897, the same arithmetic as
@@ -40,7 +44,7 @@ __global__ __launch_bounds__(256) void quantize_q8k_batch_kernel(const float *x,
 // the block maximum is exact in any order, so the values are
 // q8k_batch_store's).  n a multiple of 256.  grid (T), dynamic LDS n floats.
 __global__ __launch_bounds__(256) void rmsnorm_q8k_batch_kernel(const float *x, const float *w, float eps, int n,
-                                                                int8_t *qs, float *dx, int ldx) {
+                                                                int8_t *qs, float *dx, int ldx, _Float16 *hs) {
     extern __shared__ float s_x[];
     __shared__ float red[40];
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -56,14 +60,18 @@ __global__ __launch_bounds__(256) void rmsnorm_q8k_batch_kernel(const float *x, 
         const float amax = wave_max(fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3]))));
         const float id = amax > 0.0f ? 127.0f / amax : 0.0f;
         uint32_t packed = 0;
+        int sum = 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             int q = (int)__builtin_rintf(o[i] * id);
             q = max(-128, min(127, q));
+            sum += q;
             packed |= (uint32_t)(q & 0xFF) << (8 * i);
         }
         *(uint32_t *)(qs + (int64_t)t * n + e) = packed;
         if (lane == 0) dx[(int64_t)b * ldx + t] = amax * (1.0f / 127.0f);
+        sum = quad_sum_i32(sum);
+        if ((lane & 3) == 0) hs[((int64_t)b * ldx + t) * 16 + (lane >> 2)] = (_Float16)(float)sum;
     }
 }
 
@@ -71,11 +79,11 @@ __global__ __launch_bounds__(256) void rmsnorm_q8k_batch_kernel(const float *x, 
 // with the reference's vector exp, then Q8_K for the down projection.
 // grid (n/256, T).
 __global__ __launch_bounds__(256) void silu_mul_q8k_batch_kernel(const float *gate, const float *up, int n,
-                                                                 int8_t *qs, float *dx, int ldx) {
+                                                                 int8_t *qs, float *dx, int ldx, _Float16 *hs) {
     __shared__ float red[4];
     const int t = blockIdx.y;
     const int64_t i = (int64_t)t * n + blockIdx.x * 256 + threadIdx.x;
-    q8k_batch_store(silu_mul_ref(gate[i], up[i]), blockIdx.x, t, n, qs, dx, ldx, red);
+    q8k_batch_store(silu_mul_ref(gate[i], up[i]), blockIdx.x, t, n, qs, dx, ldx, hs, red);
 }
 
 // Final attention scale of every token (out * (1/den) where den > 0, as
@@ -83,7 +91,7 @@ __global__ __launch_bounds__(256) void silu_mul_q8k_batch_kernel(const float *ga
 // out [T][n], token t's denominators at den + t*den_tok.  grid (n/256, T).
 __global__ __launch_bounds__(256) void attn_finish_q8k_batch_kernel(const float *out, const float *den,
                                                                     int64_t den_tok, int vd, int n, int8_t *qs,
-                                                                    float *dx, int ldx) {
+                                                                    float *dx, int ldx, _Float16 *hs) {
     __shared__ float red[4];
     const int t = blockIdx.y, e = blockIdx.x * 256 + threadIdx.x;
     float v = out[(int64_t)t * n + e];
@@ -92,7 +100,7 @@ __global__ __launch_bounds__(256) void attn_finish_q8k_batch_kernel(const float 
         const float inv = 1.0f / d;
         v = v * inv;
     }
-    q8k_batch_store(v, blockIdx.x, t, n, qs, dx, ldx, red);
+    q8k_batch_store(v, blockIdx.x, t, n, qs, dx, ldx, hs, red);
 }
 
 // Embedding rows of T tokens (token_embd.row_into, src/model.rs:267-289).

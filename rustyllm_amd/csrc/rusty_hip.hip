@@ -1177,14 +1177,18 @@ struct BatchXq {
     int8_t *qs;
     float *dx;
     int ldx;
+    _Float16 *hs;
 };
 static int64_t batch_ldx(int T) { return ((int64_t)T + 63) / 64 * 64; }
-static size_t batch_xq_bytes(int T, int K) { return (size_t)T * K + (size_t)(K / 256) * batch_ldx(T) * 4 + 256; }
+static size_t batch_xq_bytes(int T, int K) {
+    return ((size_t)T * K + 255) / 256 * 256 + (size_t)(K / 256) * batch_ldx(T) * (4 + 32);
+}
 static BatchXq batch_xq_at(int8_t *buf, int T, int K) {
     BatchXq b;
     b.qs = buf;
     b.dx = (float *)(buf + ((size_t)T * K + 255) / 256 * 256);
     b.ldx = (int)batch_ldx(T);
+    b.hs = (_Float16 *)(b.dx + (size_t)(K / 256) * b.ldx);
     return b;
 }
 
@@ -1192,67 +1196,82 @@ static int quantize_batch_enqueue(const float *x, int ldxf, int T, int K, const 
     if (K % 256 != 0 || T <= 0) return 0;
     ProfScope ps("quantize_q8k_batch", s);
     rh_launch(quantize_q8k_batch_kernel, dim3((unsigned)(K / 256), (unsigned)T), dim3(256), 0, s, x, K, ldxf, b.qs,
-              b.dx, b.ldx);
+              b.dx, b.ldx, b.hs);
     RH_LAUNCH_OK();
     return 1;
 }
 
 // y[t * ldy + r] (=, or += with epi EPI_ADD) row r of W times token t, plus
-// bias[r] when given; rows of one wave tile are 32 weight rows, a workgroup
-// holds 4 tiles and covers 64 tokens.
-static int gemm_kq_enqueue(const DevW &W, const BatchXq &b, int T, float *y, int ldy, int epi, const float *bias,
-                           hipStream_t s, const char *prof_name = nullptr) {
-    if ((W.fmt != 12 && W.fmt != 14) || W.cols % 256 != 0 || W.stride % 16 != 0 || T <= 0 || ldy < W.rows)
-        return 0;
+// bias[r] when given, for n <= 2 matrices of one K that share the batch (two
+// Q4_K ones in one launch).
+struct GemmMat {
+    const DevW *w;
+    float *y;
+    int ldy;
+    const float *bias;
+};
+template <int NT>
+static void launch_q4k_gemm(const GemmArgs &A, int row_tiles, hipStream_t s) {
+    rh_launch(gemm_q4k_mfma_kernel<NT>, dim3((unsigned)row_tiles, (unsigned)((A.T + 32 * NT - 1) / (32 * NT))),
+              dim3(256), (uint32_t)gemm_q4k_lds(NT), s, A);
+}
+static int gemm_kq_enqueue(const GemmMat *ms, int n, const BatchXq &b, int T, int epi, hipStream_t s,
+                           const char *prof_name = nullptr) {
     GemmArgs A;
     memset(&A, 0, sizeof(A));
-    A.w = W.p;
-    A.row_stride = W.stride;
-    A.rows = W.rows;
-    A.K = W.cols;
+    int tiles = 0;
+    if (n < 1 || n > 2 || T <= 0) return 0;
+    for (int i = 0; i < n; i++) {
+        const DevW &W = *ms[i].w;
+        if ((W.fmt != 12 && W.fmt != 14) || W.cols % 256 != 0 || W.stride % 16 != 0 || ms[i].ldy < W.rows) return 0;
+        if (W.cols != ms[0].w->cols) return 0;
+    }
+    A.K = ms[0].w->cols;
     A.T = T;
     A.epi = epi;
     A.xq = b.qs;
     A.dx = b.dx;
+    A.hs = b.hs;
     A.ldx = b.ldx;
-    A.ldy = ldy;
-    A.y = y;
-    A.bias = bias;
-    // 32 tokens per workgroup: a 64-token tile needs twice the registers
-    // (two waves per SIMD) and measured slower (the smaller grids lose more
-    // than the 14336-row products gain).
-    // RUSTY_HIP_GEMM_KSPLIT: 0 never, 2 always, else (default) the K-split
-    // kernel for Q6_K (whose row-tile kernel holds 256 registers, one wave
-    // per SIMD) and for Q4_K when the row-tile grid would hold fewer
-    // workgroups than CUs (the 1024-row k projection of an 8B-class model;
-    // the 4096-row ones measured faster on the row-tile kernel)
-    static int ksm = -1;
-    if (ksm < 0) {
-        const char *e = getenv("RUSTY_HIP_GEMM_KSPLIT");
-        ksm = e ? atoi(e) : 1;
+    const bool q4 = ms[0].w->fmt == 12 && (n == 1 || ms[1].w->fmt == 12);
+    if (n == 2 && !q4)
+        return gemm_kq_enqueue(ms, 1, b, T, epi, s, prof_name) && gemm_kq_enqueue(ms + 1, 1, b, T, epi, s, prof_name);
+    for (int i = 0; i < n; i++) {
+        const DevW &W = *ms[i].w;
+        tiles += (W.rows + 127) / 128;
+        A.m[i] = {W.p, W.stride, ms[i].y, ms[i].bias, W.rows, ms[i].ldy, tiles};
     }
-    const int64_t row_tiles = (W.rows + 127) / 128;
-    const int tok = 32;
-    const int64_t tok_tiles = (T + tok - 1) / tok;
-    const bool ks = ksm == 2 || (ksm == 1 && (W.fmt == 14 || row_tiles * tok_tiles < (int64_t)g.n_cu));
-    ProfScope ps(prof_name ? prof_name : (W.fmt == 12 ? "gemm_q4k_mfma" : "gemm_q6k_mfma"), s);
-    if (ks) {
-        const dim3 grid((unsigned)((W.rows + 31) / 32), (unsigned)tok_tiles);
-        if (W.fmt == 12)
-            rh_launch(gemm_kq_mfma_ks_kernel<F_Q4_K>, grid, dim3(256), 0, s, A);
-        else
-            rh_launch(gemm_kq_mfma_ks_kernel<F_Q6_K>, grid, dim3(256), 0, s, A);
-        RH_LAUNCH_OK();
-        return 1;
-    }
-    const dim3 grid((unsigned)row_tiles, (unsigned)tok_tiles);
-    const uint32_t lds = 2u * tok * GEMM_XS;
-    if (W.fmt == 12)
-        rh_launch(gemm_kq_mfma_kernel<F_Q4_K, 1>, grid, dim3(256), lds, s, A);
+    if (n == 1) A.m[1] = A.m[0];
+    ProfScope ps(prof_name ? prof_name : (q4 ? "gemm_q4k_mfma" : "gemm_q6k_mfma"), s);
+    // Q4_K: 64 tokens per workgroup where two such workgroups per CU remain (the
+    // row decode is shared by two token tiles), 32 where three quarters of the CUs
+    // get one, else K split over a workgroup's waves.  Measured, us: 28672 x 4096,
+    // 512 tokens: 173 with 64 tokens, 211 with 32; 4096 x 4096, 512 tokens (256 or
+    // 512 workgroups): 34 either way; 14336 x 4096, 37 tokens (112 or 224): 29 and
+    // 21.6, K split 27; 1024 x 4096, 512 tokens (128 with 32 tokens): K split 15.1,
+    // 20.5 with 32; 4096 x 4096, 64 tokens: 10.4 and 19.6.
+    const int64_t wg1 = (int64_t)tiles * ((T + 31) / 32), wg2 = (int64_t)tiles * ((T + 63) / 64);
+    if (q4 && wg2 >= 2 * g.n_cu)
+        launch_q4k_gemm<2>(A, tiles, s);
+    else if (q4 && 4 * wg1 >= 3 * g.n_cu)
+        launch_q4k_gemm<1>(A, tiles, s);
     else
-        rh_launch(gemm_kq_mfma_kernel<F_Q6_K, 1>, grid, dim3(256), lds, s, A);
+        for (int i = 0; i < n; i++) {
+            GemmArgs B = A;
+            B.m[0] = A.m[i];
+            const dim3 grid((unsigned)((B.m[0].rows + 31) / 32), (unsigned)((T + 31) / 32));
+            if (q4)
+                rh_launch(gemm_kq_mfma_ks_kernel<F_Q4_K>, grid, dim3(256), 0, s, B);
+            else
+                rh_launch(gemm_kq_mfma_ks_kernel<F_Q6_K>, grid, dim3(256), 0, s, B);
+        }
     RH_LAUNCH_OK();
     return 1;
+}
+static int gemm_kq_enqueue(const DevW &W, const BatchXq &b, int T, float *y, int ldy, int epi, const float *bias,
+                           hipStream_t s, const char *prof_name = nullptr) {
+    const GemmMat m = {&W, y, ldy, bias};
+    return gemm_kq_enqueue(&m, 1, b, T, epi, s, prof_name);
 }
 
 // ---- per-op exports ------------------------------------------------------------------
@@ -2677,7 +2696,7 @@ static int r_prefill_alloc() {
 static int r_rmsnorm_batch(const float *norm_w, int T, const BatchXq &b, hipStream_t s) {
     ProfScope ps("rmsnorm_q8k_batch", s);
     rh_launch(rmsnorm_q8k_batch_kernel, dim3((unsigned)T), dim3(256), R.dim * 4, s, (const float *)R.px,
-              norm_w, R.eps, (int)R.dim, b.qs, b.dx, b.ldx);
+              norm_w, R.eps, (int)R.dim, b.qs, b.dx, b.ldx, b.hs);
     RH_LAUNCH_OK();
     return 1;
 }
@@ -2699,8 +2718,8 @@ static int r_prefill_chunk(const int32_t *tok, int T, int pos0, hipStream_t s) {
     for (uint32_t l = 0; l < R.n_layers; l++) {
         RLayer &Ly = R.L[l];
         if (!r_rmsnorm_batch(Ly.attn_norm, T, bd, s)) return 0;
-        if (!gemm_kq_enqueue(Ly.w[0], bd, T, R.pq, qd, EPI_STORE, Ly.bias[0], s, "pf_gemm_q") ||
-            !gemm_kq_enqueue(Ly.w[1], bd, T, R.pk, kd, EPI_STORE, Ly.bias[1], s, "pf_gemm_k") ||
+        const GemmMat qk[2] = {{&Ly.w[0], R.pq, qd, Ly.bias[0]}, {&Ly.w[1], R.pk, kd, Ly.bias[1]}};
+        if (!gemm_kq_enqueue(qk, 2, bd, T, EPI_STORE, s, "pf_gemm_qk") ||
             !gemm_kq_enqueue(Ly.w[2], bd, T, R.pv, vdim, EPI_STORE, Ly.bias[2], s, "pf_gemm_v"))
             return 0;
         {
@@ -2765,18 +2784,17 @@ static int r_prefill_chunk(const int32_t *tok, int T, int pos0, hipStream_t s) {
             ProfScope ps("attn_finish_batch", s);
             rh_launch(attn_finish_q8k_batch_kernel, dim3(attn_cols / 256, (unsigned)T), dim3(256), 0, s,
                       (const float *)R.pattn, den, (int64_t)exact_scratch_floats(R.n_kv, kvm, cap), (int)R.vd,
-                      attn_cols, ba.qs, ba.dx, ba.ldx);
+                      attn_cols, ba.qs, ba.dx, ba.ldx, ba.hs);
             RH_LAUNCH_OK();
         }
         if (!gemm_kq_enqueue(Ly.w[3], ba, T, R.px, dim, EPI_ADD, nullptr, s, "pf_gemm_o")) return 0;
         if (!r_rmsnorm_batch(Ly.ffn_norm, T, bd, s)) return 0;
-        if (!gemm_kq_enqueue(Ly.w[4], bd, T, R.ptg, hid, EPI_STORE, nullptr, s, "pf_gemm_gate_up") ||
-            !gemm_kq_enqueue(Ly.w[5], bd, T, R.ptu, hid, EPI_STORE, nullptr, s, "pf_gemm_gate_up"))
-            return 0;
+        const GemmMat gu[2] = {{&Ly.w[4], R.ptg, hid, nullptr}, {&Ly.w[5], R.ptu, hid, nullptr}};
+        if (!gemm_kq_enqueue(gu, 2, bd, T, EPI_STORE, s, "pf_gemm_gate_up")) return 0;
         {
             ProfScope ps("silu_mul_batch", s);
             rh_launch(silu_mul_q8k_batch_kernel, dim3(hid / 256, (unsigned)T), dim3(256), 0, s, (const float *)R.ptg,
-                      (const float *)R.ptu, hid, bh.qs, bh.dx, bh.ldx);
+                      (const float *)R.ptu, hid, bh.qs, bh.dx, bh.ldx, bh.hs);
             RH_LAUNCH_OK();
         }
         if (!gemm_kq_enqueue(Ly.w[6], bh, T, R.px, dim, EPI_ADD, nullptr, s,
@@ -3059,7 +3077,7 @@ static int r_prefill_chunk_moe(const int32_t *tok, int T, int pos0, hipStream_t 
             ProfScope ps("attn_finish_batch", s);
             rh_launch(attn_finish_q8k_batch_kernel, dim3(attn_cols / 256, (unsigned)T), dim3(256), 0, s,
                       (const float *)R.pattn, den, (int64_t)exact_scratch_floats(R.n_kv, kvm, cap), (int)R.vd,
-                      attn_cols, ba.qs, ba.dx, ba.ldx);
+                      attn_cols, ba.qs, ba.dx, ba.ldx, ba.hs);
             RH_LAUNCH_OK();
         }
         if (!kv_ring_copy(Ly, last0, pos0 + T - last0, last0 - P0, 1, s)) return 0;
