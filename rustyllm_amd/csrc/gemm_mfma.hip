@@ -110,51 +110,9 @@ __device__ __forceinline__ rh_v4i bytes_times(const rh_v4i &x, int s) {
     return r;
 }
 
-// Integer sums of a block for the wave's 32 rows x 32*NT tokens: isum per C
-// element, from the activation tile xs.
-template <int NT>
-__device__ __forceinline__ void gemm_block_ints(const GemmW<F_Q6_K> &W, const int8_t *xs, int lane,
-                                                int (&isum)[NT][16]) {
-    const int half = lane >> 5, n = lane & 31;
-#pragma unroll
-    for (int tt = 0; tt < NT; tt++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) isum[tt][i] = 0;
-    const uint32_t scw[4] = {W.sc.x, W.sc.y, W.sc.z, W.sc.w};
-#pragma unroll
-    for (int g = 0; g < 2; g++)
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint2 qh = W.qh[2 * g + h];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint2 ql = W.ql[4 * g + 2 * h + (k & 1)];
-                const int sh = 4 * (k >> 1);
-                const uint32_t q0 = ((ql.x >> sh) & 0x0F0F0F0Fu) | (((qh.x >> (2 * k)) & 0x03030303u) << 4);
-                const uint32_t q1 = ((ql.y >> sh) & 0x0F0F0F0Fu) | (((qh.y >> (2 * k)) & 0x03030303u) << 4);
-                const long bq = (long)((uint64_t)q6_signed4(q0) | ((uint64_t)q6_signed4(q1) << 32));
-                const int si = 8 * g + 2 * k + h;  // scale of 16-element group (g, k, h)
-                const int sc = (int)(int8_t)(scw[si >> 2] >> (8 * (si & 3)));
-                const int e0 = 128 * g + 32 * k + 16 * h + 8 * half;
-#pragma unroll
-                for (int tt = 0; tt < NT; tt++) {
-                    const long a = *(const long *)(xs + (32 * tt + n) * GEMM_XS + e0);
-                    const rh_v16i c = __builtin_amdgcn_mfma_i32_32x32x16_i8(a, bq, rh_v16i{}, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 16; i++) {
-                        isum[tt][i] = __mul24(sc, c[i]) + isum[tt][i];
-                        // opaque to the optimiser: keeps one 24-bit multiply-add per
-                        // update instead of products paired into three-input adds
-                        asm("" : "+v"(isum[tt][i]));
-                    }
-                }
-            }
-        }
-}
-
-// Q4_K products: a workgroup is 128 weight rows (a wave 32) by 32 NT tokens.
+// Batch products: a workgroup is 128 weight rows (a wave 32) by 32 NT tokens.
 //
-// The sub-block scale (6 bits) enters the B operand as two digits, sc = 8 (sc
+// Q4_K: the sub-block scale (6 bits) enters the B operand as two digits, sc = 8 (sc
 // >> 3) + (sc & 7), each digit times a nibble fitting a signed byte, so the
 // MFMAs accumulate the whole block: isum = 8 hi + lo = sum_j sc_j C_j exactly.
 // The minimums' sum imin = sum_j m_j (sum of sub-block j) is one 32x32x16 f16
@@ -172,11 +130,13 @@ __device__ __forceinline__ void gemm_block_ints(const GemmW<F_Q6_K> &W, const in
 // stored after, the 28672 x 4096 product took 176 us instead of 160), and its
 // weights straight after the digits are made.  One barrier per block.
 //
-// Bound by the VALU: 200 instructions per 32 x 32 outputs and block with NT =
-// 2 (390 with a minimum MFMA per sub-block and one token tile), about 60% busy;
+// Bound by the VALU, Q4_K: 200 instructions per 32 x 32 outputs and block with
+// NT = 2 (390 with a minimum MFMA per sub-block and one token tile), about 60% busy;
 // the waits are the barrier and the start of each tile.  Gate and up of an
 // 8B-class model, 28672 x 4096, 512 tokens in one launch: 161 us (747 TOP/s);
-// two launches of the one-tile kernel before, 244.  Measured and dropped: four
+// two launches of the one-tile kernel before, 244.  Q6_K: about 430
+// instructions per tile (256 of them the groups' scale multiply-adds), 587
+// with one token tile: 4096 x 14336, 512 tokens 242 us, K split 301.  Measured and dropped: four
 // token tiles (spills at two waves per SIMD: 189 us); each row tile's token
 // tiles on one XCD (160).
 typedef _Float16 rh_v8h __attribute__((ext_vector_type(8)));
@@ -251,13 +211,80 @@ __device__ __forceinline__ void q4k_tile(const Q4kOps &O, const int8_t *xr, rh_v
     }
 }
 
-constexpr int gemm_q4k_buf(int nt) { return 32 * nt * (GEMM_XS + 32 + 4); }
-constexpr int gemm_q4k_lds(int nt) { return 2 * gemm_q4k_buf(nt); }
+// One block of the lane's Q6_K row as MFMA B operands: the sixteen 16-element
+// groups' q - 32 (8 bytes of the lane half), their scales, d.
+struct Q6kOps {
+    uint2 b[16];
+    uint32_t sc[4];
+    float d;
+};
+__device__ __forceinline__ void q6k_decode(Q6kOps &O, const GemmW<F_Q6_K> &W) {
+    O.d = h2f((uint16_t)W.d);
+    O.sc[0] = W.sc.x;
+    O.sc[1] = W.sc.y;
+    O.sc[2] = W.sc.z;
+    O.sc[3] = W.sc.w;
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint2 qh = W.qh[2 * g + h];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint2 ql = W.ql[4 * g + 2 * h + (k & 1)];
+                const int sh = 4 * (k >> 1);
+                const uint32_t q0 = ((ql.x >> sh) & 0x0F0F0F0Fu) | (((qh.x >> (2 * k)) & 0x03030303u) << 4);
+                const uint32_t q1 = ((ql.y >> sh) & 0x0F0F0F0Fu) | (((qh.y >> (2 * k)) & 0x03030303u) << 4);
+                O.b[8 * g + 2 * k + h] = make_uint2(q6_signed4(q0), q6_signed4(q1));
+            }
+        }
+}
 
-template <int NT>
-__global__ __launch_bounds__(256, 2) void gemm_q4k_mfma_kernel(GemmArgs A) {
+// The block's values (dx d) isum of 32 rows x 32 tokens: xr the lane's token
+// row of the LDS tile (+ 8 half); dv and out as q4k_tile's.
+template <class Dv, class Out>
+__device__ __forceinline__ void q6k_tile(const Q6kOps &O, const int8_t *xr, Dv dv, Out out) {
+    int isum[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) isum[i] = 0;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const long a = *(const long *)(xr + 16 * e);
+        const long bq = (long)((uint64_t)O.b[e].x | ((uint64_t)O.b[e].y << 32));
+        const int sc = (int)(int8_t)(O.sc[e >> 2] >> (8 * (e & 3)));
+        const rh_v16i c = __builtin_amdgcn_mfma_i32_32x32x16_i8(a, bq, rh_v16i{}, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            isum[i] = __mul24(sc, c[i]) + isum[i];
+            // opaque to the optimiser: keeps one 24-bit multiply-add per update
+            // instead of products paired into three-input adds
+            asm("" : "+v"(isum[i]));
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const rh_v4f dx = dv(g);
+#pragma unroll
+        for (int r = 0; r < 4; r++) out(4 * g + r, (dx[r] * O.d) * (float)isum[4 * g + r]);
+    }
+}
+
+template <int FMT>
+struct GemmOps {
+    typedef Q6kOps type;
+};
+template <>
+struct GemmOps<F_Q4_K> {
+    typedef Q4kOps type;
+};
+
+constexpr int gemm_kq_buf(int nt) { return 32 * nt * (GEMM_XS + 32 + 4); }
+constexpr int gemm_kq_lds(int nt) { return 2 * gemm_kq_buf(nt); }
+
+template <int FMT, int NT>
+__global__ __launch_bounds__(256, 2) void gemm_kq_mfma_kernel(GemmArgs A) {
     extern __shared__ __align__(16) int8_t s_xt[];  // [2]: quants [TOK][GEMM_XS], sums [TOK][16] f16, scales [TOK]
-    constexpr int TOK = 32 * NT, HS0 = TOK * GEMM_XS, DX0 = HS0 + TOK * 32, BUF = gemm_q4k_buf(NT);
+    constexpr int TOK = 32 * NT, HS0 = TOK * GEMM_XS, DX0 = HS0 + TOK * 32, BUF = gemm_kq_buf(NT);
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int bx = blockIdx.x, by = blockIdx.y;
@@ -278,16 +305,17 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k_mfma_kernel(GemmArgs A) {
         return __builtin_amdgcn_raw_buffer_load_b128(xres, xoff, 16 * j * A.K + 256 * b, 0);
     };
     typedef decltype(__builtin_amdgcn_raw_buffer_load_b128(xres, 0, 0, 0)) piece_t;
-    GemmW<F_Q4_K> W;
-    auto load_w = [&](int b) { gemm_w_load(W, wr + (int64_t)b * 144, half); };
+    constexpr int BB = FMT == F_Q4_K ? 144 : 210;
+    GemmW<FMT> W;
+    auto load_w = [&](int b) { gemm_w_load(W, wr + (int64_t)b * BB, half); };
     rh_v4i hsr;
     float dxr = 0.0f;
     auto load_hd = [&](int b) {
-        if (tid < 2 * TOK) hsr = *(const rh_v4i *)(A.hs + ((int64_t)b * A.ldx + ht) * 16 + 8 * (tid & 1));
+        if (FMT == F_Q4_K && tid < 2 * TOK) hsr = *(const rh_v4i *)(A.hs + ((int64_t)b * A.ldx + ht) * 16 + 8 * (tid & 1));
         if (tid < TOK) dxr = A.dx[(int64_t)b * A.ldx + dt];
     };
     auto store_hd = [&](int8_t *buf) {
-        if (tid < 2 * TOK) *(rh_v4i *)(buf + HS0 + 16 * tid) = hsr;
+        if (FMT == F_Q4_K && tid < 2 * TOK) *(rh_v4i *)(buf + HS0 + 16 * tid) = hsr;
         if (tid < TOK) *(float *)(buf + DX0 + 4 * tid) = dxr;
     };
     piece_t st[2 * NT];
@@ -311,8 +339,11 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k_mfma_kernel(GemmArgs A) {
         const int8_t *cur = s_xt + (b & 1) * BUF;
         int8_t *nxt = s_xt + ((b + 1) & 1) * BUF;
         const int bn = min(b + 1, nb - 1);  // (the last block stages itself again, unread)
-        Q4kOps O;
-        q4k_decode(O, W, half);
+        typename GemmOps<FMT>::type O;
+        if constexpr (FMT == F_Q4_K)
+            q4k_decode(O, W, half);
+        else
+            q6k_decode(O, W);
         load_w(bn);
         // the next block's activations, loaded a block ago, then the one after
         store_hd(nxt);
@@ -325,11 +356,13 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k_mfma_kernel(GemmArgs A) {
 #pragma unroll
         for (int tt = 0; tt < NT; tt++) {
             // the reference's per-block combine, accumulated in block order
-            q4k_tile(
-                O, cur + (32 * tt + n) * GEMM_XS + 16 * half,
-                *(const rh_v8h *)(cur + HS0 + (32 * tt + n) * 32 + 16 * half),
-                [&](int g) { return *(const rh_v4f *)(cur + DX0 + 4 * (32 * tt + 8 * g + 4 * half)); },
-                [&](int i, float v) { acc[tt][i] += v; });
+            const int8_t *xr = cur + (32 * tt + n) * GEMM_XS;
+            const auto dv = [&](int g) { return *(const rh_v4f *)(cur + DX0 + 4 * (32 * tt + 8 * g + 4 * half)); };
+            const auto out = [&](int i, float v) { acc[tt][i] += v; };
+            if constexpr (FMT == F_Q4_K)
+                q4k_tile(O, xr + 16 * half, *(const rh_v8h *)(cur + HS0 + (32 * tt + n) * 32 + 16 * half), dv, out);
+            else
+                q6k_tile(O, xr + 8 * half, dv, out);
         }
         __syncthreads();
     }
@@ -419,11 +452,10 @@ __global__ __launch_bounds__(256) void gemm_kq_mfma_ks_kernel(GemmArgs A) {
                 q4k_tile(O, xs + n * GEMM_XS + 16 * half, hs, [&](int g) { return dv[g]; },
                          [&](int i, float val) { v[i] = val; });
             } else {
-                int isum[1][16];
-                gemm_block_ints<1>(W, xs, lane, isum);
-                const float d = h2f(W.d & 0xFFFF);
-#pragma unroll
-                for (int i = 0; i < 16; i++) v[i] = (dv[i >> 2][i & 3] * d) * (float)isum[0][i];
+                Q6kOps O;
+                q6k_decode(O, W);
+                q6k_tile(O, xs + n * GEMM_XS + 8 * half, [&](int g) { return dv[g]; },
+                         [&](int i, float val) { v[i] = val; });
             }
         }
         // the next block's activations, in flight over the barrier (issued

@@ -1210,10 +1210,10 @@ struct GemmMat {
     int ldy;
     const float *bias;
 };
-template <int NT>
-static void launch_q4k_gemm(const GemmArgs &A, int row_tiles, hipStream_t s) {
-    rh_launch(gemm_q4k_mfma_kernel<NT>, dim3((unsigned)row_tiles, (unsigned)((A.T + 32 * NT - 1) / (32 * NT))),
-              dim3(256), (uint32_t)gemm_q4k_lds(NT), s, A);
+template <int FMT, int NT>
+static void launch_kq_gemm(const GemmArgs &A, int row_tiles, hipStream_t s) {
+    rh_launch((gemm_kq_mfma_kernel<FMT, NT>), dim3((unsigned)row_tiles, (unsigned)((A.T + 32 * NT - 1) / (32 * NT))),
+              dim3(256), (uint32_t)gemm_kq_lds(NT), s, A);
 }
 static int gemm_kq_enqueue(const GemmMat *ms, int n, const BatchXq &b, int T, int epi, hipStream_t s,
                            const char *prof_name = nullptr) {
@@ -1250,11 +1250,16 @@ static int gemm_kq_enqueue(const GemmMat *ms, int n, const BatchXq &b, int T, in
     // 512 workgroups): 34 either way; 14336 x 4096, 37 tokens (112 or 224): 29 and
     // 21.6, K split 27; 1024 x 4096, 512 tokens (128 with 32 tokens): K split 15.1,
     // 20.5 with 32; 4096 x 4096, 64 tokens: 10.4 and 19.6.
+    // Q6_K: 64 tokens per workgroup where every CU gets one, else K split:
+    // 4096 x 14336, 512 tokens (256 workgroups) 242 and 301; 14336 x 4096, 512
+    // tokens 213 and 333; 4096 x 14336, 100 tokens (64) 224 and 91.
     const int64_t wg1 = (int64_t)tiles * ((T + 31) / 32), wg2 = (int64_t)tiles * ((T + 63) / 64);
     if (q4 && wg2 >= 2 * g.n_cu)
-        launch_q4k_gemm<2>(A, tiles, s);
+        launch_kq_gemm<F_Q4_K, 2>(A, tiles, s);
+    else if (!q4 && wg2 >= g.n_cu)
+        launch_kq_gemm<F_Q6_K, 2>(A, tiles, s);
     else if (q4 && 4 * wg1 >= 3 * g.n_cu)
-        launch_q4k_gemm<1>(A, tiles, s);
+        launch_kq_gemm<F_Q4_K, 1>(A, tiles, s);
     else
         for (int i = 0; i < n; i++) {
             GemmArgs B = A;
