@@ -124,6 +124,9 @@ struct Ctx {
     Profile prof;
     float *noalloc[16] = {};  // device address of `scratch`, per device (set up by init)
     uint8_t *stage[2] = {nullptr, nullptr};  // pinned staging of weight uploads
+    // pinned activations in / outputs out of the per-op exports (one call at a
+    // time holds the mutex; RH_IO_FLOATS each)
+    float *io_in = nullptr, *io_out = nullptr;
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
 };
 static Ctx g;
@@ -199,19 +202,25 @@ static int ensure_xq(XQ *xq, size_t *cap, size_t n) {
     return 1;
 }
 
-// FNV-1a over 256 16-byte samples spread across the buffer (plus both
-// ends): cheap next to an upload, and it catches a host address that was
-// freed and reused for different bytes.
+// FNV-1a over the eight-byte words of 256 16-byte samples spread across the
+// buffer (plus both ends): cheap next to an upload, and it catches a host
+// address that was freed and reused for different bytes.  Two hashes, one per
+// word of a sample, keep their multiplies independent: 0.7 us per weight where
+// a byte at a time took 5, of every per-op call and weight.
 static uint64_t fingerprint(const uint8_t *p, size_t len) {
-    uint64_t h = 1469598103934665603ull ^ len;
+    uint64_t h = 1469598103934665603ull ^ len, h2 = h * 1099511628211ull;
     auto mix = [&](size_t off) {
-        size_t n = std::min<size_t>(16, len - off);
-        for (size_t i = 0; i < n; i++) h = (h ^ p[off + i]) * 1099511628211ull;
+        uint64_t w[2] = {0, 0};
+        memcpy(w, p + off, std::min<size_t>(16, len - off));
+        h = (h ^ w[0]) * 1099511628211ull;
+        h2 = (h2 ^ w[1]) * 1099511628211ull;
+        h ^= h >> 29;  // (the multiply alone never moves a word's high bits down)
+        h2 ^= h2 >> 29;
     };
     if (len == 0) return h;
     for (int k = 0; k < 256; k++) mix((size_t)((unsigned __int128)len * k / 256));
     mix(len > 16 ? len - 16 : 0);
-    return h;
+    return h ^ (h2 * 0x9E3779B97F4A7C15ull);
 }
 
 static bool weight_shape_ok(const uint8_t *host, size_t len, int64_t rows, int64_t cols, int fmt) {
@@ -1280,9 +1289,88 @@ static int gemm_kq_enqueue(const DevW &W, const BatchXq &b, int T, float *y, int
 }
 
 // ---- per-op exports ------------------------------------------------------------------
-static int stage_x(const float *x, size_t n) {
+// Activations and outputs of at most RH_IO_FLOATS floats cross through pinned
+// memory that the kernels address themselves: the quantizer reads x there (or
+// one launch copies it to the device), and the last launch of a call writes the
+// outputs there.  The runtime's copies of pageable memory took 13 of the 38 us
+// of a 256 x 2048 matvec call, and 9 of the 134 of a 128256-row product.  A counter that the last launch writes for the host to
+// watch, in place of the stream synchronisation, measured the same in a row of
+// calls and 7 us slower alone.
+#define RH_IO_FLOATS ((size_t)1 << 20)
+static bool io_ready() {
+    if (!g.io_in && hipHostMalloc((void **)&g.io_in, RH_IO_FLOATS * 4, hipHostMallocDefault) != hipSuccess) {
+        g.io_in = nullptr;
+        return false;
+    }
+    if (!g.io_out && hipHostMalloc((void **)&g.io_out, RH_IO_FLOATS * 4, hipHostMallocDefault) != hipSuccess) {
+        g.io_out = nullptr;
+        return false;
+    }
+    return true;
+}
+
+__global__ __launch_bounds__(256) void stage_in_kernel(const float *src, int n, float *dst) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+// Up to three device arrays, one after the other, to the pinned output.
+struct StageOut {
+    const float *src[3];
+    int n[3];
+};
+__global__ __launch_bounds__(256) void stage_out_kernel(StageOut S, float *dst) {
+    int i = blockIdx.x * 256 + threadIdx.x;
+    float *d = dst + i;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        if (i >= 0 && i < S.n[k]) *d = S.src[k][i];
+        i -= S.n[k];
+    }
+}
+
+// Enqueues the copy of the outputs, waits for it and hands them to the caller:
+// out[k] gets S.n[k] floats (or is null).
+static int finish_out(const StageOut &S, void *const *out) {
+    const size_t total = (size_t)S.n[0] + S.n[1] + S.n[2];
+    const bool pinned = total <= RH_IO_FLOATS && io_ready();
+    if (pinned) {
+        rh_launch(stage_out_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, g.s, S, g.io_out);
+        RH_LAUNCH_OK();
+    } else {
+        for (int k = 0; k < 3; k++)
+            if (S.n[k] && out[k])
+                RH_CHECK(hipMemcpyAsync(out[k], S.src[k], (size_t)S.n[k] * 4, hipMemcpyDeviceToHost, g.s));
+    }
+    RH_CHECK(hipStreamSynchronize(g.s));
+    if (pinned) {
+        const float *p = g.io_out;
+        for (int k = 0; k < 3; k++) {
+            if (S.n[k] && out[k]) memcpy(out[k], p, (size_t)S.n[k] * 4);
+            p += S.n[k];
+        }
+    }
+    prof_drain();
+    return 1;
+}
+
+// n host floats for kernels to read: in g.x, and where they fit, in *pinned for
+// a first launch that wants them without the copy (want_dev false: only there).
+static int stage_x(const float *x, size_t n, bool want_dev = true, const float **first = nullptr) {
     if (!ensure(&g.x, &g.x_cap, n)) return 0;
-    RH_CHECK(hipMemcpyAsync(g.x, x, n * sizeof(float), hipMemcpyHostToDevice, g.s));
+    if (first) *first = g.x;
+    if (n > RH_IO_FLOATS || !io_ready()) {
+        RH_CHECK(hipMemcpyAsync(g.x, x, n * sizeof(float), hipMemcpyHostToDevice, g.s));
+        return 1;
+    }
+    memcpy(g.io_in, x, n * 4);
+    if (first) *first = g.io_in;
+    if (want_dev) {
+        rh_launch(stage_in_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, g.s, (const float *)g.io_in, (int)n,
+                  g.x);
+        RH_LAUNCH_OK();
+        if (first) *first = g.x;
+    }
     return 1;
 }
 
@@ -1299,7 +1387,10 @@ static int matvec_n(int n, const int *fmts, const uint8_t *const *w, const uintp
         if (!get_weight(w[i], wl[i], (int64_t)rows[i], (int64_t)cols, fmts[i], &ms[i].w)) return 0;
         total += rows[i];
     }
-    if (!stage_x(x, cols)) return 0;
+    bool need_q = false, need_f = false;
+    for (int i = 0; i < n; i++) (cat_of(fmts[i], (int)cols) != CAT_F32 ? need_q : need_f) = true;
+    const float *xq_src;
+    if (!stage_x(x, cols, need_f, &xq_src)) return 0;
     if (!ensure(&g.y, &g.y_cap, total)) return 0;
     size_t off = 0;
     for (int i = 0; i < n; i++) {
@@ -1307,22 +1398,20 @@ static int matvec_n(int n, const int *fmts, const uint8_t *const *w, const uintp
         ms[i].bias = nullptr;
         off += rows[i];
     }
-    bool need_q = false;
-    for (int i = 0; i < n; i++)
-        if (cat_of(fmts[i], (int)cols) != CAT_F32) need_q = true;
     if (need_q) {
         if (!ensure_xq(&g.xq, &g.xq_cap, cols)) return 0;
-        if (!launch_quant(g.x, (int)cols, g.xq, g.s)) return 0;
+        if (!launch_quant(xq_src, (int)cols, g.xq, g.s)) return 0;
     }
     if (!gemv_multi(ms, n, (int)cols, EPI_STORE, g.xq, g.x, g.s)) return 0;
-    off = 0;
+    StageOut S;
+    memset(&S, 0, sizeof(S));
+    void *to[3] = {};
     for (int i = 0; i < n; i++) {
-        RH_CHECK(hipMemcpyAsync(outs[i], g.y + off, rows[i] * sizeof(float), hipMemcpyDeviceToHost, g.s));
-        off += rows[i];
+        S.src[i] = ms[i].y;
+        S.n[i] = (int)rows[i];
+        to[i] = outs[i];
     }
-    RH_CHECK(hipStreamSynchronize(g.s));
-    prof_drain();
-    return 1;
+    return finish_out(S, to);
 }
 
 static int ffn_device(const DevW &gate, const DevW &up, const DevW &down, int in_cols, const XQ &xq_in,
@@ -1619,13 +1708,14 @@ int rusty_hip_q4k_q4k_q6k_ffn(const uint8_t *gw, uintptr_t gl, const uint8_t *uw
     if (!get_weight(gw, gl, hidden_rows, in_cols, 12, &G) || !get_weight(uw, ul, hidden_rows, in_cols, 12, &U) ||
         !get_weight(dw, dl, down_rows, down_cols, 14, &D))
         return 0;
-    if (!stage_x(x, in_cols) || !ensure(&g.y, &g.y_cap, down_rows)) return 0;
-    if (!ensure_xq(&g.xq, &g.xq_cap, in_cols) || !launch_quant(g.x, (int)in_cols, g.xq, g.s)) return 0;
+    // (both widths are multiples of 256, so only the quantizer reads x)
+    const float *xs;
+    if (!stage_x(x, in_cols, false, &xs) || !ensure(&g.y, &g.y_cap, down_rows)) return 0;
+    if (!ensure_xq(&g.xq, &g.xq_cap, in_cols) || !launch_quant(xs, (int)in_cols, g.xq, g.s)) return 0;
     if (!ffn_device(G, U, D, (int)in_cols, g.xq, g.x, g.y, EPI_STORE)) return 0;
-    RH_CHECK(hipMemcpyAsync(out, g.y, down_rows * sizeof(float), hipMemcpyDeviceToHost, g.s));
-    RH_CHECK(hipStreamSynchronize(g.s));
-    prof_drain();
-    return 1;
+    const StageOut S = {{g.y}, {(int)down_rows}};
+    void *to[3] = {out};
+    return finish_out(S, to);
 }
 
 int rusty_hip_mistral_post_attention_ffn(const uint8_t *ow, uintptr_t ol, const uint8_t *gw, uintptr_t gl,
@@ -1654,10 +1744,9 @@ int rusty_hip_mistral_post_attention_ffn(const uint8_t *ow, uintptr_t ol, const 
     if (!gemv_multi(&mo, 1, (int)attn_cols, EPI_ADD, g.xq, da, g.s)) return 0;
     if (!launch_rmsnorm(dx, dw_, eps, (int)dim, dxn, &g.xq, g.s)) return 0;
     if (!ffn_device(G, U, D, (int)dim, g.xq, dxn, dx, EPI_ADD)) return 0;
-    RH_CHECK(hipMemcpyAsync(x, dx, dim * 4, hipMemcpyDeviceToHost, g.s));
-    RH_CHECK(hipStreamSynchronize(g.s));
-    prof_drain();
-    return 1;
+    const StageOut S = {{dx}, {(int)dim}};
+    void *to[3] = {x};
+    return finish_out(S, to);
 }
 
 }  // extern "C"
@@ -1902,19 +1991,16 @@ int rusty_hip_moe_ffn(const float *x, uintptr_t dim, const uint8_t *router_w, ui
         M.db = (const float *)db.p;
         M.db_stride = (int)(db.stride / 4);
     }
-    if (!ensure(&g.x, &g.x_cap, dim) || !ensure(&g.y, &g.y_cap, dim) ||
+    if (!ensure(&g.y, &g.y_cap, dim) ||
         !ensure(&g.moe, &g.moe_cap, moe_scratch_floats(M.n_exp, M.k, M.dim, M.hidden) + 8))
         return 0;
-    RH_CHECK(hipMemcpyAsync(g.x, x, dim * 4, hipMemcpyHostToDevice, g.s));
+    if (!stage_x(x, dim)) return 0;
     int32_t *sel = nullptr;
     float *prob = nullptr;
     if (!moe_ffn_enqueue(M, g.x, XQ{}, g.y, nullptr, g.moe, g.s, &sel, &prob)) return 0;
-    RH_CHECK(hipMemcpyAsync(out, g.y, dim * 4, hipMemcpyDeviceToHost, g.s));
-    if (selected) RH_CHECK(hipMemcpyAsync(selected, sel, top_k * 4, hipMemcpyDeviceToHost, g.s));
-    if (probs) RH_CHECK(hipMemcpyAsync(probs, prob, top_k * 4, hipMemcpyDeviceToHost, g.s));
-    RH_CHECK(hipStreamSynchronize(g.s));
-    prof_drain();
-    return 1;
+    const StageOut S = {{g.y, (const float *)sel, prob}, {(int)dim, (int)top_k, (int)top_k}};
+    void *to[3] = {out, selected, probs};
+    return finish_out(S, to);
 }
 
 __global__ void expf_kernel(const float *x, int n, float *out) {
@@ -3723,13 +3809,24 @@ int rusty_hip_kquant_matvec_batch(uint32_t kind, const uint8_t *w, uintptr_t w_l
     if (T > (1u << 20) || out_len < T * rows * 4) return 0;
     DevW W;
     if (!get_weight(w, w_len, (int64_t)rows, (int64_t)cols, fmt, &W)) return 0;
-    if (!ensure(&g.bx, &g.bx_cap, T * cols) || !ensure(&g.by, &g.by_cap, T * rows) ||
-        !ensure(&g.bq, &g.bq_cap, batch_xq_bytes((int)T, (int)cols)))
-        return 0;
+    if (!ensure(&g.by, &g.by_cap, T * rows) || !ensure(&g.bq, &g.bq_cap, batch_xq_bytes((int)T, (int)cols))) return 0;
     const BatchXq b = batch_xq_at(g.bq, (int)T, (int)cols);
-    RH_CHECK(hipMemcpyAsync(g.bx, inputs, T * cols * 4, hipMemcpyHostToDevice, g.s));
-    if (!quantize_batch_enqueue(g.bx, (int)cols, (int)T, (int)cols, b, g.s)) return 0;
+    const float *src;  // read by the quantizer alone
+    if (T * cols <= RH_IO_FLOATS && io_ready()) {
+        memcpy(g.io_in, inputs, T * cols * 4);
+        src = g.io_in;
+    } else {
+        if (!ensure(&g.bx, &g.bx_cap, T * cols)) return 0;
+        RH_CHECK(hipMemcpyAsync(g.bx, inputs, T * cols * 4, hipMemcpyHostToDevice, g.s));
+        src = g.bx;
+    }
+    if (!quantize_batch_enqueue(src, (int)cols, (int)T, (int)cols, b, g.s)) return 0;
     if (!gemm_kq_enqueue(W, b, (int)T, g.by, (int)rows, EPI_STORE, nullptr, g.s)) return 0;
+    if (T * rows <= RH_IO_FLOATS) {
+        const StageOut S = {{g.by}, {(int)(T * rows)}};
+        void *to[3] = {out};
+        return finish_out(S, to);
+    }
     RH_CHECK(hipMemcpyAsync(out, g.by, T * rows * 4, hipMemcpyDeviceToHost, g.s));
     RH_CHECK(hipStreamSynchronize(g.s));
     prof_drain();
