@@ -7,9 +7,9 @@
 // x4 kernels are bit-identical to its single-token dots, tests
 // src/simd.rs:8540-8608).
 //
-// v_mfma_i32_32x32x32_i8 / _32x32x16_i8 lane layout (checked on gfx950):
-// A[m = l%32][k = K8*(l/32) + j], B[k][n = l%32], C[i] at
-// m = 8*(i/4) + 4*(l/32) + i%4, n = l%32, with K8 = 16 (x32) or 8 (x16).
+// v_mfma_i32_32x32x32_i8 lane layout (checked on gfx950): A[m = l%32][k =
+// 16*(l/32) + j], B[k][n = l%32], C[i] at m = 8*(i/4) + 4*(l/32) + i%4,
+// n = l%32.
 // Here m = token and n = weight row: a lane owns one weight row, so its
 // scales and minimums are per-lane values, and 16 tokens.
 //   Q4_K: two x32 MFMAs per 32-element sub-block on the nibbles times the
@@ -17,8 +17,9 @@
 //         block, so isum = sum_j sc_j * C_j (C_j = sum q x) exactly; imin =
 //         sum_j m_j * bsums_j is one f16 MFMA per block on the sums of 16
 //         quants; value = dx * (d*isum - dmin*imin).
-//   Q6_K: one x16 MFMA per 16-element scale group on q - 32 as signed
-//         bytes, isum += sc_g * C_g; value = (dx*d) * isum.
+//   Q6_K: two x32 MFMAs per 32 elements on the high and low bytes of
+//         sc_g (q - 32), accumulated over the block, so isum = sum_g sc_g *
+//         C_g exactly; value = (dx*d) * isum.
 // Rows and tokens past the ends read clamped (in-bounds) data or zeros and
 // are not stored.
 #pragma once
@@ -49,15 +50,9 @@ struct GemmArgs {
     int32_t ldx;        // >= T, a multiple of 64
 };
 
-// Q6_K bytes q (0..63, four per dword) as signed q - 32: (q + 0x60) ^ 0x80
-// per byte, where q + 0x60 <= 0x9F never carries into the next byte (one add
-// and one xor per dword; a copy of bit 5 into bits 6 and 7 compiled to a
-// quarter-rate multiply by 6).
-__device__ __forceinline__ uint32_t q6_signed4(uint32_t q) { return (q + 0x60606060u) ^ 0x80808080u; }
-
 // One block of the lane's weight row, as the lane's MFMA B operands need it
-// (lane half h = lane / 32 takes k = 16h.. of each 32-element Q4_K sub-block,
-// k = 8h.. of each 16-element Q6_K group).
+// (lane half h = lane / 32 takes k = 16h.. of each 32 elements: half a Q4_K
+// sub-block, one Q6_K scale group).
 template <int FMT>
 struct GemmW;
 template <>
@@ -66,7 +61,7 @@ struct GemmW<F_Q4_K> {
 };
 template <>
 struct GemmW<F_Q6_K> {
-    uint2 ql[8], qh[4];
+    uint4 ql[4], qh[2];  // [64-byte half g][32 bytes kk], [g]: 16 bytes of this lane half
     uint4 sc;
     uint32_t d;
 };
@@ -78,13 +73,11 @@ __device__ __forceinline__ void gemm_w_load(GemmW<F_Q4_K> &W, const uint8_t *blk
 }
 __device__ __forceinline__ void gemm_w_load(GemmW<F_Q6_K> &W, const uint8_t *blk, int half) {
 #pragma unroll
-    for (int g = 0; g < 2; g++)
+    for (int g = 0; g < 2; g++) {
+        W.qh[g] = ld16(blk + 128 + 32 * g + 16 * half);
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            W.qh[2 * g + h] = ld8(blk + 128 + 32 * g + 16 * h + 8 * half);
-#pragma unroll
-            for (int kk = 0; kk < 2; kk++) W.ql[4 * g + 2 * h + kk] = ld8(blk + 64 * g + 32 * kk + 16 * h + 8 * half);
-        }
+        for (int kk = 0; kk < 2; kk++) W.ql[2 * g + kk] = ld16(blk + 64 * g + 32 * kk + 16 * half);
+    }
     W.sc = ld16(blk + 192);
     W.d = ld2(blk + 208);
 }
@@ -134,11 +127,12 @@ __device__ __forceinline__ rh_v4i bytes_times(const rh_v4i &x, int s) {
 // NT = 2 (390 with a minimum MFMA per sub-block and one token tile), about 60% busy;
 // the waits are the barrier and the start of each tile.  Gate and up of an
 // 8B-class model, 28672 x 4096, 512 tokens in one launch: 161 us (747 TOP/s);
-// two launches of the one-tile kernel before, 244.  Q6_K: about 430
-// instructions per tile (256 of them the groups' scale multiply-adds), 587
-// with one token tile: 4096 x 14336, 512 tokens 242 us, K split 301.  Measured and dropped: four
-// token tiles (spills at two waves per SIMD: 189 us); each row tile's token
-// tiles on one XCD (160).
+// two launches of the one-tile kernel before, 244.  Q6_K: the row decode is 330
+// instructions, a tile 80: with a multiply-add per scale group and output
+// instead (430 per tile), 4096 x 14336 and 14336 x 4096, 512 tokens took 242 and
+// 213 us, now 164 and 163 (367 TOP/s).  Measured and dropped: four token tiles
+// (spills at two waves per SIMD: 189 us); each row tile's token tiles on one XCD
+// (160).
 typedef _Float16 rh_v8h __attribute__((ext_vector_type(8)));
 typedef float rh_v16f __attribute__((ext_vector_type(16)));
 typedef float rh_v4f __attribute__((ext_vector_type(4)));
@@ -211,61 +205,63 @@ __device__ __forceinline__ void q4k_tile(const Q4kOps &O, const int8_t *xr, rh_v
     }
 }
 
-// One block of the lane's Q6_K row as MFMA B operands: the sixteen 16-element
-// groups' q - 32 (8 bytes of the lane half), their scales, d.
+// One block of the lane's Q6_K row as MFMA B operands.  Lane half h holds
+// elements 16 h .. + 15 of every 32, i.e. one scale group, so the products
+// sc (q - 32) (at most 4096 in magnitude) can be the operand: as the signed
+// bytes hi and lo of 256 hi + lo, one pair per 32 elements.
 struct Q6kOps {
-    uint2 b[16];
-    uint32_t sc[4];
+    rh_v4i hi[8], lo[8];
     float d;
 };
-__device__ __forceinline__ void q6k_decode(Q6kOps &O, const GemmW<F_Q6_K> &W) {
+__device__ __forceinline__ void q6k_decode(Q6kOps &O, const GemmW<F_Q6_K> &W, int half) {
     O.d = h2f((uint16_t)W.d);
-    O.sc[0] = W.sc.x;
-    O.sc[1] = W.sc.y;
-    O.sc[2] = W.sc.z;
-    O.sc[3] = W.sc.w;
+    const uint32_t sc4[4] = {W.sc.x, W.sc.y, W.sc.z, W.sc.w};
 #pragma unroll
-    for (int g = 0; g < 2; g++)
+    for (int g = 0; g < 2; g++) {
+        const uint32_t qh4[4] = {W.qh[g].x, W.qh[g].y, W.qh[g].z, W.qh[g].w};
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint2 qh = W.qh[2 * g + h];
+        for (int k = 0; k < 4; k++) {
+            const uint4 ql = W.ql[2 * g + (k & 1)];
+            const uint32_t ql4[4] = {ql.x, ql.y, ql.z, ql.w};
+            // scale 8 g + 2 k + half; p + 128 = sc q + (128 - 32 sc), 16 bits each
+            const int sc = (int)(int8_t)(sc4[2 * g + (k >> 1)] >> (16 * (k & 1) + 8 * half));
+            const unsigned short su = (unsigned short)sc, cu = (unsigned short)(128 - 32 * sc);
+            const rh_u16x2 s2 = {su, su}, c2 = {cu, cu};
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint2 ql = W.ql[4 * g + 2 * h + (k & 1)];
-                const int sh = 4 * (k >> 1);
-                const uint32_t q0 = ((ql.x >> sh) & 0x0F0F0F0Fu) | (((qh.x >> (2 * k)) & 0x03030303u) << 4);
-                const uint32_t q1 = ((ql.y >> sh) & 0x0F0F0F0Fu) | (((qh.y >> (2 * k)) & 0x03030303u) << 4);
-                O.b[8 * g + 2 * k + h] = make_uint2(q6_signed4(q0), q6_signed4(q1));
+            for (int i = 0; i < 4; i++) {
+                const uint32_t hb = (k < 2 ? qh4[i] << (4 - 2 * k) : qh4[i] >> (2 * k - 4)) & 0x30303030u;
+                const uint32_t q = ((k < 2 ? ql4[i] : ql4[i] >> 4) & 0x0F0F0F0Fu) | hb;
+                const uint32_t qe = q & 0x00FF00FFu;
+                const rh_u16x2 qo = __builtin_bit_cast(rh_u16x2, q) >> 8;
+                const uint32_t pe = __builtin_bit_cast(uint32_t, __builtin_bit_cast(rh_u16x2, qe) * s2 + c2);
+                const uint32_t po = __builtin_bit_cast(uint32_t, qo * s2 + c2);
+                // bytes of (po:pe): 0..3 are pe's, 4..7 po's
+                O.hi[4 * g + k][i] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
+                O.lo[4 * g + k][i] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
             }
         }
+    }
 }
 
 // The block's values (dx d) isum of 32 rows x 32 tokens: xr the lane's token
-// row of the LDS tile (+ 8 half); dv and out as q4k_tile's.
+// row of the LDS tile (+ 16 half); dv and out as q4k_tile's.
 template <class Dv, class Out>
 __device__ __forceinline__ void q6k_tile(const Q6kOps &O, const int8_t *xr, Dv dv, Out out) {
-    int isum[16];
+    rh_v16i hi = {}, lo = {};
 #pragma unroll
-    for (int i = 0; i < 16; i++) isum[i] = 0;
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-        const long a = *(const long *)(xr + 16 * e);
-        const long bq = (long)((uint64_t)O.b[e].x | ((uint64_t)O.b[e].y << 32));
-        const int sc = (int)(int8_t)(O.sc[e >> 2] >> (8 * (e & 3)));
-        const rh_v16i c = __builtin_amdgcn_mfma_i32_32x32x16_i8(a, bq, rh_v16i{}, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            isum[i] = __mul24(sc, c[i]) + isum[i];
-            // opaque to the optimiser: keeps one 24-bit multiply-add per update
-            // instead of products paired into three-input adds
-            asm("" : "+v"(isum[i]));
-        }
+    for (int e = 0; e < 8; e++) {
+        const rh_v4i a = *(const rh_v4i *)(xr + 32 * e);
+        hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, O.hi[e], hi, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, O.lo[e], lo, 0, 0, 0);
     }
 #pragma unroll
     for (int g = 0; g < 4; g++) {
         const rh_v4f dx = dv(g);
 #pragma unroll
-        for (int r = 0; r < 4; r++) out(4 * g + r, (dx[r] * O.d) * (float)isum[4 * g + r]);
+        for (int r = 0; r < 4; r++) {
+            const int i = 4 * g + r;
+            out(i, (dx[r] * O.d) * (float)((hi[i] << 8) + lo[i]));
+        }
     }
 }
 
@@ -343,7 +339,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kq_mfma_kernel(GemmArgs A) {
         if constexpr (FMT == F_Q4_K)
             q4k_decode(O, W, half);
         else
-            q6k_decode(O, W);
+            q6k_decode(O, W, half);
         load_w(bn);
         // the next block's activations, loaded a block ago, then the one after
         store_hd(nxt);
@@ -362,7 +358,7 @@ __global__ __launch_bounds__(256, 2) void gemm_kq_mfma_kernel(GemmArgs A) {
             if constexpr (FMT == F_Q4_K)
                 q4k_tile(O, xr + 16 * half, *(const rh_v8h *)(cur + HS0 + (32 * tt + n) * 32 + 16 * half), dv, out);
             else
-                q6k_tile(O, xr + 8 * half, dv, out);
+                q6k_tile(O, xr + 16 * half, dv, out);
         }
         __syncthreads();
     }
@@ -387,8 +383,8 @@ __global__ __launch_bounds__(256, 2) void gemm_kq_mfma_kernel(GemmArgs A) {
 }
 
 // The same products with the blocks of K split over the workgroup's four
-// waves, for Q6_K and for Q4_K launches with too few (row tile, token tile)
-// pairs to fill the chip: one workgroup per 32 weight rows x 32 tokens, wave w
+// waves, for launches with too few (row tile, token tile) pairs to fill the
+// chip: one workgroup per 32 weight rows x 32 tokens, wave w
 // computing blocks w, w+4, w+8, ...  Each wave stages its own block's
 // activations in its own LDS tile, computes the block's per-output value
 // exactly as the unsplit kernel does, and leaves the 16 values of each lane in
@@ -453,8 +449,8 @@ __global__ __launch_bounds__(256) void gemm_kq_mfma_ks_kernel(GemmArgs A) {
                          [&](int i, float val) { v[i] = val; });
             } else {
                 Q6kOps O;
-                q6k_decode(O, W);
-                q6k_tile(O, xs + n * GEMM_XS + 8 * half, [&](int g) { return dv[g]; },
+                q6k_decode(O, W, half);
+                q6k_tile(O, xs + n * GEMM_XS + 16 * half, [&](int g) { return dv[g]; },
                          [&](int i, float val) { v[i] = val; });
             }
         }

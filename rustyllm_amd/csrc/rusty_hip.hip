@@ -1259,16 +1259,24 @@ static int gemm_kq_enqueue(const GemmMat *ms, int n, const BatchXq &b, int T, in
     // 512 workgroups): 34 either way; 14336 x 4096, 37 tokens (112 or 224): 29 and
     // 21.6, K split 27; 1024 x 4096, 512 tokens (128 with 32 tokens): K split 15.1,
     // 20.5 with 32; 4096 x 4096, 64 tokens: 10.4 and 19.6.
-    // Q6_K: 64 tokens per workgroup where every CU gets one, else K split:
-    // 4096 x 14336, 512 tokens (256 workgroups) 242 and 301; 14336 x 4096, 512
-    // tokens 213 and 333; 4096 x 14336, 100 tokens (64) 224 and 91.
+    // Q6_K: 32 tokens per workgroup where they give three quarters of the CUs
+    // one, 64 once a CU would get a second, else K split.  us with 32 tokens, 64,
+    // K split: 14336 x 4096, 512 tokens (1792 or 896 workgroups) 223, 163, 338;
+    // 100 tokens (448 or 224) 69, 51, 89; 37 tokens (224 or 112) 42, 47, 51; 4096 x
+    // 14336, 512 tokens (512 or 256) 231, 164, 298; 256 tokens (256 or 128) 132,
+    // 150, 155; 150 tokens (160 or 96) 129, 148, 118; 1024 x 4096, 512 tokens (128
+    // or 64) 40, 47, 28.
+    // Up to 32 tokens a 64-token workgroup would only add padding.
     const int64_t wg1 = (int64_t)tiles * ((T + 31) / 32), wg2 = (int64_t)tiles * ((T + 63) / 64);
-    if (q4 && wg2 >= 2 * g.n_cu)
+    const bool two = wg2 < wg1 && (q4 ? wg2 >= 2 * g.n_cu : wg1 > g.n_cu);
+    if (q4 && two)
         launch_kq_gemm<F_Q4_K, 2>(A, tiles, s);
-    else if (!q4 && wg2 >= g.n_cu)
+    else if (two)
         launch_kq_gemm<F_Q6_K, 2>(A, tiles, s);
     else if (q4 && 4 * wg1 >= 3 * g.n_cu)
         launch_kq_gemm<F_Q4_K, 1>(A, tiles, s);
+    else if (4 * wg1 >= 3 * g.n_cu)
+        launch_kq_gemm<F_Q6_K, 1>(A, tiles, s);
     else
         for (int i = 0; i < n; i++) {
             GemmArgs B = A;
