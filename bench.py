@@ -403,10 +403,9 @@ def measure_prefill_gptoss(hip, res, toks, log):
     tot, cnt = prof.get("pf_mxfp4_gate_up", (0.0, 0))
     tflops = ops / (tot * 1e-3) / 1e12 if cnt else 0.0
     roofline = {"kernel": "pf_mxfp4_gate_up (%s: %d pairs x %d rows x %d, f32)"
-                % ("gemm_mxfp4_experts_mfma_kernel, f32 MFMA" if mfma else
-                   "gemv_mxfp4_experts_kernel, serial reference-order sums", n * cfg["top_k"],
-                   2 * cfg["hidden_dim"], cfg["dim"]),
-                "bound": "mfma" if mfma else "valu", "achieved": round(tflops, 2), "peak": FP32_PEAK_TFLOPS,
+                % ("gemm_mxfp4_experts_kernel, " + ("unrounded products" if mfma else "serial reference-order sums"),
+                   n * cfg["top_k"], 2 * cfg["hidden_dim"], cfg["dim"]),
+                "bound": "mfma", "achieved": round(tflops, 2), "peak": FP32_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(tflops / FP32_PEAK_TFLOPS, 4),
                 "ops_per_launch": ops / cnt if cnt else None,
                 "avg_launch_us": round(tot / cnt * 1e3, 1) if cnt else None, "launches": cnt}
@@ -419,8 +418,8 @@ def measure_prefill(hip, res, toks, cfg, log):
     """Batched prefill (rusty_hip_resident_prefill) of `toks` from position 0:
     whole-call wall time (host clock around the synchronous call; the tokens
     are uploaded inside it), then a profiling pass for per-launch times.  The
-    MFMA roofline is the fused gate/up batched product: 2*ffn*d_model*T int8
-    operations per launch, T = the chunk's tokens."""
+    MFMA roofline is the gate/up batched product: 2*(2*ffn)*d_model*T int8
+    operations per layer and chunk of T tokens, both matrices in one launch."""
     n = int(toks.size)
     res.prefill(toks, 0)  # warm-up (allocates the chunk buffers)
     t0 = time.perf_counter()
@@ -436,7 +435,7 @@ def measure_prefill(hip, res, toks, cfg, log):
     chunk = min(n, int(os.environ.get("RUSTY_HIP_PREFILL_CHUNK", "512")))
     tot, cnt = prof.get("pf_gemm_gate_up", (0.0, 0))
     avg_ms = tot / cnt if cnt else float("nan")
-    ops = 2.0 * cfg["hidden_dim"] * cfg["dim"] * chunk
+    ops = 4.0 * cfg["hidden_dim"] * cfg["dim"] * n * cfg["n_layers"] / max(cnt, 1)  # of an average launch
     tops = ops / (avg_ms * 1e-3) / 1e12 if cnt else 0.0
     log(f"prefill {n} tokens: {sec * 1e3:.1f} ms -> {n / sec:.1f} tok/s; gate/up product {avg_ms * 1e3:.1f} us "
         f"= {tops:.1f} TOP/s")
@@ -446,7 +445,7 @@ def measure_prefill(hip, res, toks, cfg, log):
         "ms": round(sec * 1e3, 2),
         "chunk": chunk,
         "roofline": {
-            "kernel": "pf_gemm_gate_up (Q4_K %dx%d x %d tokens, i8 MFMA)" % (cfg["hidden_dim"], cfg["dim"], chunk),
+            "kernel": "pf_gemm_gate_up (Q4_K %dx%d x %d tokens, i8 MFMA)" % (2 * cfg["hidden_dim"], cfg["dim"], chunk),
             "bound": "mfma",
             "achieved": round(tops, 1),
             "peak": INT8_PEAK_TOPS,
