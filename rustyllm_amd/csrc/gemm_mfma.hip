@@ -20,11 +20,12 @@
 //   Q6_K: two x32 MFMAs per 32 elements on the high and low bytes of
 //         sc_g (q - 32), accumulated over the block, so isum = sum_g sc_g *
 //         C_g exactly; value = (dx*d) * isum.
-// Rows and tokens past the ends read clamped (in-bounds) data or zeros and
-// are not stored.
+// Rows past the end read the last row, tokens past the end the last token or
+// the batch's padding rows (batch_rows), and neither is stored.
 #pragma once
 #include "common.hpp"
 #include "gemv.hip"
+#include "tile_index.hpp"
 
 namespace rh {
 
@@ -44,7 +45,7 @@ struct GemmArgs {
     GemmOut m[2];       // (m[1] in two-matrix Q4_K launches)
     int32_t K, T;
     int32_t epi;        // EPI_STORE or EPI_ADD
-    const int8_t *xq;   // [T][K] Q8_K quants, token-major
+    const int8_t *xq;   // [batch_rows(T)][K] Q8_K quants, token-major
     const float *dx;    // [K/256][ldx] Q8_K scales, token-minor
     const _Float16 *hs; // [K/256][ldx][16] sums of 16 quants
     int32_t ldx;        // >= T, a multiple of 64
@@ -291,14 +292,14 @@ __global__ __launch_bounds__(256, 2) void gemm_kq_mfma_kernel(GemmArgs A) {
     const uint8_t *wr = (m1 ? A.m[1].w : A.m[0].w) +
                         (int64_t)min(r0 + n, rows - 1) * (m1 ? A.m[1].row_stride : A.m[0].row_stride);
     const int nb = A.K >> 8;
-    // activation pieces: piece j of thread t is part t % 16 of token t / 16 + 16 j;
-    // tokens past the batch read zeros (their outputs are not stored)
-    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(A.xq + (int64_t)t0 * A.K), (short)0, (int)min((int64_t)(A.T - t0), (int64_t)TOK) * A.K, 0x00020000);
-    const int xoff = (tid >> 4) * A.K + 16 * (tid & 15), xdst = (tid >> 4) * GEMM_XS + 16 * (tid & 15);
+    // activation pieces (gemm_x_lane); tokens past the batch read the rows that
+    // batch_rows adds for them (their outputs are not stored)
+    const __amdgpu_buffer_rsrc_t xres =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(A.xq + (int64_t)t0 * A.K), (short)0, TOK * A.K, 0x00020000);
+    const int xoff = gemm_x_lane(tid, A.K), xdst = (tid >> 4) * GEMM_XS + 16 * (tid & 15);
     const int ht = min(t0 + min(tid, 2 * TOK - 1) / 2, A.T - 1), dt = min(t0 + min(tid, TOK - 1), A.T - 1);
     auto load_x = [&](int b, int j) {
-        return __builtin_amdgcn_raw_buffer_load_b128(xres, xoff, 16 * j * A.K + 256 * b, 0);
+        return __builtin_amdgcn_raw_buffer_load_b128(xres, xoff, gemm_x_step(j, b, A.K), 0);
     };
     typedef decltype(__builtin_amdgcn_raw_buffer_load_b128(xres, 0, 0, 0)) piece_t;
     constexpr int BB = FMT == F_Q4_K ? 144 : 210;

@@ -1179,24 +1179,23 @@ static int attn_exact_launch(AttnExactArgs A, float *scratch, const XQ &xq, hipS
 }
 
 // ---- batched K-quant products (prefill) ------------------------------------------
-// Q8_K activations of T tokens in one buffer: quants [T][K], then the scales
-// token-minor [K/256][ldx] with ldx = T rounded up to the 64-token tile, so the
-// product kernel reads four tokens' scales per 16-byte load without a bound.
+// Q8_K activations of T tokens in one buffer: quants [batch_rows(T)][K], then the
+// scales token-minor [K/256][ldx] with ldx = batch_rows(T), so that the product
+// kernels read whole tiles without a bound, then the sums of 16 [K/256][ldx][16].
 struct BatchXq {
     int8_t *qs;
     float *dx;
     int ldx;
     _Float16 *hs;
 };
-static int64_t batch_ldx(int T) { return ((int64_t)T + 63) / 64 * 64; }
 static size_t batch_xq_bytes(int T, int K) {
-    return ((size_t)T * K + 255) / 256 * 256 + (size_t)(K / 256) * batch_ldx(T) * (4 + 32);
+    return (size_t)batch_rows(T) * K + (size_t)(K / 256) * batch_rows(T) * (4 + 32);
 }
 static BatchXq batch_xq_at(int8_t *buf, int T, int K) {
     BatchXq b;
     b.qs = buf;
-    b.dx = (float *)(buf + ((size_t)T * K + 255) / 256 * 256);
-    b.ldx = (int)batch_ldx(T);
+    b.dx = (float *)(buf + (size_t)batch_rows(T) * K);
+    b.ldx = (int)batch_rows(T);
     b.hs = (_Float16 *)(b.dx + (size_t)(K / 256) * b.ldx);
     return b;
 }
