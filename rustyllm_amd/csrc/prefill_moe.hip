@@ -413,59 +413,77 @@ struct MxExpArgs {
 // pairs come first (they take twice the time of the others, and the last to
 // start should be the short ones), each kind in expert order.  One workgroup
 // of 16 waves, each with a contiguous sixteenth of the pairs: it counts its
-// pairs per expert (a ballot per expert and 64 pairs), then writes its hits
-// after the earlier waves'.  Pairs that name no expert are in no list.
+// pairs per expert, then writes its hits after the earlier waves'.  The lanes
+// of 64 pairs that share an expert come from six ballots, one per bit of its
+// number (a ballot per expert took 27 us for 4004 pairs over 32 experts, with
+// every step of the tile lists spilled; now 7.8).  Pairs that name no expert are
+// in no list.
 #define MXE_MAX_PAIRS 1024  // a token routes to an expert at most once: pairs per expert <= T
 #define MXM_PAIRS 64
 #define MXM_ROWS 128
 #define MXE_MAX_TILES (8 * MXE_MAX_PAIRS / MXM_PAIRS + 64)  // top_k <= 8, n_exp <= 64
+// The lanes of the wave whose se is this lane's (0 where it names no expert).
+__device__ __forceinline__ unsigned long long same_expert_lanes(int se, int n_exp) {
+    const bool ok = (unsigned)se < (unsigned)n_exp;
+    unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        const bool bit = (se >> i) & 1;
+        const unsigned long long set = __builtin_amdgcn_ballot_w64(bit);
+        m &= bit ? set : ~set;
+    }
+    return ok ? m : 0ull;
+}
+
 __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *sel, int n_pairs, int n_exp, int cap,
                                                                  int32_t *lists, int32_t *counts, int32_t *tiles) {
-    __shared__ int32_t s_cnt[16][64], s_long[64], s_short[64];
+    __shared__ int32_t s_cnt[16][64], s_at[16][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int per = ((n_pairs + 15) / 16 + 63) / 64 * 64, pa = min(n_pairs, wave * per), pb = min(n_pairs, pa + per);
-    int mine = 0;  // lane e: this wave's pairs of expert e
+    s_cnt[wave][lane] = 0;
+    __syncthreads();
     for (int base = pa; base < pb; base += 64) {
         const int se = base + lane < pb ? sel[base + lane] : -1;
-        for (int e = 0; e < n_exp; e++) {
-            const int c = __builtin_popcountll(__builtin_amdgcn_ballot_w64(se == e));
-            mine += lane == e ? c : 0;
-        }
+        const unsigned long long m = same_expert_lanes(se, n_exp);
+        if (m != 0 && (m & ((1ull << lane) - 1ull)) == 0) atomicAdd(&s_cnt[wave][se], __builtin_popcountll(m));
     }
-    s_cnt[wave][lane] = mine;
     __syncthreads();
     int off = 0, tot = 0;  // lane e: pairs of expert e in the earlier waves, in all waves
+#pragma unroll
     for (int w = 0; w < 16; w++) {
         const int c = s_cnt[w][lane];
         off += w < wave ? c : 0;
         tot += c;
     }
+    s_at[wave][lane] = off;
+    __syncthreads();
     for (int base = pa; base < pb; base += 64) {
         const int se = base + lane < pb ? sel[base + lane] : -1;
-        for (int e = 0; e < n_exp; e++) {
-            const unsigned long long m = __builtin_amdgcn_ballot_w64(se == e);
-            const int at = __builtin_amdgcn_readlane(off, e) + __builtin_popcountll(m & ((1ull << lane) - 1ull));
-            if (se == e && at < cap) lists[(size_t)e * cap + at] = base + lane;
-            off += lane == e ? __builtin_popcountll(m) : 0;
-        }
+        const unsigned long long m = same_expert_lanes(se, n_exp);
+        const int before = __builtin_popcountll(m & ((1ull << lane) - 1ull));
+        int at = 0;  // the first lane of each expert takes the places of all of them
+        if (m != 0 && before == 0) at = atomicAdd(&s_at[wave][se], __builtin_popcountll(m));
+        at = __shfl(at, m != 0 ? __builtin_ctzll(m) : lane, 64) + before;
+        if (m != 0 && at < cap) lists[(size_t)se * cap + at] = base + lane;
     }
     if (wave == 0) {
         tot = lane < n_exp ? min(tot, cap) : 0;
         const int rem = tot % MXM_PAIRS, full = tot / MXM_PAIRS;
         const int n_long = full + (rem > MXM_PAIRS / 2 ? 1 : 0), n_short = rem > 0 && rem <= MXM_PAIRS / 2 ? 1 : 0;
-        s_long[lane] = n_long;
-        s_short[lane] = n_short;
         if (lane < n_exp) counts[lane] = tot;
-        int a = 0, b = 0, all = 0;  // earlier experts' long and short tiles, every long tile
-        for (int e = 0; e < 64; e++) {
-            const int l = s_long[e];
-            all += l;
-            a += e < lane ? l : 0;
-            b += e < lane ? s_short[e] : 0;
+        // long and short tiles of the experts up to and including this one (at
+        // most MXE_MAX_TILES of both: 16 bits each)
+        int upto = n_long << 16 | n_short;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(upto, o, 64);
+            upto += lane >= o ? v : 0;
         }
-        for (int i = 0; i < n_long; i++) tiles[1 + a + i] = lane | i << 8;
-        if (n_short) tiles[1 + all + b] = lane | full << 8;
-        if (lane == 63) tiles[0] = all + b + n_short;
+        const int total = __builtin_amdgcn_readlane(upto, 63), all_long = total >> 16;
+        const int l0 = (upto >> 16) - n_long, s0 = all_long + (upto & 0xFFFF) - n_short;
+        for (int i = 0; i < n_long; i++) tiles[1 + l0 + i] = lane | i << 8;
+        if (n_short) tiles[1 + s0] = lane | full << 8;
+        if (lane == 0) tiles[0] = all_long + (total & 0xFFFF);
     }
 }
 

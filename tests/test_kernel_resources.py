@@ -1,0 +1,36 @@
+"""Registers and scratch memory of the built kernels, from the code object's
+own metadata: no kernel keeps spilled vector registers in memory."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LLVM = "/opt/rocm/llvm/bin"
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    d = tmp_path_factory.mktemp("code")
+    shutil.copy(os.path.join(ROOT, "rustyllm_amd", "librusty_hip.so"), d / "lib.so")
+    subprocess.run([f"{LLVM}/llvm-objdump", "--offloading", "lib.so"], cwd=d, check=True, capture_output=True)
+    obj = next(f for f in os.listdir(d) if f.endswith("gfx950"))
+    notes = subprocess.run([f"{LLVM}/llvm-readelf", "--notes", obj], cwd=d, check=True, capture_output=True, text=True)
+    found = {}
+    for part in notes.stdout.split("- .agpr_count:")[1:]:
+        name = re.search(r"\.name:\s+(\S+)", part).group(1)
+        found[name] = {k: int(v) for k, v in re.findall(r"\.(\w+):\s+(\d+)\s*$", part, re.M)}
+    return found
+
+
+def test_no_kernel_spills_vector_registers(kernels):
+    assert kernels
+    bad = {n: k["vgpr_spill_count"] for n, k in kernels.items() if k["vgpr_spill_count"]}
+    assert not bad
+
+
+def test_expert_lists_use_no_scratch(kernels):
+    lists = [k for n, k in kernels.items() if "moe_expert_lists" in n]
+    assert lists and all(k["private_segment_fixed_size"] == 0 and k["sgpr_spill_count"] == 0 for k in lists)
