@@ -408,18 +408,20 @@ struct MxExpArgs {
 };
 
 // For every expert, the pairs routed to it in pair order (lists[e * cap ..]),
-// their count, and the pair tiles of all experts: tiles[0] of them, tiles[1 +
-// i] = e | (first pair / MXM_PAIRS) << 8.  Tiles of more than MXM_PAIRS / 2
-// pairs come first (they take twice the time of the others, and the last to
-// start should be the short ones), each kind in expert order.  One workgroup
-// of 16 waves, each with a contiguous sixteenth of the pairs: it counts its
-// pairs per expert, then writes its hits after the earlier waves'.  The lanes
-// of 64 pairs that share an expert come from six ballots, one per bit of its
-// number (a ballot per expert took 27 us for 4004 pairs over 32 experts, with
-// every step of the tile lists spilled; now 7.8).  Pairs that name no expert are
-// in no list.
+// their count, and the pair tiles of all experts.  For the serial product
+// tiles[0] of them, tiles[1 + i] = e | (first pair / MXM_PAIRS) << 8: tiles of
+// more than MXM_PAIRS / 2 pairs come first (they take twice the time of the
+// others, and the last to start should be the short ones), each kind in expert
+// order.  For the opt-in one (OFFSETS) tiles[e] = the tiles of MXO_PAIRS before
+// expert e's, tiles[n_exp] = all.  One workgroup of up to 16 waves, each with a
+// contiguous share of the pairs: it counts its pairs per expert, then writes its
+// hits after the earlier waves'.  The lanes of 64 pairs that share an expert
+// come from six ballots, one per bit of its number (a ballot per expert took 27
+// us for 4004 pairs over 32 experts, with every step of the tile lists spilled;
+// now 7.8).  Pairs that name no expert are in no list.
 #define MXE_MAX_PAIRS 1024  // a token routes to an expert at most once: pairs per expert <= T
-#define MXM_PAIRS 64
+#define MXM_PAIRS 64  // pairs per tile of the serial product
+#define MXO_PAIRS 32  // ... and of the opt-in one
 #define MXM_ROWS 128
 #define MXE_MAX_TILES (8 * MXE_MAX_PAIRS / MXM_PAIRS + 64)  // top_k <= 8, n_exp <= 64
 // The lanes of the wave whose se is this lane's (0 where it names no expert).
@@ -435,22 +437,25 @@ __device__ __forceinline__ unsigned long long same_expert_lanes(int se, int n_ex
     return ok ? m : 0ull;
 }
 
+template <bool OFFSETS>
 __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *sel, int n_pairs, int n_exp, int cap,
                                                                  int32_t *lists, int32_t *counts, int32_t *tiles) {
     __shared__ int32_t s_cnt[16][64], s_at[16][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int per = ((n_pairs + 15) / 16 + 63) / 64 * 64, pa = min(n_pairs, wave * per), pb = min(n_pairs, pa + per);
+    const int nw = blockDim.x >> 6, per = ((n_pairs + nw - 1) / nw + 63) / 64 * 64;
+    const int pa = min(n_pairs, wave * per), pb = min(n_pairs, pa + per);
+    // the first 64 pairs' experts stay in a register for the second pass
+    const int first = pa + lane < pb ? sel[pa + lane] : -1;
     s_cnt[wave][lane] = 0;
     __syncthreads();
     for (int base = pa; base < pb; base += 64) {
-        const int se = base + lane < pb ? sel[base + lane] : -1;
+        const int se = base == pa ? first : base + lane < pb ? sel[base + lane] : -1;
         const unsigned long long m = same_expert_lanes(se, n_exp);
         if (m != 0 && (m & ((1ull << lane) - 1ull)) == 0) atomicAdd(&s_cnt[wave][se], __builtin_popcountll(m));
     }
     __syncthreads();
     int off = 0, tot = 0;  // lane e: pairs of expert e in the earlier waves, in all waves
-#pragma unroll
-    for (int w = 0; w < 16; w++) {
+    for (int w = 0; w < nw; w++) {
         const int c = s_cnt[w][lane];
         off += w < wave ? c : 0;
         tot += c;
@@ -458,7 +463,7 @@ __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *s
     s_at[wave][lane] = off;
     __syncthreads();
     for (int base = pa; base < pb; base += 64) {
-        const int se = base + lane < pb ? sel[base + lane] : -1;
+        const int se = base == pa ? first : base + lane < pb ? sel[base + lane] : -1;
         const unsigned long long m = same_expert_lanes(se, n_exp);
         const int before = __builtin_popcountll(m & ((1ull << lane) - 1ull));
         int at = 0;  // the first lane of each expert takes the places of all of them
@@ -468,16 +473,22 @@ __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *s
     }
     if (wave == 0) {
         tot = lane < n_exp ? min(tot, cap) : 0;
-        const int rem = tot % MXM_PAIRS, full = tot / MXM_PAIRS;
-        const int n_long = full + (rem > MXM_PAIRS / 2 ? 1 : 0), n_short = rem > 0 && rem <= MXM_PAIRS / 2 ? 1 : 0;
         if (lane < n_exp) counts[lane] = tot;
-        // long and short tiles of the experts up to and including this one (at
-        // most MXE_MAX_TILES of both: 16 bits each)
+        constexpr int PER = OFFSETS ? MXO_PAIRS : MXM_PAIRS;
+        const int rem = tot % PER, full = tot / PER;
+        const int n_long = full + (rem > PER / 2 ? 1 : 0), n_short = rem > 0 && rem <= PER / 2 ? 1 : 0;
+        // long and short tiles of the experts up to and including this one (below
+        // 2^15 of both: 16 bits each)
         int upto = n_long << 16 | n_short;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             const int v = __shfl_up(upto, o, 64);
             upto += lane >= o ? v : 0;
+        }
+        if (OFFSETS) {
+            if (lane < n_exp) tiles[lane + 1] = (upto >> 16) + (upto & 0xFFFF);
+            if (lane == 0) tiles[0] = 0;
+            return;
         }
         const int total = __builtin_amdgcn_readlane(upto, 63), all_long = total >> 16;
         const int l0 = (upto >> 16) - n_long, s0 = all_long + (upto & 0xFFFF) - n_short;
@@ -492,7 +503,7 @@ __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *s
 // workgroups past the last tile return.  Wave w owns rows row0 + 32 w ..
 // + 31 and the tile's pairs in one or two groups of 32.
 //
-// SERIAL: dot_mxfp4_f32_scalar's running sum, sum = sum + (w x) per element in
+// Every sum is dot_mxfp4_f32_scalar's running sum, sum = sum + (w x) per element in
 // order, bit for bit, on the matrix cores.  v_mfma_f32_32x32x2_f32 is a chain
 // of two fused multiply-adds in k order, each rounded (checked on the device
 // over normal, subnormal and mixed magnitudes), so a step of the chain with an
@@ -507,9 +518,6 @@ __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *s
 // whose scales are within 2^-40 .. 2^40 qualifies (products stay above 2^-126
 // and below 2^126); any other (zero, huge or non-finite values, scale bytes 0
 // and 255 among them) takes the element-by-element sums on the VALU.
-//
-// Otherwise (the opt-in product): the same chain with unrounded products,
-// element 2 i + h in k slot h of MFMA i.
 //
 // The bound is the matrix cores, 64 clocks per 32 rows x 32 pairs x element
 // (78 TFLOP/s of the reference's products), and f32 MFMAs leave the VALU
@@ -529,14 +537,14 @@ __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *s
 // 1000 pairs over 32 experts of 2880 x 2880 (31 per expert: half-filled tiles)
 // 574 against 903 us.
 #define MXM_C 8  // weight blocks per LDS chunk
-template <bool SERIAL, int PT>
+template <int PT>
 __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uint8_t *w, float *y, int row0, int np,
                                                    uint2 *s_b, float *s_x, uint32_t *s_bad, const int32_t *s_pair) {
     typedef float v4f __attribute__((ext_vector_type(4)));
     typedef float v16f __attribute__((ext_vector_type(16)));
     constexpr int XP = 68, XN = MXM_PAIRS * XP;     // pair pitch and buffer size of s_x, in floats
     constexpr int WP = MXM_C * 17, WN = MXM_ROWS * 17;  // row bytes and buffer size (8-byte pieces) of s_b
-    constexpr int NW = SERIAL ? 32 : 16;            // MFMAs per block and pair group
+    constexpr int NW = 32;                          // MFMAs per block and pair group
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int nb = A.K >> 5;
@@ -559,23 +567,16 @@ __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uin
         for (int j = 0; j < PT; j++) {
             float *r = s_x + (b & 1) * XN + (pr0 + 32 * j) * XP;
             const v4f v = xs[j];
-            if (SERIAL) {
-                *(v4f *)(r + 4 * c4) = v;
-                *(v4f *)(r + 32 + 4 * c4) = v * 3.0f;
+            *(v4f *)(r + 4 * c4) = v;
+            *(v4f *)(r + 32 + 4 * c4) = v * 3.0f;
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float f = fabsf(v[i]);
-                    bad |= (f < 0x1p-84f && f != 0.0f) || !(f < 0x1p80f);
-                }
-            } else {
-                *(float2 *)(r + 2 * c4) = make_float2(v[0], v[2]);
-                *(float2 *)(r + 32 + 2 * c4) = make_float2(v[1], v[3]);
+            for (int i = 0; i < 4; i++) {
+                const float f = fabsf(v[i]);
+                bad |= (f < 0x1p-84f && f != 0.0f) || !(f < 0x1p80f);
             }
         }
-        if (SERIAL) {
-            const uint32_t any = __builtin_amdgcn_ballot_w64(bad) != 0 ? 1u : 0u;
-            if (lane == 0) s_bad[4 * (b & 1) + wave] = any;
-        }
+        const uint32_t any = __builtin_amdgcn_ballot_w64(bad) != 0 ? 1u : 0u;
+        if (lane == 0) s_bad[4 * (b & 1) + wave] = any;
     };
     // weights: piece f = 256 i + t of a chunk is row f / 17, bytes 8 (f % 17)
     constexpr int NP = (WN + 255) / 256;
@@ -615,26 +616,17 @@ __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uin
         const float sc = __builtin_bit_cast(float, ex << 23);  // 2^(ex - 127) where it is used: 0 < ex < 255
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            if (SERIAL) {
-                const uint32_t lo = __builtin_amdgcn_perm(thi, tlo, wd[q] & 0x07070707u);
-                const uint32_t hi = __builtin_amdgcn_perm(thi, tlo, (wd[q] >> 4) & 0x07070707u);
-                const uint32_t u = (lo | (hi << 4)) | (wd[q] & 0x88888888u);
+            const uint32_t lo = __builtin_amdgcn_perm(thi, tlo, wd[q] & 0x07070707u);
+            const uint32_t hi = __builtin_amdgcn_perm(thi, tlo, (wd[q] >> 4) & 0x07070707u);
+            const uint32_t u = (lo | (hi << 4)) | (wd[q] & 0x88888888u);
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const fp4x2_f32 p = fp4x2_scaled(u, sc, i);
-                    wv[(8 * q + 2 * i) % NW] = p.x;
-                    wv[(8 * q + 2 * i + 1) % NW] = p.y;
-                }
-            } else {
-                const uint32_t t = (wd[q] >> (4 * h)) & 0x0F0F0F0Fu, u = t | (t >> 4);
-                const fp4x2_f32 lo = fp4x2_scaled(u, sc, 0), hi = fp4x2_scaled(u, sc, 2);
-                wv[4 * q] = lo.x;
-                wv[4 * q + 1] = lo.y;
-                wv[4 * q + 2] = hi.x;
-                wv[4 * q + 3] = hi.y;
+            for (int i = 0; i < 4; i++) {
+                const fp4x2_f32 p = fp4x2_scaled(u, sc, i);
+                wv[8 * q + 2 * i] = p.x;
+                wv[8 * q + 2 * i + 1] = p.y;
             }
         }
-        return SERIAL ? ex - 87u > 80u : ex - 1u > 253u;
+        return ex - 87u > 80u;
     };
     v16f acc[PT];
 #pragma unroll
@@ -650,12 +642,11 @@ __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uin
         for (int e = 0; e < 32; e++) {
             const uint32_t byte = blk[e >> 1];
             const float wv = mxfp4_nibble((e & 1) ? byte >> 4 : byte & 0xFu) * sc;
-            const int at = SERIAL ? e : (e & 1) * 32 + (e >> 1);
 #pragma unroll
             for (int g = 0; g < PT; g++)
 #pragma unroll
                 for (int i = 0; i < 16; i++)
-                    acc[g][i] += wv * xc[(32 * g + 8 * (i >> 2) + (i & 3)) * XP + at];
+                    acc[g][i] += wv * xc[(32 * g + 8 * (i >> 2) + (i & 3)) * XP + e];
         }
     };
     load_w(0);
@@ -677,11 +668,8 @@ __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uin
             if (j == MXM_C - 2) store_w(c + 1);
         }
         if (b == 0) odd = __builtin_amdgcn_ballot_w64(decode(0, wcur)) != 0;
-        uint32_t xbad = 0;
-        if (SERIAL) {
-            const uint4 b4 = *(const uint4 *)(s_bad + 4 * (b & 1));
-            xbad = __builtin_amdgcn_readfirstlane(b4.x | b4.y | b4.z | b4.w);
-        }
+        const uint4 b4 = *(const uint4 *)(s_bad + 4 * (b & 1));
+        const uint32_t xbad = __builtin_amdgcn_readfirstlane(b4.x | b4.y | b4.z | b4.w);
         if (odd || xbad != 0) {
             slow_block(b);
         } else {
@@ -710,7 +698,6 @@ __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uin
         }
 }
 
-template <bool SERIAL>
 __global__ __launch_bounds__(256, 2) void gemm_mxfp4_experts_kernel(MxExpArgs A, const int32_t *lists,
                                                                     const int32_t *counts, const int32_t *tiles,
                                                                     int cap) {
@@ -728,9 +715,157 @@ __global__ __launch_bounds__(256, 2) void gemm_mxfp4_experts_kernel(MxExpArgs A,
     float *y = A.y[mat];
     const int row0 = blockIdx.x * MXM_ROWS;
     if (np > 32)
-        mxfp4_experts_tile<SERIAL, 2>(A, w, y, row0, np, s_b, s_x, s_bad, s_pair);
+        mxfp4_experts_tile<2>(A, w, y, row0, np, s_b, s_x, s_bad, s_pair);
     else
-        mxfp4_experts_tile<SERIAL, 1>(A, w, y, row0, np, s_b, s_x, s_bad, s_pair);
+        mxfp4_experts_tile<1>(A, w, y, row0, np, s_b, s_x, s_bad, s_pair);
+}
+
+// ---- opt-in expert product on the matrix cores ------------------------------
+// Sums of unrounded products in the matrix cores' own order: not bit-exact, and
+// off unless rusty_hip_set_expert_mfma(1) selects it.  Its inputs keep the
+// reference's precision: the weights lut[n] * 2^(e-127) are exact in f32 and
+// the activations are the f32 rows; only the order and rounding of the f32
+// additions of the K products differ (v_mfma_f32_32x32x2_f32).
+//
+// y[mat] row p = expert rows times pair p's activation for one (128-row tile,
+// 32-pair tile of one expert, matrix): grid (ceil(rows / 128), an upper bound
+// of the pair tiles, n_mats); workgroups past tile0[n_exp] return.  Wave w
+// owns rows row0 + 32 w + (lane % 32); per 32-element block, 16 MFMAs
+// 32x32x2: MFMA i takes element 16 h + i (h = lane / 32) of the block from
+// both operands, A = the pair's activation (m = pair), B = the weight (n =
+// row), so lane h decodes bytes 8h..8h+7 of its row's block (element 2b + 1
+// is the high nibble of byte b).  The weights arrive in 16-block chunks of
+// 272 bytes per row by coalesced direct loads into a double-buffered LDS
+// chunk; each lane then reads its row's chunk into registers (17 reads, an
+// odd number of 16-byte units per row: conflict-free); the activations come
+// from global memory one block ahead.
+//
+// Bound by the latency of a workgroup's K loop until the grid passes two
+// workgroups per CU: hence 32 pairs per tile, a second tile going to a second
+// CU, and one barrier per 16 blocks.  Measured, us per call, against this
+// product in the serial kernel's tiles (64 pairs, activations in LDS, a barrier
+// per block): 6 experts x 720 x 2880, 256 pairs 73 : 137, 1000 pairs 84 : 141;
+// 32 experts x 2880 x 2880, 64 pairs 171 : 212, 1000 pairs 277 : 306; prefill of
+// 1001 tokens, 4 gpt-oss-20b layers, 18.9 ms (26.8 with the serial sums).  A
+// workgroup looks its expert up by walking the offsets: with the tile list
+// instead all start at once, the 736 workgroups of 32 experts x 2880 rows end
+// together too, and the second round lands two to a CU: 215 : 172.
+__global__ __launch_bounds__(256) void gemm_mxfp4_experts_mfma_kernel(MxExpArgs A, const int32_t *lists,
+                                                                      const int32_t *counts, const int32_t *tile0,
+                                                                      int cap) {
+    __shared__ __align__(16) uint4 s_b[2][MXM_ROWS * 17];
+    __shared__ int32_t s_pair[MXO_PAIRS];
+    typedef float v16f __attribute__((ext_vector_type(16)));
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int mat = blockIdx.z, gt = blockIdx.y;
+    const int n_exp = A.n_exp;
+    if (gt >= tile0[n_exp]) return;  // uniform
+    int e = 0;
+    while (e + 1 < n_exp && tile0[e + 1] <= gt) e++;
+    const int p0 = (gt - tile0[e]) * MXO_PAIRS;
+    const int np = min(MXO_PAIRS, counts[e] - p0);
+    if (tid < MXO_PAIRS) s_pair[tid] = lists[(size_t)e * cap + p0 + min(tid, np - 1)];
+    const int m = lane & 31, h = lane >> 5;
+    const int row0 = blockIdx.x * MXM_ROWS, row = row0 + 32 * wave + m;
+    const uint8_t *w = A.w[mat] + (int64_t)e * A.exp_stride;
+    const int64_t stride = A.row_stride;
+    const int nb = A.K >> 5, nch = (nb + MXF_C - 1) / MXF_C;
+    // piece f = 256 i + tid of a chunk: row f / 17, bytes 16 (f % 17); the
+    // 2176 pieces are 34 whole wave instructions, so a wave's instruction is
+    // either all inside the chunk or skipped
+    auto issue_chunk = [&](int c, int buf) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) {
+            if (256 * i + 64 * wave >= MXM_ROWS * 17) continue;  // uniform
+            const int f = 256 * i + tid, r = f / 17, pc = f - 17 * r;
+            const int rr = min(row0 + r, A.rows - 1);
+            const int64_t o = min((int64_t)(MXF_C * 17 * c + 16 * pc), stride - 16);
+            dma16(w + (int64_t)rr * stride + o, &s_b[buf][256 * i + 64 * wave]);
+        }
+    };
+    issue_chunk(0, 0);
+    __syncthreads();  // s_pair
+    const int pair = s_pair[m];
+    const float *xr = A.x + (A.x_pair ? (int64_t)pair : (int64_t)(pair / A.k)) * A.ldx + 16 * h;
+    float4 xa[4], xb[4];
+    auto load_x = [&](int b, float4 (&xv)[4]) {
+        const float4 *p = (const float4 *)(xr + 32 * (int64_t)min(b, nb - 1));
+#pragma unroll
+        for (int q = 0; q < 4; q++) xv[q] = p[q];
+    };
+    load_x(0, xa);
+    v16f acc = {};
+    for (int c = 0; c < nch; c++) {
+        RH_WAIT_VM(0);
+        __syncthreads();  // chunk c landed from every wave; every read of chunk c - 1 done
+        uint32_t wr[68];
+        {
+            const uint4 *rp = &s_b[c & 1][(32 * wave + m) * 17];
+#pragma unroll
+            for (int q = 0; q < 17; q++) {
+                const uint4 v = rp[q];
+                wr[4 * q] = v.x;
+                wr[4 * q + 1] = v.y;
+                wr[4 * q + 2] = v.z;
+                wr[4 * q + 3] = v.w;
+            }
+        }
+        // block j of the chunk with its activations in cur; the next block's
+        // go to nxt (clamped past the end), then, late in the chunk, the next
+        // chunk's weights are issued: a load issued after them would wait for
+        // them too (loads retire in order), and only the next chunk's first
+        // activations are
+        auto block = [&](int j, const float4 (&cur)[4], float4 (&nxt)[4]) {
+            const int b = MXF_C * c + j;
+            if (b >= nb) return;  // uniform
+            load_x(b + 1, nxt);
+            if (j == MXF_C - 2 && c + 1 < nch) issue_chunk(c + 1, (c + 1) & 1);
+            // bytes 17 j + 8 h .. + 7 and the scale byte 17 j + 16
+            const int o0 = 17 * j, o1 = 17 * j + 8, os = 17 * j + 16;
+            const uint32_t a0 = __builtin_amdgcn_alignbyte(wr[o0 / 4 + 1], wr[o0 / 4], o0 % 4);
+            const uint32_t a1 = __builtin_amdgcn_alignbyte(wr[o0 / 4 + 2], wr[o0 / 4 + 1], o0 % 4);
+            const uint32_t c0 = __builtin_amdgcn_alignbyte(wr[o1 / 4 + 1], wr[o1 / 4], o1 % 4);
+            const uint32_t c1 = __builtin_amdgcn_alignbyte(wr[o1 / 4 + 2], wr[o1 / 4 + 1], o1 % 4);
+            const uint32_t d0 = h ? c0 : a0, d1 = h ? c1 : a1;
+            const uint32_t ex = (wr[os / 4] >> (8 * (os % 4))) & 0xFFu;
+            const float sc = mxfp4_scale(ex);
+            float wv[16];
+            if (__builtin_amdgcn_ballot_w64(ex == 0u || ex == 255u) == 0) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const fp4x2_f32 lo = fp4x2_scaled(d0, sc, u), hi = fp4x2_scaled(d1, sc, u);
+                    wv[2 * u] = lo.x;
+                    wv[2 * u + 1] = lo.y;
+                    wv[8 + 2 * u] = hi.x;
+                    wv[9 + 2 * u] = hi.y;
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const uint32_t b0 = (d0 >> (8 * u)) & 0xFFu, b1 = (d1 >> (8 * u)) & 0xFFu;
+                    wv[2 * u] = mxfp4_nibble(b0 & 0xFu) * sc;
+                    wv[2 * u + 1] = mxfp4_nibble(b0 >> 4) * sc;
+                    wv[8 + 2 * u] = mxfp4_nibble(b1 & 0xFu) * sc;
+                    wv[9 + 2 * u] = mxfp4_nibble(b1 >> 4) * sc;
+                }
+            }
+            const float xs[16] = {cur[0].x, cur[0].y, cur[0].z, cur[0].w, cur[1].x, cur[1].y, cur[1].z, cur[1].w,
+                                  cur[2].x, cur[2].y, cur[2].z, cur[2].w, cur[3].x, cur[3].y, cur[3].z, cur[3].w};
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xs[i], wv[i], acc, 0, 0, 0);
+        };
+#pragma unroll
+        for (int j = 0; j < MXF_C; j += 2) {
+            block(j, xa, xb);
+            block(j + 1, xb, xa);
+        }
+    }
+    if (row >= A.rows) return;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int mi = 8 * (i >> 2) + 4 * h + (i & 3);
+        if (mi < np) A.y[mat][(int64_t)s_pair[mi] * A.ldy + row] = acc[i];
+    }
 }
 
 // K/V rows between a ring cache and the linear buffer of a batched ring

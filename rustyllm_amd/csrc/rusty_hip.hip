@@ -2261,8 +2261,7 @@ struct Resident {
     float *pxn = nullptr, *plk = nullptr, *plv = nullptr, *plog = nullptr, *pprob = nullptr, *pgate = nullptr,
           *pup = nullptr, *pproj = nullptr;
     int32_t *psel = nullptr;
-    // the matrix-core expert product's per-expert pair lists, counts and
-    // tile offsets (rusty_hip_set_expert_mfma)
+    // the expert product's per-expert pair lists, counts and pair tiles
     int32_t *plists = nullptr, *pcounts = nullptr, *ptiles = nullptr;
     std::map<std::pair<int, uint32_t>, hipGraphExec_t> graphs;  // by (mode, penalty bits)
     std::vector<void *> allocs;
@@ -2936,9 +2935,10 @@ static int r_prefill_moe_alloc() {
 }
 
 // The expert product of the batched gpt-oss prefill on the matrix cores (the
-// pair lists first, then gemm_mxfp4_experts_kernel): the reference's serial
-// row sums (bit-exact; the default) or, when rusty_hip_set_expert_mfma(1)
-// chose it, sums of unrounded products.  lists/counts/tiles: the list
+// pair lists first): the reference's serial row sums
+// (gemm_mxfp4_experts_kernel, bit-exact; the default) or, when
+// rusty_hip_set_expert_mfma(1) chose it, sums of unrounded products
+// (gemm_mxfp4_experts_mfma_kernel).  lists/counts/tiles: the list
 // buffers; with lists_ready the lists of this sel are already built.
 static int g_expert_mfma = -1;
 static bool expert_mfma_on() {
@@ -2956,22 +2956,28 @@ static int experts_enqueue(MxExpArgs A, int n_mats, bool mfma, int32_t *lists, i
     if (A.n_pairs > MXE_MAX_PAIRS * A.k || A.row_stride % 16 != 0) return 0;
     // (the opt-in product refuses activations off 16-byte rows, as it always has)
     if (mfma && (A.ldx % 4 != 0 || ((uintptr_t)A.x & 15) != 0)) return 0;
+    const int per_tile = mfma ? MXO_PAIRS : MXM_PAIRS;
     if (!lists_ready) {
         ProfScope ps("moe_expert_lists", s);
-        rh_launch(moe_expert_lists_kernel, dim3(1), dim3(1024), 0, s, A.sel, A.n_pairs, A.n_exp, MXE_MAX_PAIRS, lists,
-                  counts, tiles);
+        const dim3 waves(A.n_pairs <= 256 ? 256 : 1024);
+        if (mfma)
+            rh_launch(moe_expert_lists_kernel<true>, dim3(1), waves, 0, s, A.sel, A.n_pairs, A.n_exp, MXE_MAX_PAIRS,
+                      lists, counts, tiles);
+        else
+            rh_launch(moe_expert_lists_kernel<false>, dim3(1), waves, 0, s, A.sel, A.n_pairs, A.n_exp,
+                      MXE_MAX_PAIRS, lists, counts, tiles);
         RH_LAUNCH_OK();
     }
-    // at most floor(n_pairs / 64) full pair tiles and one partial tile per expert
-    const unsigned n_tiles = (unsigned)(A.n_pairs / MXM_PAIRS + std::min(A.n_exp, A.n_pairs));
+    // at most floor(n_pairs / per_tile) full pair tiles and one partial tile per expert
+    const unsigned n_tiles = (unsigned)(A.n_pairs / per_tile + std::min(A.n_exp, A.n_pairs));
     const dim3 grid((unsigned)((A.rows + MXM_ROWS - 1) / MXM_ROWS), n_tiles, (unsigned)n_mats);
     ProfScope ps(name, s);
     if (mfma)
-        rh_launch(gemm_mxfp4_experts_kernel<false>, grid, dim3(256), 0, s, A, (const int32_t *)lists,
-                  (const int32_t *)counts, (const int32_t *)tiles, (int)MXE_MAX_PAIRS);
+        rh_launch(gemm_mxfp4_experts_mfma_kernel, grid, dim3(256), 0, s, A, (const int32_t *)lists, (const int32_t *)counts,
+                  (const int32_t *)tiles, (int)MXE_MAX_PAIRS);
     else
-        rh_launch(gemm_mxfp4_experts_kernel<true>, grid, dim3(256), 0, s, A, (const int32_t *)lists,
-                  (const int32_t *)counts, (const int32_t *)tiles, (int)MXE_MAX_PAIRS);
+        rh_launch(gemm_mxfp4_experts_kernel, grid, dim3(256), 0, s, A, (const int32_t *)lists, (const int32_t *)counts,
+                  (const int32_t *)tiles, (int)MXE_MAX_PAIRS);
     RH_LAUNCH_OK();
     return 1;
 }
@@ -3626,7 +3632,7 @@ int rusty_hip_mxfp4_experts(const uint8_t *w, int64_t row_stride, int64_t exp_st
         row_stride < (int64_t)cols / 32 * 17 || row_stride % 16 != 0 || exp_stride < (int64_t)rows * row_stride ||
         ldy < (int64_t)rows || ldx < (int64_t)cols)
         return 0;
-    static int32_t *lists[64] = {};  // per device: pair lists, counts, tile offsets
+    static int32_t *lists[64] = {};  // per device: pair lists, counts, pair tiles
     if (g.dev < 0 || g.dev >= 64) return 0;
     int32_t *&L = lists[g.dev];
     if (!L && hipMalloc((void **)&L, ((size_t)64 * MXE_MAX_PAIRS + 64 + 1 + MXE_MAX_TILES) * 4) != hipSuccess) {

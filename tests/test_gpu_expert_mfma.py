@@ -161,3 +161,32 @@ def test_gptoss_prefill_with_expert_mfma(hip, name, max_len, pieces):
     finally:
         hip.set_expert_mfma(prev)
         hip.attention_mode(prev_mode)
+
+
+@pytest.mark.parametrize("rows,cols,counts", [(40, 96, [33, 1, 0, 31]), (129, 544, [65, 2])])
+def test_expert_product_mfma_order(hip, rows, cols, counts):
+    """The opt-in sums' order is part of what a caller sees from run to run:
+    one chain of fused multiply-adds per output that takes elements i and
+    16 + i of each 32-element block in turn, i = 0 .. 15, at any tile."""
+    import torch
+    dev = torch.device("cuda:0")
+    n_exp = len(counts)
+    w, stride, _ = _experts(n_exp, rows, cols, 43, dequant=False)
+    rb = synth.row_bytes(MX, cols)
+    deq = np.stack([O.dequant(MX, np.ascontiguousarray(w[e, :, :rb]), rows, cols) for e in range(n_exp)])
+    sel = np.random.default_rng(2).permutation(np.repeat(np.arange(n_exp), counts)).astype(np.int32)
+    x = synth.normal_f32(19, sel.size, cols).reshape(sel.size, cols)
+    tw, tx, ts = (torch.from_numpy(a).to(dev) for a in (w.reshape(-1), x, sel))
+    ty = torch.zeros(sel.size, rows, dtype=torch.float32, device=dev)
+    torch.cuda.synchronize()
+    assert hip.mxfp4_experts_dev(tw.data_ptr(), stride, rows * stride, n_exp, rows, cols, tx.data_ptr(), cols, True, 1,
+                                 ts.data_ptr(), sel.size, ty.data_ptr(), rows, True)
+    # the product is exact in 64 bits of mantissa, and so is all but the last
+    # rounding of the sum
+    wd = deq.reshape(n_exp, rows, cols)[sel].astype(np.longdouble)
+    ref = np.zeros((sel.size, rows), np.float32)
+    for b in range(0, cols, 32):
+        for i in range(16):
+            for e in (b + i, b + 16 + i):
+                ref = (ref.astype(np.longdouble) + wd[:, :, e] * x[:, None, e].astype(np.longdouble)).astype(np.float32)
+    assert np.array_equal(ty.cpu().numpy().view(np.uint32), ref.view(np.uint32))
