@@ -437,6 +437,33 @@ __device__ __forceinline__ unsigned long long same_expert_lanes(int se, int n_ex
     return ok ? m : 0ull;
 }
 
+// The tiles of PER pairs of the wave's experts, lane e's tot pairs being expert
+// e's: n_long tiles more than half full, n_short (0 or 1) others, and how many
+// there are of both up to and including this expert (below 2^15) and in all.
+struct PairTiles {
+    int full, n_long, n_short, long_upto, short_upto, long_all, short_all;
+};
+template <int PER>
+__device__ __forceinline__ PairTiles pair_tiles(int tot, int lane) {
+    PairTiles t;
+    const int rem = tot % PER;
+    t.full = tot / PER;
+    t.n_long = t.full + (rem > PER / 2 ? 1 : 0);
+    t.n_short = rem > 0 && rem <= PER / 2 ? 1 : 0;
+    int upto = t.n_long << 16 | t.n_short;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(upto, o, 64);
+        upto += lane >= o ? v : 0;
+    }
+    const int all = __builtin_amdgcn_readlane(upto, 63);
+    t.long_upto = upto >> 16;
+    t.short_upto = upto & 0xFFFF;
+    t.long_all = all >> 16;
+    t.short_all = all & 0xFFFF;
+    return t;
+}
+
 template <bool OFFSETS>
 __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *sel, int n_pairs, int n_exp, int cap,
                                                                  int32_t *lists, int32_t *counts, int32_t *tiles) {
@@ -474,28 +501,88 @@ __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *s
     if (wave == 0) {
         tot = lane < n_exp ? min(tot, cap) : 0;
         if (lane < n_exp) counts[lane] = tot;
-        constexpr int PER = OFFSETS ? MXO_PAIRS : MXM_PAIRS;
-        const int rem = tot % PER, full = tot / PER;
-        const int n_long = full + (rem > PER / 2 ? 1 : 0), n_short = rem > 0 && rem <= PER / 2 ? 1 : 0;
-        // long and short tiles of the experts up to and including this one (below
-        // 2^15 of both: 16 bits each)
-        int upto = n_long << 16 | n_short;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(upto, o, 64);
-            upto += lane >= o ? v : 0;
-        }
+        const PairTiles t = pair_tiles<OFFSETS ? MXO_PAIRS : MXM_PAIRS>(tot, lane);
         if (OFFSETS) {
-            if (lane < n_exp) tiles[lane + 1] = (upto >> 16) + (upto & 0xFFFF);
+            if (lane < n_exp) tiles[lane + 1] = t.long_upto + t.short_upto;
             if (lane == 0) tiles[0] = 0;
             return;
         }
-        const int total = __builtin_amdgcn_readlane(upto, 63), all_long = total >> 16;
-        const int l0 = (upto >> 16) - n_long, s0 = all_long + (upto & 0xFFFF) - n_short;
-        for (int i = 0; i < n_long; i++) tiles[1 + l0 + i] = lane | i << 8;
-        if (n_short) tiles[1 + s0] = lane | full << 8;
-        if (lane == 0) tiles[0] = all_long + (total & 0xFFFF);
+        const int l0 = t.long_upto - t.n_long, s0 = t.long_all + t.short_upto - t.n_short;
+        for (int i = 0; i < t.n_long; i++) tiles[1 + l0 + i] = lane | i << 8;
+        if (t.n_short) tiles[1 + s0] = lane | t.full << 8;
+        if (lane == 0) tiles[0] = t.long_all + t.short_all;
     }
+}
+
+// The same for one workgroup of the serial product without the list kernel:
+// pair tile number `tile` of at most MXE_OWN_PAIRS pairs.  Fills s_pair and
+// returns the tile's pairs (0: there is no such tile) and its expert.  Up to 64
+// pairs every wave sees them all, and tile i is the expert of the i-th pair
+// that is its expert's first; beyond, four waves with a quarter of the pairs in
+// registers each count and rank as the list kernel does (0.5 us more).
+#define MXE_OWN_PAIRS 1024
+__device__ __forceinline__ int own_pair_tile(const int32_t *sel, int n_pairs, int n_exp, int tile, int32_t (*s_cnt)[64],
+                                             int32_t *s_pair, int &expert) {
+    constexpr int G = MXE_OWN_PAIRS / 256;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (n_pairs <= 64) {
+        const int mine = lane < n_pairs ? sel[lane] : -1;
+        const unsigned long long m = same_expert_lanes(mine, n_exp);
+        const bool first = m != 0 && (m & below) == 0;
+        const unsigned long long firsts = __builtin_amdgcn_ballot_w64(first);
+        const unsigned long long at = __builtin_amdgcn_ballot_w64(first && __builtin_popcountll(firsts & below) == tile);
+        if (at == 0) return 0;
+        expert = __builtin_amdgcn_readlane(mine, __builtin_ctzll(at));
+        const bool hit = mine == expert;
+        const unsigned long long hits = __builtin_amdgcn_ballot_w64(hit);
+        if (wave == 0 && hit) s_pair[__builtin_popcountll(hits & below)] = lane;
+        return __builtin_popcountll(hits);
+    }
+    const int groups = (n_pairs + 255) / 256, pa = wave * groups * 64;
+    int se[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        const int p = pa + 64 * g + lane;
+        se[g] = g < groups && p < n_pairs ? sel[p] : -1;
+    }
+    s_cnt[wave][lane] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        if (g >= groups) break;  // uniform
+        const unsigned long long m = same_expert_lanes(se[g], n_exp);
+        if (m != 0 && (m & below) == 0) atomicAdd(&s_cnt[wave][se[g]], __builtin_popcountll(m));
+    }
+    __syncthreads();
+    int off = 0, tot = 0;  // lane e: pairs of expert e in the earlier waves, in all waves
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const int c = s_cnt[w][lane];
+        off += w < wave ? c : 0;
+        tot += c;
+    }
+    const PairTiles t = pair_tiles<MXM_PAIRS>(tot, lane);
+    if (tile >= t.long_all + t.short_all) return 0;
+    int e, p0;
+    if (tile < t.long_all) {
+        e = __builtin_ctzll(__builtin_amdgcn_ballot_w64(t.long_upto > tile));
+        p0 = (tile - __builtin_amdgcn_readlane(t.long_upto - t.n_long, e)) * MXM_PAIRS;
+    } else {
+        e = __builtin_ctzll(__builtin_amdgcn_ballot_w64(t.short_upto > tile - t.long_all));
+        p0 = __builtin_amdgcn_readlane(t.full, e) * MXM_PAIRS;
+    }
+    int at = __builtin_amdgcn_readlane(off, e) - p0;
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        const bool hit = se[g] == e;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
+        const int i = at + __builtin_popcountll(m & below);
+        if (hit && i >= 0 && i < MXM_PAIRS) s_pair[i] = pa + 64 * g + lane;
+        at += __builtin_popcountll(m);
+    }
+    expert = e;
+    return min(MXM_PAIRS, __builtin_amdgcn_readlane(tot, e) - p0);
 }
 
 // y[mat] row p for one (128-row tile, 64-pair tile of one expert, matrix).
@@ -520,63 +607,78 @@ __global__ __launch_bounds__(1024) void moe_expert_lists_kernel(const int32_t *s
 // and 255 among them) takes the element-by-element sums on the VALU.
 //
 // The bound is the matrix cores, 64 clocks per 32 rows x 32 pairs x element
-// (78 TFLOP/s of the reference's products), and f32 MFMAs leave the VALU
-// almost no room: beside 16x16x4 MFMAs each VALU instruction adds 2.5 to 4
-// clocks of a SIMD's 32 per MFMA.  Hence the 32x32 shape (half the operands
-// per product of 16x16; 16-pair groups, 64 rows per workgroup and the factor 3
-// in the loop took 1504 us for 1024 pairs of 11520 x 2880, 57% of the bound),
-// RN(3 x) computed once per workgroup into a plane of its own, and the code
-// lookup on four nibbles per v_perm.  Weights come from a double-buffered LDS
-// chunk of 8 blocks (rows of 136 bytes: 32 rows of a dword read are on distinct
-// banks), the activations from a double-buffered block of two planes per pair
-// (pitch 68 floats, 16-byte reads); both are loaded through registers one
-// chunk or block ahead, one barrier per block, 70 KB of LDS and two workgroups
-// per CU.  Measured: 1024 pairs of 11520 x 2880 1195 us (57 TFLOP/s, 0.72 of
-// the bound); the 4004 gate/up pairs of a 1001-token gpt-oss-20b chunk 2.68 ms
-// (49.5 TFLOP/s) where eight VALU sums per wave, x by scalar loads, took 6.92;
-// 1000 pairs over 32 experts of 2880 x 2880 (31 per expert: half-filled tiles)
-// 574 against 903 us.
+// (78 TFLOP/s of the reference's products), and an f32 MFMA leaves the VALU no
+// room: a chain of 32x32x2 MFMAs takes 64 clocks each, 122 with twelve adds and
+// multiplies after each one, interleaved or not.  Hence the 32x32 shape (half
+// the operands per product of 16x16; 16-pair groups, 64 rows per workgroup and
+// the factor 3 in the loop took 1504 us for 1024 pairs of 11520 x 2880, 57% of
+// the bound), RN(3 x) computed once per workgroup into a plane of its own, and
+// the code lookup on four nibbles per v_perm.  Weights come from a
+// double-buffered LDS chunk of 8 blocks (rows of 136 bytes: 32 rows of a dword
+// read are on distinct banks), the activations from two double-buffered planes
+// (pitch 68 floats, 16-byte reads); both are loaded through registers one chunk
+// or barrier ahead, 71 KB of LDS and two workgroups per CU.  A tile of up to 32
+// pairs runs two blocks between barriers in the room of the second group's
+// activations: where the grid leaves CUs idle a workgroup's time per block is
+// what counts, 1.5 us with one block per barrier, the decode after the MFMAs and
+// the range check as 24 compares, now 1.27 (0.85 of it MFMAs).
+//
+// Measured, us per call, against eight VALU sums per wave (x by scalar loads,
+// 64-row workgroups): 1024 pairs of 11520 x 2880 1197 (57 TFLOP/s, 0.72 of the
+// bound) : 11733; 1000 pairs over 32 experts of 2880 x 2880 (31 per expert:
+// half-filled tiles) 499 : 898; 12 pairs 131 : 245; 6 pairs of 720 x 2880 126 :
+// 136; 12 pairs of 96 x 96 19 : 19.  Over 288 shapes of 6 to 32 experts, 6 to
+// 1000 pairs, 96 to 2880 rows and columns it is slower, by 3%, only where the
+// tiles barely exceed the CUs and hold a pair or two each (264 workgroups: 224 :
+// 216).  The 4004 gate/up pairs of a 1001-token gpt-oss-20b chunk take 2.5 ms
+// (53 TFLOP/s), 6.9 with the VALU sums.
 #define MXM_C 8  // weight blocks per LDS chunk
 template <int PT>
 __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uint8_t *w, float *y, int row0, int np,
                                                    uint2 *s_b, float *s_x, uint32_t *s_bad, const int32_t *s_pair) {
     typedef float v4f __attribute__((ext_vector_type(4)));
     typedef float v16f __attribute__((ext_vector_type(16)));
-    constexpr int XP = 68, XN = MXM_PAIRS * XP;     // pair pitch and buffer size of s_x, in floats
+    constexpr int UB = 3 - PT;                      // blocks between barriers
+    constexpr int XP = 68, XN = MXM_PAIRS * XP;     // row pitch and buffer size of s_x, in floats
     constexpr int WP = MXM_C * 17, WN = MXM_ROWS * 17;  // row bytes and buffer size (8-byte pieces) of s_b
     constexpr int NW = 32;                          // MFMAs per block and pair group
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int nb = A.K >> 5;
-    // activations: thread t stages float4 t % 8 of the block for pairs t / 8 + 32 j
-    const int c4 = tid & 7, pr0 = tid >> 3;
+    // activations of UB blocks: thread t stages float4 t % 8 for rows t / 8 + 32 j
+    // of s_x, row 32 j + i being pair 32 j + i (PT = 2) or block j of pair i
+    const int c4 = tid & 7, pr0 = tid >> 3, nu = (nb + UB - 1) / UB;
     const float *xr[PT];
 #pragma unroll
     for (int j = 0; j < PT; j++) {
-        const int p = s_pair[pr0 + 32 * j];
+        const int p = s_pair[min(pr0 + 32 * j, np - 1)];
         xr[j] = A.x + (A.x_pair ? (int64_t)p : (int64_t)(p / A.k)) * A.ldx + 4 * c4;
     }
-    v4f xs[PT];
-    auto load_x = [&](int b) {
+    v4f xs[2];
+    auto load_x = [&](int u) {
 #pragma unroll
-        for (int j = 0; j < PT; j++) __builtin_memcpy(&xs[j], xr[j] + 32 * b, 16);
+        for (int j = 0; j < 2; j++)
+            __builtin_memcpy(&xs[j], PT == 2 ? xr[PT == 2 ? j : 0] + 32 * u : xr[0] + 32 * min(2 * u + j, nb - 1), 16);
     };
-    auto store_x = [&](int b) {
-        bool bad = false;
+    auto store_x = [&](int u) {
+        // the largest magnitude's bits, and the smallest's that is not 0, less 1
+        uint32_t hi = 0, lo = 0xFFFFFFFFu;
 #pragma unroll
-        for (int j = 0; j < PT; j++) {
-            float *r = s_x + (b & 1) * XN + (pr0 + 32 * j) * XP;
+        for (int j = 0; j < 2; j++) {
+            float *r = s_x + (u & 1) * XN + (pr0 + 32 * j) * XP;
             const v4f v = xs[j];
             *(v4f *)(r + 4 * c4) = v;
             *(v4f *)(r + 32 + 4 * c4) = v * 3.0f;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const float f = fabsf(v[i]);
-                bad |= (f < 0x1p-84f && f != 0.0f) || !(f < 0x1p80f);
+                const uint32_t f = __float_as_uint(v[i]) & 0x7FFFFFFFu;  // (a bit_cast of v[i] reads v[0])
+                hi = max(hi, f);
+                lo = min(lo, f - 1u);
             }
         }
+        const bool bad = hi >= __builtin_bit_cast(uint32_t, 0x1p80f) || lo < __builtin_bit_cast(uint32_t, 0x1p-84f) - 1u;
         const uint32_t any = __builtin_amdgcn_ballot_w64(bad) != 0 ? 1u : 0u;
-        if (lane == 0) s_bad[4 * (b & 1) + wave] = any;
+        if (lane == 0) s_bad[4 * (u & 1) + wave] = any;
     };
     // weights: piece f = 256 i + t of a chunk is row f / 17, bytes 8 (f % 17)
     constexpr int NP = (WN + 255) / 256;
@@ -637,7 +739,7 @@ __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uin
         const int j = b & (MXM_C - 1);
         const uint8_t *blk = rowb0 + ((b / MXM_C) & 1) * (WN * 8) + 17 * j;
         const float sc = mxfp4_scale(blk[16]);
-        const float *xc = s_x + (b & 1) * XN + 4 * h * XP;
+        const float *xc = s_x + ((b / UB) & 1) * XN + (32 * (b % UB) + 4 * h) * XP;
 #pragma unroll 1
         for (int e = 0; e < 32; e++) {
             const uint32_t byte = blk[e >> 1];
@@ -653,39 +755,56 @@ __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uin
     load_x(0);
     store_w(0);
     store_x(0);
-    load_x(min(1, nb - 1));
-    float wcur[NW];
-    bool odd = false;
+    load_x(min(1, nu - 1));
+    float wa[NW], wb[NW];
     const float *xb0 = s_x + n * XP + 32 * h;
-    for (int b = 0; b < nb; b++) {
-        __syncthreads();  // block b is in LDS; block b - 1's reads are done
-        if (b + 1 < nb) store_x(b + 1);
-        if (b + 2 < nb) load_x(b + 2);
-        // the next weight chunk, one block before the decode ahead reads it
-        const int c = b / MXM_C, j = b & (MXM_C - 1);
-        if (MXM_C * (c + 1) < nb) {
-            if (j == 1) load_w(c + 1);
-            if (j == MXM_C - 2) store_w(c + 1);
-        }
-        if (b == 0) odd = __builtin_amdgcn_ballot_w64(decode(0, wcur)) != 0;
-        const uint4 b4 = *(const uint4 *)(s_bad + 4 * (b & 1));
-        const uint32_t xbad = __builtin_amdgcn_readfirstlane(b4.x | b4.y | b4.z | b4.w);
-        if (odd || xbad != 0) {
+    __syncthreads();  // the first chunk is in LDS
+    bool odd = __builtin_amdgcn_ballot_w64(decode(0, wa)) != 0;
+    v4f xv[NW / 4][2];
+    // block b, its weights in cur, its activations in xv; the next block's
+    // weights go to nxt, decoded while the MFMAs run
+    auto block = [&](int b, auto half, bool slow, const float (&cur)[NW], float (&nxt)[NW]) {
+        constexpr int O = decltype(half)::value;  // b % 2
+        bool bad;
+        if (slow) {
             slow_block(b);
+            bad = decode(min(b + 1, nb - 1), nxt);
         } else {
-            const float *xc = xb0 + (b & 1) * XN;
-            v4f xv[NW / 4][PT];
-#pragma unroll
-            for (int q = 0; q < NW / 4; q++)
-#pragma unroll
-                for (int g = 0; g < PT; g++) xv[q][g] = *(const v4f *)(xc + 32 * g * XP + 4 * q);
+            bad = decode(min(b + 1, nb - 1), nxt);
 #pragma unroll
             for (int i = 0; i < NW; i++)
 #pragma unroll
                 for (int g = 0; g < PT; g++)
-                    acc[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[i >> 2][g][i & 3], wcur[i], acc[g], 0, 0, 0);
+                    acc[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[i >> 2][PT == 2 ? g : O][i & 3], cur[i], acc[g],
+                                                                  0, 0, 0);
         }
-        odd = __builtin_amdgcn_ballot_w64(decode(min(b + 1, nb - 1), wcur)) != 0;
+        odd = __builtin_amdgcn_ballot_w64(bad) != 0;
+    };
+    // unit u of UB blocks: returns whether its activations need the element path
+    auto enter = [&](int u) -> bool {
+        __syncthreads();  // unit u is in LDS; unit u - 1's reads are done
+        if (u + 1 < nu) store_x(u + 1);
+        if (u + 2 < nu) load_x(u + 2);
+        // the next weight chunk, one barrier before the decode ahead reads it
+        const int c = UB * u / MXM_C, j = UB * u & (MXM_C - 1);
+        if (MXM_C * (c + 1) < nb) {
+            if (j == UB) load_w(c + 1);
+            if (j == MXM_C - 2 * UB) store_w(c + 1);
+        }
+        const float *xc = xb0 + (u & 1) * XN;
+#pragma unroll
+        for (int q = 0; q < NW / 4; q++)
+#pragma unroll
+            for (int g = 0; g < 2; g++) xv[q][g] = *(const v4f *)(xc + 32 * g * XP + 4 * q);
+        const uint4 b4 = *(const uint4 *)(s_bad + 4 * (u & 1));
+        return __builtin_amdgcn_readfirstlane(b4.x | b4.y | b4.z | b4.w) != 0;
+    };
+    for (int b = 0; b < nb; b += 2) {
+        bool xbad = enter(b / UB);
+        block(b, std::integral_constant<int, 0>(), odd || xbad, wa, wb);
+        if (b + 1 >= nb) break;
+        if (UB == 1) xbad = enter(b + 1);
+        block(b + 1, std::integral_constant<int, 1>(), odd || xbad, wb, wa);
     }
     const int row = row0 + 32 * wave + n;
     if (row >= A.rows) return;
@@ -698,18 +817,26 @@ __device__ __forceinline__ void mxfp4_experts_tile(const MxExpArgs &A, const uin
         }
 }
 
+// lists null: every workgroup finds its own pairs (own_pair_tile).
 __global__ __launch_bounds__(256, 2) void gemm_mxfp4_experts_kernel(MxExpArgs A, const int32_t *lists,
                                                                     const int32_t *counts, const int32_t *tiles,
                                                                     int cap) {
     __shared__ __align__(16) uint2 s_b[2 * MXM_ROWS * 17];
     __shared__ __align__(16) float s_x[2 * MXM_PAIRS * 68];
     __shared__ __align__(16) uint32_t s_bad[8];
-    __shared__ int32_t s_pair[MXM_PAIRS];
+    __shared__ int32_t s_pair[MXM_PAIRS], s_cnt[4][64];
     const int mat = blockIdx.z;
-    if ((int)blockIdx.y >= tiles[0]) return;  // uniform
-    const int tile = tiles[1 + blockIdx.y], e = tile & 0xFF;
-    const int p0 = (tile >> 8) * MXM_PAIRS, np = min(MXM_PAIRS, counts[e] - p0);
-    if (threadIdx.x < MXM_PAIRS) s_pair[threadIdx.x] = lists[(size_t)e * cap + p0 + min((int)threadIdx.x, np - 1)];
+    int e, np;
+    if (lists) {
+        if ((int)blockIdx.y >= tiles[0]) return;  // uniform
+        const int tile = tiles[1 + blockIdx.y], p0 = (tile >> 8) * MXM_PAIRS;
+        e = tile & 0xFF;
+        np = min(MXM_PAIRS, counts[e] - p0);
+        if ((int)threadIdx.x < np) s_pair[threadIdx.x] = lists[(size_t)e * cap + p0 + threadIdx.x];
+    } else {
+        np = own_pair_tile(A.sel, A.n_pairs, A.n_exp, blockIdx.y, s_cnt, s_pair, e);
+        if (np == 0) return;  // uniform
+    }
     __syncthreads();
     const uint8_t *w = A.w[mat] + (int64_t)e * A.exp_stride;
     float *y = A.y[mat];

@@ -2934,11 +2934,10 @@ static int r_prefill_moe_alloc() {
     return 1;
 }
 
-// The expert product of the batched gpt-oss prefill on the matrix cores (the
-// pair lists first): the reference's serial row sums
-// (gemm_mxfp4_experts_kernel, bit-exact; the default) or, when
-// rusty_hip_set_expert_mfma(1) chose it, sums of unrounded products
-// (gemm_mxfp4_experts_mfma_kernel).  lists/counts/tiles: the list
+// The expert product of the batched gpt-oss prefill on the matrix cores: the
+// reference's serial row sums (gemm_mxfp4_experts_kernel, bit-exact; the
+// default) or, when rusty_hip_set_expert_mfma(1) chose it, sums of unrounded
+// products (gemm_mxfp4_experts_mfma_kernel).  lists/counts/tiles: the list
 // buffers; with lists_ready the lists of this sel are already built.
 static int g_expert_mfma = -1;
 static bool expert_mfma_on() {
@@ -2954,29 +2953,35 @@ static int experts_enqueue(MxExpArgs A, int n_mats, bool mfma, int32_t *lists, i
         return 0;
     // every expert's list holds at most MXE_MAX_PAIRS pairs
     if (A.n_pairs > MXE_MAX_PAIRS * A.k || A.row_stride % 16 != 0) return 0;
-    // (the opt-in product refuses activations off 16-byte rows, as it always has)
+    // (the opt-in product loads activations as 16-byte pieces)
     if (mfma && (A.ldx % 4 != 0 || ((uintptr_t)A.x & 15) != 0)) return 0;
     const int per_tile = mfma ? MXO_PAIRS : MXM_PAIRS;
-    if (!lists_ready) {
+    // at most floor(n_pairs / per_tile) full pair tiles and one partial tile per expert
+    const unsigned n_tiles = (unsigned)(A.n_pairs / per_tile + std::min(A.n_exp, A.n_pairs));
+    const dim3 grid((unsigned)((A.rows + MXM_ROWS - 1) / MXM_ROWS), n_tiles, (unsigned)n_mats);
+    // Up to 1024 pairs the serial product's workgroups find their own pairs: a
+    // list launch took 2.5 us more of a 20 us call (6 to 256 pairs, 96 columns), 3
+    // of 130 (2880 columns), and nothing less at 1000 pairs of 2880 x 2880 (500
+    // either way).
+    const bool own = !mfma && A.n_pairs <= MXE_OWN_PAIRS;
+    if (!own && !lists_ready) {
         ProfScope ps("moe_expert_lists", s);
         const dim3 waves(A.n_pairs <= 256 ? 256 : 1024);
         if (mfma)
             rh_launch(moe_expert_lists_kernel<true>, dim3(1), waves, 0, s, A.sel, A.n_pairs, A.n_exp, MXE_MAX_PAIRS,
                       lists, counts, tiles);
         else
-            rh_launch(moe_expert_lists_kernel<false>, dim3(1), waves, 0, s, A.sel, A.n_pairs, A.n_exp,
-                      MXE_MAX_PAIRS, lists, counts, tiles);
+            rh_launch(moe_expert_lists_kernel<false>, dim3(1), waves, 0, s, A.sel, A.n_pairs, A.n_exp, MXE_MAX_PAIRS,
+                      lists, counts, tiles);
         RH_LAUNCH_OK();
     }
-    // at most floor(n_pairs / per_tile) full pair tiles and one partial tile per expert
-    const unsigned n_tiles = (unsigned)(A.n_pairs / per_tile + std::min(A.n_exp, A.n_pairs));
-    const dim3 grid((unsigned)((A.rows + MXM_ROWS - 1) / MXM_ROWS), n_tiles, (unsigned)n_mats);
     ProfScope ps(name, s);
+    const int32_t *from = own ? nullptr : lists;
     if (mfma)
-        rh_launch(gemm_mxfp4_experts_mfma_kernel, grid, dim3(256), 0, s, A, (const int32_t *)lists, (const int32_t *)counts,
+        rh_launch(gemm_mxfp4_experts_mfma_kernel, grid, dim3(256), 0, s, A, from, (const int32_t *)counts,
                   (const int32_t *)tiles, (int)MXE_MAX_PAIRS);
     else
-        rh_launch(gemm_mxfp4_experts_kernel, grid, dim3(256), 0, s, A, (const int32_t *)lists, (const int32_t *)counts,
+        rh_launch(gemm_mxfp4_experts_kernel, grid, dim3(256), 0, s, A, from, (const int32_t *)counts,
                   (const int32_t *)tiles, (int)MXE_MAX_PAIRS);
     RH_LAUNCH_OK();
     return 1;
@@ -3632,10 +3637,10 @@ int rusty_hip_mxfp4_experts(const uint8_t *w, int64_t row_stride, int64_t exp_st
         row_stride < (int64_t)cols / 32 * 17 || row_stride % 16 != 0 || exp_stride < (int64_t)rows * row_stride ||
         ldy < (int64_t)rows || ldx < (int64_t)cols)
         return 0;
-    static int32_t *lists[64] = {};  // per device: pair lists, counts, pair tiles
+    static int32_t *lists[64] = {};  // per device: the opt-in product's pair lists, counts and tiles
     if (g.dev < 0 || g.dev >= 64) return 0;
     int32_t *&L = lists[g.dev];
-    if (!L && hipMalloc((void **)&L, ((size_t)64 * MXE_MAX_PAIRS + 64 + 1 + MXE_MAX_TILES) * 4) != hipSuccess) {
+    if (mfma && !L && hipMalloc((void **)&L, ((size_t)64 * MXE_MAX_PAIRS + 64 + 1 + MXE_MAX_TILES) * 4) != hipSuccess) {
         L = nullptr;
         return 0;
     }
@@ -3656,7 +3661,7 @@ int rusty_hip_mxfp4_experts(const uint8_t *w, int64_t row_stride, int64_t exp_st
     A.sel = sel;
     A.n_exp = (int32_t)n_exp;
     RH_CHECK(hipDeviceSynchronize());  // the caller's writes of w, x and sel are complete
-    int32_t *lp = L, *cp = L + (size_t)64 * MXE_MAX_PAIRS, *tp = cp + 64;
+    int32_t *lp = L, *cp = L ? L + (size_t)64 * MXE_MAX_PAIRS : nullptr, *tp = cp ? cp + 64 : nullptr;
     if (!experts_enqueue(A, 1, mfma != 0, lp, cp, tp, false, mfma ? "mxfp4_experts_mfma" : "mxfp4_experts", g.s))
         return 0;
     RH_CHECK(hipStreamSynchronize(g.s));

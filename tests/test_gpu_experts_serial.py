@@ -1,11 +1,11 @@
 """The serial (reference-order) routed expert product at the edges of its
 tiles and of the range its matrix-core form covers.
 
-The kernel works in tiles of 64 rows and up to 64 pairs (in groups of 16),
-chunks of 2 activation and 16 weight blocks; blocks whose activations are
-outside [2^-60, 2^60) or whose scale bytes are outside [87, 167] take an
-element-by-element path.  Every output is the oracle's dot_mxfp4_f32_scalar
-sum, bit for bit (NaN where it is NaN)."""
+The kernel works in tiles of 128 rows and up to 64 pairs (two groups of 32, or
+one group two blocks at a time), with the weights of 8 blocks in LDS; blocks
+with an activation outside 0 or [2^-84, 2^80) or a scale byte outside
+[87, 167] take an element-by-element path.  Every output is the oracle's
+dot_mxfp4_f32_scalar sum, bit for bit (NaN where it is NaN)."""
 import numpy as np
 import pytest
 
@@ -87,4 +87,75 @@ def test_values_outside_the_matrix_core_range(hip, kind):
     if kind in ("nonfinite", "mixed"):
         x[2, 40], x[5, 3], x[9, 100] = np.inf, -np.inf, np.nan
     got = _run(hip, w, stride, n_exp, rows, cols, x, True, 1, sel)
+    _check(got, w, rb, rows, cols, x, True, 1, sel, n_exp)
+
+
+def _weights(n_exp, rows, cols, rng, scale):
+    """Random nibbles (every weight, -0 among them), one scale byte."""
+    rb = synth.row_bytes(MX, cols)
+    stride = (rb + 15) // 16 * 16
+    w = np.zeros((n_exp, rows, stride), np.uint8)
+    w[:, :, :rb] = rng.integers(0, 256, (n_exp, rows, rb))
+    w[:, :, 16:rb:17] = scale
+    return w, rb, stride
+
+
+@pytest.mark.parametrize("rows,cols,n_pairs", [(127, 256, 3), (128, 288, 33), (129, 544, 40)])
+@pytest.mark.parametrize("xe,scale", [
+    (-84, 87), (-84, 167), (79, 87), (79, 167),  # every block on the matrix cores, at the edges of their range
+    (-86, 87), (-84, 85), (-100, 127),           # every block outside: products below the normal range would differ
+    (86, 167), (79, 174), (100, 150),            # ... and sums past the largest number
+])
+def test_edges_of_the_matrix_core_range(hip, rows, cols, n_pairs, xe, scale):
+    rng = np.random.default_rng(rows + xe + scale)
+    w, rb, stride = _weights(2, rows, cols, rng, scale)
+    sel = rng.integers(0, 2, n_pairs).astype(np.int32)
+    # full mantissas in [2^xe, 2^(xe + 1)), either sign
+    mant = rng.integers(0, 1 << 23, (n_pairs, cols), dtype=np.uint32)
+    x = (mant | np.uint32((xe + 127) << 23) | (rng.integers(0, 2, mant.shape, dtype=np.uint32) << 31)).view(np.float32)
+    x[:, :32] = np.where(rng.random((n_pairs, 32)) < 0.2, np.float32(0), x[:, :32])
+    _check(_run(hip, w, stride, 2, rows, cols, x, True, 1, sel), w, rb, rows, cols, x, True, 1, sel, 2)
+
+
+@pytest.mark.parametrize("what", ["x below", "x above", "scale below", "scale above", "last block"])
+def test_one_value_outside_the_matrix_core_range(hip, what):
+    """One block of one pair or row on the element path, its neighbours not."""
+    rows, cols, n_pairs = 130, 32 * 17, 37
+    rng = np.random.default_rng(len(what))
+    w, rb, stride = _weights(1, rows, cols, rng, 87 if "below" in what else 160)
+    x = (synth.normal_f32(5, n_pairs, cols) * np.float32(2.0 ** (-82 if "below" in what else 70))).reshape(n_pairs, cols)
+    x[np.abs(x) < 2.0 ** -84] = 0.0
+    if what == "x below":
+        x[3, 32 * 9 + 5] = np.float32(1.9 * 2.0 ** -90)
+    elif what == "x above":
+        x[36, 32 * 8] = np.float32(1.3 * 2.0 ** 88)
+    elif what == "last block":
+        x[0, cols - 1] = np.inf
+    else:
+        w[0, 129, 17 * 7 + 16] = 80 if what == "scale below" else 180
+    sel = np.zeros(n_pairs, np.int32)
+    _check(_run(hip, w, stride, 1, rows, cols, x, True, 1, sel), w, rb, rows, cols, x, True, 1, sel, 1)
+
+
+@pytest.mark.parametrize("n_pairs,kind", [(800, "spread"), (1024, "spread"), (1024, "one expert"), (1000, "half unrouted"),
+                                          (257, "spread"), (65, "spread"), (64, "one expert"), (1, "one expert")])
+def test_pairs_found_in_the_workgroups(hip, n_pairs, kind):
+    """Up to 1024 pairs the product is one launch (a list launch before it had
+    made calls of few pairs slower than without)."""
+    rows, n_exp, cols = 33, 64, 32
+    rng = np.random.default_rng(n_pairs)
+    w, rb, stride = _weights(n_exp, rows, cols, rng, 120)
+    sel = rng.integers(0, n_exp, n_pairs).astype(np.int32)
+    if kind == "one expert":
+        sel[:] = n_exp - 1
+    if kind == "half unrouted":
+        sel[::2] = rng.choice([-1, -2, n_exp, 1 << 30], sel[::2].shape)
+    x = synth.normal_f32(3, n_pairs, cols).reshape(n_pairs, cols)
+    hip.profile_enable(True)
+    try:
+        got = _run(hip, w, stride, n_exp, rows, cols, x, True, 1, sel)
+        launches = {name: n for name, (_, n) in hip.profile_results().items() if n}
+    finally:
+        hip.profile_enable(False)
+    assert launches == {"mxfp4_experts": 1}
     _check(got, w, rb, rows, cols, x, True, 1, sel, n_exp)
