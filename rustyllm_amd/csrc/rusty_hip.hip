@@ -130,6 +130,7 @@ struct Ctx {
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
 };
 static Ctx g;
+static size_t g_alloc_limit = 0;  // rusty_hip_debug_alloc_limit
 
 static int64_t row_bytes_of(int fmt, int64_t cols) {
     switch (fmt) {
@@ -2251,7 +2252,8 @@ struct Resident {
     uint32_t n_exp = 0, top_k = 0, window = 0;
     float rope_conc = 1.0f;
     float *moebuf = nullptr;
-    // batched prefill, allocated on first use for pf_cap tokens per chunk
+    // batched prefill, allocated by the prompts that need them for pf_cap tokens
+    // per chunk
     uint32_t pf_cap = 0;
     float *px = nullptr, *pq = nullptr, *pk = nullptr, *pv = nullptr, *pattn = nullptr, *ptg = nullptr,
           *ptu = nullptr, *pex = nullptr;
@@ -2263,6 +2265,8 @@ struct Resident {
     int32_t *psel = nullptr;
     // the expert product's per-expert pair lists, counts and pair tiles
     int32_t *plists = nullptr, *pcounts = nullptr, *ptiles = nullptr;
+    uint32_t pf_limit = 0;          // most tokens per chunk once a larger chunk's buffers did not fit
+    std::vector<void *> pf_allocs;  // the batched-prefill buffers
     std::map<std::pair<int, uint32_t>, hipGraphExec_t> graphs;  // by (mode, penalty bits)
     std::vector<void *> allocs;
     std::vector<std::pair<const void *, DevW>> wown;  // weight copies owned by the decoder
@@ -2275,6 +2279,23 @@ static int r_alloc(void **p, size_t bytes) {
     RH_CHECK(hipMalloc(p, bytes));
     R.allocs.push_back(*p);
     return 1;
+}
+
+// Buffers of the batched prefill: a failure leaves no error behind for the next
+// launch check, and pf_free gives back what came before it.
+static int pf_alloc(void **p, size_t bytes) {
+    if ((g_alloc_limit && bytes > g_alloc_limit) || hipMalloc(p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+        return 0;
+    }
+    R.pf_allocs.push_back(*p);
+    return 1;
+}
+static void pf_free() {
+    for (void *p : R.pf_allocs) (void)hipFree(p);
+    R.pf_allocs.clear();
+    R.pf_cap = 0;
 }
 
 // The resident decoder's own device copy of a weight, freed only by the next
@@ -2300,6 +2321,8 @@ static void r_reset() {
     R.graphs.clear();
     for (void *p : R.allocs) (void)hipFree(p);
     R.allocs.clear();
+    pf_free();
+    R.pf_limit = 0;
     R.wown.clear();
     if (R.st_host) (void)hipHostFree(R.st_host);
     R.st_host = nullptr;
@@ -2312,8 +2335,6 @@ static void r_reset() {
     R.n_exp = R.top_k = R.window = 0;
     R.rope_conc = 1.0f;
     R.moebuf = nullptr;
-    R.pf_cap = 0;
-    R.pxn = nullptr;  // with the other batched-prefill buffers, freed through allocs
 }
 
 static void r_invalidate_graphs() {
@@ -2740,17 +2761,18 @@ static int r_run(int mode, float penalty) {
 // tokens one by one.
 // Tokens per chunk: RUSTY_HIP_PREFILL_CHUNK (64..2048), else 512 (a sweep
 // over 256/512/1024 on a 2048-token prompt put 512 first, by 2-4%).  A gpt-oss
-// chunk is 1024 tokens where its attention scratch (moe_scratch bytes per
-// token; 0 for other models) stays within 8 GB: the experts' 64-pair tiles
-// fill up (32 experts, top 4: 128 pairs per expert instead of 64).
-static int pf_chunk(size_t moe_scratch) {
+// prompt of more than 512 tokens takes 1024 where the attention scratch
+// (moe_scratch bytes per token; 0 for other models) stays within 8 GB: the
+// experts' 64-pair tiles fill up (32 experts, top 4: 128 pairs per expert
+// instead of 64).
+static int pf_chunk(size_t moe_scratch, int n) {
     static int v = -1;
     if (v < 0) {
         const char *e = getenv("RUSTY_HIP_PREFILL_CHUNK");
         v = e ? std::max(64, std::min(2048, atoi(e))) : 0;
     }
     if (v) return v;
-    return moe_scratch && moe_scratch * 1024 <= ((size_t)8 << 30) ? 1024 : 512;
+    return n > 512 && moe_scratch && moe_scratch * 1024 <= ((size_t)8 << 30) ? 1024 : 512;
 }
 
 static bool r_prefill_enabled() {
@@ -2773,21 +2795,34 @@ static bool r_prefill_batchable() {
     return true;
 }
 
-static int r_prefill_alloc() {
-    if (R.pf_cap) return 1;
+static int r_prefill_moe_alloc(size_t C);
+
+// The buffers of a prompt of n tokens, grown when a longer prompt takes a
+// larger chunk.  Where the larger chunk's do not fit, 512 tokens are tried
+// again and stay the limit until the next configure.
+static int r_prefill_alloc(int n) {
     const size_t ex = exact_scratch_floats((int)R.n_kv, (int)(R.n_heads / R.n_kv), R.ex_cap);
-    const size_t C = (size_t)pf_chunk(R.moe ? ex * 4 : 0);
     const size_t qd = (size_t)R.n_heads * R.hd, kd = (size_t)R.n_kv * R.hd, vdim = (size_t)R.n_kv * R.vd;
     const size_t attn_cols = (size_t)R.n_heads * R.vd;
     const size_t kmax = std::max<size_t>(std::max<size_t>(R.dim, attn_cols), R.hidden);
-    if (!r_alloc((void **)&R.px, C * R.dim * 4) || !r_alloc((void **)&R.pq, C * qd * 4) ||
-        !r_alloc((void **)&R.pk, C * kd * 4) || !r_alloc((void **)&R.pv, C * vdim * 4) ||
-        !r_alloc((void **)&R.pattn, C * attn_cols * 4) || !r_alloc((void **)&R.ptg, C * R.hidden * 4) ||
-        !r_alloc((void **)&R.ptu, C * R.hidden * 4) || !r_alloc((void **)&R.pex, C * ex * 4) ||
-        !r_alloc((void **)&R.pbq, batch_xq_bytes((int)C, (int)kmax)))
-        return 0;
-    R.pf_cap = (uint32_t)C;
-    return 1;
+    size_t C = (size_t)pf_chunk(R.moe ? ex * 4 : 0, n);
+    if (R.pf_limit) C = std::min<size_t>(C, R.pf_limit);
+    if (R.pf_cap >= C) return 1;
+    if (!R.pf_allocs.empty()) RH_CHECK(hipStreamSynchronize(g.s));  // no earlier chunk still reads them
+    for (;;) {
+        pf_free();
+        if (pf_alloc((void **)&R.px, C * R.dim * 4) && pf_alloc((void **)&R.pq, C * qd * 4) &&
+            pf_alloc((void **)&R.pk, C * kd * 4) && pf_alloc((void **)&R.pv, C * vdim * 4) &&
+            pf_alloc((void **)&R.pattn, C * attn_cols * 4) && pf_alloc((void **)&R.ptg, C * R.hidden * 4) &&
+            pf_alloc((void **)&R.ptu, C * R.hidden * 4) && pf_alloc((void **)&R.pex, C * ex * 4) &&
+            pf_alloc((void **)&R.pbq, batch_xq_bytes((int)C, (int)kmax)) && (!R.moe || r_prefill_moe_alloc(C))) {
+            R.pf_cap = (uint32_t)C;
+            return 1;
+        }
+        pf_free();
+        if (C <= 512) return 0;
+        C = R.pf_limit = 512;
+    }
 }
 
 static int r_rmsnorm_batch(const float *norm_w, int T, const BatchXq &b, hipStream_t s) {
@@ -2919,19 +2954,15 @@ static bool r_prefill_moe_batchable() {
     return true;
 }
 
-static int r_prefill_moe_alloc() {
-    if (R.pxn) return 1;
-    if (!r_prefill_alloc()) return 0;
-    const size_t C = R.pf_cap, k = R.top_k, kd = (size_t)R.n_kv * R.hd, vdim = (size_t)R.n_kv * R.vd;
+static int r_prefill_moe_alloc(size_t C) {
+    const size_t k = R.top_k, kd = (size_t)R.n_kv * R.hd, vdim = (size_t)R.n_kv * R.vd;
     const size_t hid = R.L.empty() ? 0 : (size_t)R.L[0].moe.hidden, rows = R.storage + C;
-    if (!r_alloc((void **)&R.plk, rows * kd * 4) || !r_alloc((void **)&R.plv, rows * vdim * 4) ||
-        !r_alloc((void **)&R.plog, C * 64 * 4) || !r_alloc((void **)&R.psel, C * k * 4) ||
-        !r_alloc((void **)&R.pprob, C * k * 4) || !r_alloc((void **)&R.pgate, C * k * hid * 4) ||
-        !r_alloc((void **)&R.pup, C * k * hid * 4) || !r_alloc((void **)&R.pproj, C * k * R.dim * 4) ||
-        !r_alloc((void **)&R.pxn, C * R.dim * 4) || !r_alloc((void **)&R.plists, (size_t)64 * MXE_MAX_PAIRS * 4) ||
-        !r_alloc((void **)&R.pcounts, 64 * 4) || !r_alloc((void **)&R.ptiles, (1 + MXE_MAX_TILES) * 4))
-        return 0;
-    return 1;
+    return pf_alloc((void **)&R.plk, rows * kd * 4) && pf_alloc((void **)&R.plv, rows * vdim * 4) &&
+           pf_alloc((void **)&R.plog, C * 64 * 4) && pf_alloc((void **)&R.psel, C * k * 4) &&
+           pf_alloc((void **)&R.pprob, C * k * 4) && pf_alloc((void **)&R.pgate, C * k * hid * 4) &&
+           pf_alloc((void **)&R.pup, C * k * hid * 4) && pf_alloc((void **)&R.pproj, C * k * R.dim * 4) &&
+           pf_alloc((void **)&R.pxn, C * R.dim * 4) && pf_alloc((void **)&R.plists, (size_t)64 * MXE_MAX_PAIRS * 4) &&
+           pf_alloc((void **)&R.pcounts, 64 * 4) && pf_alloc((void **)&R.ptiles, (1 + MXE_MAX_TILES) * 4);
 }
 
 // The expert product of the batched gpt-oss prefill on the matrix cores: the
@@ -3265,14 +3296,13 @@ static int r_prefill_chunk_moe(const int32_t *tok, int T, int pos0, hipStream_t 
 
 // n tokens already in R.tokens[0..n) at positions pos0.. in chunks.
 static int r_prefill_tokens(int n, int pos0) {
+    if (!r_prefill_alloc(n)) return 0;
     if (R.moe) {
-        if (!r_prefill_moe_alloc()) return 0;
         const int cap = std::min<int>((int)R.pf_cap, MXE_MAX_PAIRS);  // the experts' pair lists hold one chunk
         for (int c = 0; c < n; c += cap)
             if (!r_prefill_chunk_moe(R.tokens + c, std::min<int>(cap, n - c), pos0 + c, g.s)) return 0;
         return 1;
     }
-    if (!r_prefill_alloc()) return 0;
     for (int c = 0; c < n; c += (int)R.pf_cap)
         if (!r_prefill_chunk(R.tokens + c, std::min<int>((int)R.pf_cap, n - c), pos0 + c, g.s)) return 0;
     return 1;
@@ -3703,6 +3733,15 @@ int rusty_hip_resident_time_decode(uint32_t n_tokens, float penalty, double *ms)
     *ms = t;
     prof_drain();
     return r_stream_ok();
+}
+
+// Test hook for allocations that fail: those of the batched prefill's buffers
+// that are larger than `bytes` do (0: none), as if memory had run out.
+int rusty_hip_debug_alloc_limit(uint64_t bytes) {
+    std::lock_guard<std::mutex> lk(g.mu);
+    if (!init_locked()) return 0;
+    g_alloc_limit = (size_t)bytes;
+    return 1;
 }
 
 // Test hook for the streamed attention's timeout path: marks the next

@@ -35,6 +35,7 @@ SYMBOLS = [
     "rusty_hip_kquant_matvec_batch", "rusty_hip_resident_prefill", "rusty_hip_bench_matvec",
     "rusty_hip_bench_attention", "rusty_hip_attention_noalloc", "rusty_hip_gguf_summary",
     "rusty_hip_resident_load_gguf", "rusty_hip_resident_enable_bf16", "rusty_hip_debug_stream_mark",
+    "rusty_hip_debug_alloc_limit",
     "rusty_hip_set_expert_mfma", "rusty_hip_mxfp4_experts",
 ]
 
@@ -93,6 +94,7 @@ _sig("rusty_hip_debug_rope", _i, _p, _p, _u32, _u32, _u32, _u32, _p, _u32)
 _sig("rusty_hip_debug_greedy", _i, _p, _u, _p, _u32, _f, _p)
 _sig("rusty_hip_debug_f16", _i, _p, _u, _p)
 _sig("rusty_hip_debug_stream_mark", _i)
+_sig("rusty_hip_debug_alloc_limit", _i, C.c_uint64)
 _sig("rusty_hip_set_expert_mfma", _i, _i)
 _sig("rusty_hip_mxfp4_experts", _i, _p, _i64, _i64, _u32, _u32, _u32, _p, _i64, _i, _u32, _p, _u32, _p, _i64, _i)
 _sig("rusty_hip_resident_configure_moe", _i, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _f,
@@ -638,6 +640,12 @@ def debug_stream_mark() -> bool:
     """Marks the resident decoder's next streamed attention launch as timed
     out (the failure path's test hook)."""
     return lib.rusty_hip_debug_stream_mark() == 1
+
+
+def debug_alloc_limit(n_bytes: int) -> bool:
+    """Makes the batched prefill's allocations above n_bytes fail (0: none), a
+    test hook."""
+    return lib.rusty_hip_debug_alloc_limit(n_bytes) == 1
 
 
 def set_expert_mfma(on: bool) -> bool:
