@@ -404,8 +404,9 @@ int rusty_hip_debug_expf(const float *x, uintptr_t n, float *out);
  * ends normally with invalid values, and the decode call that ran it returns
  * 0.  Test hook for that failure path; 0 when no streamed launch exists. */
 int rusty_hip_debug_stream_mark(void);
-/* Lets every allocation of the batched prefill's buffers above `bytes` fail as
- * if memory had run out (0: none does).  Test hook for that failure path. */
+/* Lets every allocation of the batched prefill's buffers and of the per-op
+ * calls' pinned memory above `bytes` fail as if memory had run out (0: none
+ * does).  Test hook for those failure paths. */
 int rusty_hip_debug_alloc_limit(uint64_t bytes);
 
 #ifdef __cplusplus

@@ -1301,18 +1301,21 @@ static int gemm_kq_enqueue(const DevW &W, const BatchXq &b, int T, float *y, int
 // memory that the kernels address themselves: the quantizer reads x there (or
 // one launch copies it to the device), and the last launch of a call writes the
 // outputs there.  The runtime's copies of pageable memory took 13 of the 38 us
-// of a 256 x 2048 matvec call, and 9 of the 134 of a 128256-row product.  A counter that the last launch writes for the host to
-// watch, in place of the stream synchronisation, measured the same in a row of
-// calls and 7 us slower alone.
+// of a 256 x 2048 matvec call, and 9 of the 134 of a 128256-row product.  A
+// counter that the last launch writes for the host to watch, in place of the
+// stream synchronisation, measured the same in a row of calls and 7 us slower
+// alone.
 #define RH_IO_FLOATS ((size_t)1 << 20)
 static bool io_ready() {
-    if (!g.io_in && hipHostMalloc((void **)&g.io_in, RH_IO_FLOATS * 4, hipHostMallocDefault) != hipSuccess) {
-        g.io_in = nullptr;
-        return false;
-    }
-    if (!g.io_out && hipHostMalloc((void **)&g.io_out, RH_IO_FLOATS * 4, hipHostMallocDefault) != hipSuccess) {
-        g.io_out = nullptr;
-        return false;
+    for (float **p : {&g.io_in, &g.io_out}) {
+        if (*p) continue;
+        // (every device of the process reads and writes it)
+        if ((g_alloc_limit && RH_IO_FLOATS * 4 > g_alloc_limit) ||
+            hipHostMalloc((void **)p, RH_IO_FLOATS * 4, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();  // the call goes on without: leave no error for its launch checks
+            *p = nullptr;
+            return false;
+        }
     }
     return true;
 }
@@ -3735,12 +3738,19 @@ int rusty_hip_resident_time_decode(uint32_t n_tokens, float penalty, double *ms)
     return r_stream_ok();
 }
 
-// Test hook for allocations that fail: those of the batched prefill's buffers
-// that are larger than `bytes` do (0: none), as if memory had run out.
+// Test hook for allocations that fail: those of the batched prefill's buffers and
+// of the per-op exports' pinned memory that are larger than `bytes` do (0: none),
+// as if memory had run out.  Pinned memory beyond it is given back.
 int rusty_hip_debug_alloc_limit(uint64_t bytes) {
     std::lock_guard<std::mutex> lk(g.mu);
     if (!init_locked()) return 0;
     g_alloc_limit = (size_t)bytes;
+    if (bytes && bytes < RH_IO_FLOATS * 4) {
+        RH_CHECK(hipStreamSynchronize(g.s));
+        if (g.io_in) (void)hipHostFree(g.io_in);
+        if (g.io_out) (void)hipHostFree(g.io_out);
+        g.io_in = g.io_out = nullptr;
+    }
     return 1;
 }
 

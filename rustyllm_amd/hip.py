@@ -643,8 +643,8 @@ def debug_stream_mark() -> bool:
 
 
 def debug_alloc_limit(n_bytes: int) -> bool:
-    """Makes the batched prefill's allocations above n_bytes fail (0: none), a
-    test hook."""
+    """Makes the prefill's and the pinned allocations above n_bytes fail (0:
+    none), a test hook."""
     return lib.rusty_hip_debug_alloc_limit(n_bytes) == 1
 
 

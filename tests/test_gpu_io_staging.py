@@ -51,3 +51,31 @@ def test_weight_change_at_one_address_is_seen(hip):
         w[byte] ^= 0x80 if byte != w.size - 1 else 1
         assert hip.matvec_into(8, w, x, 16, 64, out)
         assert np.array_equal(out, O.matvec(8, w, x, 16, 64), equal_nan=True), byte
+
+
+def test_without_pinned_memory(hip):
+    """Where the pinned buffers cannot be had, the same calls go by the
+    runtime's copies, and with them again afterwards."""
+    cols, rows = 512, (300, 40, 7)
+    ws = [(synth.normal_quantized(t, r, r, cols, 0.05), t, r) for t, r in zip((12, 12, 14), rows)]
+    xs = synth.normal_f32(6, 40, cols)
+    refs = [O.matvec(t, w, xs[0], r, cols) for w, t, r in ws]
+    dim, hidden = 256, 512
+    f = [synth.normal_quantized(t, 9 + i, r, c, 0.05) for i, (t, r, c) in
+         enumerate(((12, hidden, dim), (12, hidden, dim), (14, dim, hidden)))]
+    blocks = []
+    try:
+        for n in (1024, 0):
+            assert hip.debug_alloc_limit(n)
+            outs = [np.zeros(r, np.float32) for r in rows]
+            assert hip.quant_matvec3_into(*ws, xs[0], cols, outs)
+            batch = np.zeros((40, rows[0]), np.float32)
+            assert hip.kquant_matvec_batch_into(12, ws[0][0], rows[0], cols, xs, batch)
+            block = np.zeros(dim, np.float32)
+            assert hip.q4k_q4k_q6k_ffn_into(*f, xs[1, :dim], dim, hidden, dim, hidden, block)
+            blocks.append(block)
+            for got, ref in zip(outs + [batch[0]], refs + [refs[0]]):
+                assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+        assert np.array_equal(blocks[0].view(np.uint32), blocks[1].view(np.uint32)) and np.any(blocks[0])
+    finally:
+        hip.debug_alloc_limit(0)
