@@ -3021,18 +3021,23 @@ static int experts_enqueue(MxExpArgs A, int n_mats, bool mfma, int32_t *lists, i
     return 1;
 }
 
-// Whether a Q8_0 batch of n matrices (tiles 64-row tiles in all) goes to the
-// matrix-core kernels.  Their shortest launch takes K's whole loop, 75 us with
-// f32 activations (K = 2880) and 104 with int8 ones (K = 4096); the per-row
-// kernel's take about 24 us per launch plus 0.033 us per tile and token (f32),
-// or 45 plus 0.02 (int8).  Measured, matrix cores against per-row kernel, us:
-// q/k/v in one launch against three (80 tiles): 4 tokens 74 : 77, 33 tokens
-// 77 : 148, 1001 tokens 300 : 2253; router (1 tile) 1001 tokens 77 : 25; wo
-// (int8, 45 tiles): 33 tokens 106 : 63, 65 tokens 104 : 86, 129 tokens 105 :
-// 169, 1001 tokens 212 : 975.
-static bool q80_gemm_pays(int cat, int n, int64_t tiles, int64_t T) {
-    if (cat == CAT_F32) return tiles * T >= (n == 3 ? 256 : n == 2 ? 900 : 1536);
-    return tiles * T >= 3584;
+// Whether a Q8_0 batch of n matrices of K columns (tiles 64-row tiles in all)
+// goes to the matrix-core kernels.  Their shortest launch takes K's whole loop,
+// 6 us + 0.024 per column with f32 activations, 8 + 0.023 with int8 ones; the
+// per-row kernel pays per matrix, and per tile and token about 2e-5 us per column
+// (f32) or 5e-6 (int8).  Measured, matrix cores against per-row kernel, us:
+// f32, q/k/v in one launch against three (tiles x K): 24 x 1440, 16 tokens 40 :
+// 38, 33 tokens 41 : 47; 80 x 2880, 8 tokens 76 : 74, 16 tokens 77 : 84, 512
+// tokens 192 : 1189; 80 x 4320, 8 tokens 111 : 152.  One f32 matrix is only the
+// router, one tile: 512 tokens 76 : 23.
+// int8, wo: 7 x 512, 512 tokens 20 : 18; 23 x 1024, 129 tokens 32 : 24, 257 tokens
+// 32 : 39; 32 x 2048, 65 tokens 52 : 36, 129 tokens 54 : 57; 45 x 4096, 65 tokens
+// 101 : 87, 129 tokens 101 : 158.  So the int8 line falls from 4600 tiles x tokens
+// at 512 columns to 3430 at 4096.  q/k/v of int8 activations would pay at once
+// (12 x 512, 4 tokens 14 : 25; 80 x 4096 94 : 130).
+static bool q80_gemm_pays(int cat, int n, int K, int64_t tiles, int64_t T) {
+    if (cat == CAT_F32) return n == 3 && tiles * T > 640;
+    return tiles * T >= 4800 - std::min(K, 4096) / 3;
 }
 
 // y[t][r] (=, or += with EPI_ADD) Q8_0 row r of W times token t (+ bias) for
@@ -3046,7 +3051,7 @@ struct Q80Mat {
     int ldy;
 };
 static int q80_batch_enqueue(const Q80Mat *ms, int n, int K, int T, const float *x, const BatchXq *bq, int epi,
-                             const char *name, hipStream_t s) {
+                             const char *name, const char *rows_name, hipStream_t s) {
     const int cat = cat_of(8, K);
     if (n < 1 || n > 3 || T <= 0 || (cat != CAT_F32 && cat != CAT_Q8I)) return 0;
     if (cat == CAT_F32 ? (!x || K % 4 != 0) : !bq) return 0;
@@ -3075,8 +3080,9 @@ static int q80_batch_enqueue(const Q80Mat *ms, int n, int K, int T, const float 
         G.tiles[i] = tiles;
     }
     for (int i = n; i < 3; i++) G.tiles[i] = tiles;
-    ProfScope ps(name, s);
-    if (q80_gemm_pays(cat, n, tiles, T)) {
+    const bool gemm = q80_gemm_pays(cat, n, K, tiles, T);
+    ProfScope ps(gemm ? name : rows_name, s);
+    if (gemm) {
         const dim3 grid((unsigned)tiles, (unsigned)((T + 63) / 64));
         if (cat == CAT_F32)
             rh_launch(gemm_q8_0_f32_kernel, grid, dim3(256), 0, s, G);
@@ -3159,7 +3165,7 @@ static int r_prefill_chunk_moe(const int32_t *tok, int T, int pos0, hipStream_t 
         const Q80Mat qkv[3] = {{&Ly.w[0], qd, Ly.bias[0], R.pq, qd},
                                {&Ly.w[1], kd, Ly.bias[1], R.pk, kd},
                                {&Ly.w[2], vdim, Ly.bias[2], R.pv, vdim}};
-        if (!q80_batch_enqueue(qkv, 3, dim, T, R.pxn, &bd, EPI_STORE, "pf_q80_qkv", s)) return 0;
+        if (!q80_batch_enqueue(qkv, 3, dim, T, R.pxn, &bd, EPI_STORE, "pf_q80_qkv", "pf_q80_qkv_rows", s)) return 0;
         if (!kv_ring_copy(Ly, P0, npre, 0, 0, s)) return 0;
         {
             RopeArgs A;
@@ -3226,13 +3232,13 @@ static int r_prefill_chunk_moe(const int32_t *tok, int T, int pos0, hipStream_t 
         if (!kv_ring_copy(Ly, last0, pos0 + T - last0, last0 - P0, 1, s)) return 0;
         // x += wo attn + bo (src/model.rs:6837-6840)
         const Q80Mat wo = {&Ly.w[3], dim, Ly.bo, R.px, dim};
-        if (!q80_batch_enqueue(&wo, 1, attn_cols, T, nullptr, &ba, EPI_ADD, "pf_q80_o", s)) return 0;
+        if (!q80_batch_enqueue(&wo, 1, attn_cols, T, nullptr, &ba, EPI_ADD, "pf_q80_o", "pf_q80_o_rows", s)) return 0;
         // xn2 = rms_norm(x, post_attn_norm); x += moe(xn2) (src/model.rs:6846-6898)
         if (!r_norm_batch_moe(Ly.ffn_norm, T, bd, s)) return 0;
         const int k = M.k, hid = M.hidden, np = T * k;
         const bool mfma = expert_mfma_on();
         const Q80Mat router = {&M.router, M.n_exp, M.router_bias, R.plog, 64};
-        if (!q80_batch_enqueue(&router, 1, dim, T, R.pxn, &bd, EPI_STORE, "pf_router", s)) return 0;
+        if (!q80_batch_enqueue(&router, 1, dim, T, R.pxn, &bd, EPI_STORE, "pf_router", "pf_router_rows", s)) return 0;
         {
             ProfScope ps("moe_topk_batch", s);
             rh_launch(moe_topk_batch_kernel, dim3((unsigned)T), dim3(64), 0, s, (const float *)R.plog, 64, M.n_exp, k,

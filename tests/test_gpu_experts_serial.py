@@ -159,3 +159,18 @@ def test_pairs_found_in_the_workgroups(hip, n_pairs, kind):
         hip.profile_enable(False)
     assert launches == {"mxfp4_experts": 1}
     _check(got, w, rb, rows, cols, x, True, 1, sel, n_exp)
+
+
+@pytest.mark.parametrize("n_pairs", [2, 34])
+def test_every_element_of_a_block_is_checked(hip, n_pairs):
+    """One infinite activation at each place of a block: rows whose weight there
+    is not 0 get an infinite sum, not NaN."""
+    rows, cols = 40, 96
+    rng = np.random.default_rng(n_pairs)
+    w, rb, stride = _weights(1, rows, cols, rng, 125)
+    sel = np.zeros(n_pairs, np.int32)
+    base = synth.normal_f32(2, n_pairs, cols).reshape(n_pairs, cols)
+    for e in range(32):
+        x = base.copy()
+        x[n_pairs - 1, 32 * (e % 3) + e] = np.inf
+        _check(_run(hip, w, stride, 1, rows, cols, x, True, 1, sel), w, rb, rows, cols, x, True, 1, sel, 1)
