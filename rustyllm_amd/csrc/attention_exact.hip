@@ -1561,8 +1561,14 @@ __global__ __launch_bounds__(64 * C4_WAVES) void attn_exact_chain4_kernel(AttnEx
 // each for a flag (see stream_wait), and the scores workgroups never do.
 // The last workgroup to finish advances the epoch and resets the ticket for
 // the next launch.
+//
+// The code (58 KB) starts at a multiple of 64 KB: its time depends on where it
+// lies, and without that on every kernel before it.  The same instructions took
+// 33.2 us per layer of an 8B model at 4096 positions at one place and 33.9 at
+// another (16 tokens through 6 layers 9.26, 9.33 or 9.39 ms; 9.26 so aligned).
 template <int HD>
-__global__ __launch_bounds__(64 * C4_WAVES) void attn_exact_stream_kernel(AttnExactArgs A0) {
+__global__ __launch_bounds__(64 * C4_WAVES) __attribute__((aligned(65536))) void attn_exact_stream_kernel(
+    AttnExactArgs A0) {
     AttnExactArgs A = A0;
     A.ep = __hip_atomic_load(A0.sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int ns = (int)gridDim.x - chain4_blocks(A);
