@@ -403,7 +403,8 @@ def measure_prefill_gptoss(hip, res, toks, log):
     tot, cnt = prof.get("pf_mxfp4_gate_up", (0.0, 0))
     tflops = ops / (tot * 1e-3) / 1e12 if cnt else 0.0
     roofline = {"kernel": "pf_mxfp4_gate_up (%s: %d pairs x %d rows x %d, f32)"
-                % ("gemm_mxfp4_experts_kernel, " + ("unrounded products" if mfma else "serial reference-order sums"),
+                % ("gemm_mxfp4_experts_mfma_kernel, unrounded products" if mfma else
+                   "gemm_mxfp4_experts_kernel, serial reference-order sums",
                    n * cfg["top_k"], 2 * cfg["hidden_dim"], cfg["dim"]),
                 "bound": "mfma", "achieved": round(tflops, 2), "peak": FP32_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(tflops / FP32_PEAK_TFLOPS, 4),

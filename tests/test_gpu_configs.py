@@ -25,9 +25,9 @@ decode, src/model.rs:2877-2955; forward_prefill_gpt_oss per token,
 src/runtime.rs:3760-3790):
 - config 3: the 512-token prompt through the MFMA products at the 8B shape,
   KV of every layer and the next logits bit-exact;
-- config 5: the 1024-token prompt at the 20B shape in two chunks (ring
-  layers through the linear view), ring KV of every layer and the next
-  logits bit-exact, then 64 greedy tokens.
+- config 5: the 1024-token prompt at the 20B shape (ring layers through the
+  linear view), ring KV of every layer and the next logits bit-exact, then 64
+  greedy tokens.
 """
 import numpy as np
 import pytest
@@ -172,7 +172,7 @@ def test_config5_gptoss20b_past_two_windows(hip, exact):
 
 def test_config5_gptoss20b_prompt_prefill_1024(hip, exact):
     """BASELINE config 5's 1024-token prompt at the gpt-oss-20B shape through
-    the batched prefill (two chunks: 512 + 511 tokens, then the last token's
+    the batched prefill (one chunk of 1023 tokens, then the last token's
     decode step), against the reference's token-by-token prefill: the ring
     K/V of every layer and the next logits bit-identical, then the prompt
     again with 64 greedy tokens after it, identical to the oracle's decode
