@@ -125,15 +125,15 @@ __device__ __forceinline__ rh_v4i bytes_times(const rh_v4i &x, int s) {
 // weights straight after the digits are made.  One barrier per block.
 //
 // Bound by the VALU, Q4_K: 200 instructions per 32 x 32 outputs and block with
-// NT = 2 (390 with a minimum MFMA per sub-block and one token tile), about 60% busy;
-// the waits are the barrier and the start of each tile.  Gate and up of an
-// 8B-class model, 28672 x 4096, 512 tokens in one launch: 161 us (747 TOP/s);
-// two launches of the one-tile kernel before, 244.  Q6_K: the row decode is 330
-// instructions, a tile 80: with a multiply-add per scale group and output
-// instead (430 per tile), 4096 x 14336 and 14336 x 4096, 512 tokens took 242 and
-// 213 us, now 164 and 163 (367 TOP/s).  Measured and dropped: four token tiles
-// (spills at two waves per SIMD: 189 us); each row tile's token tiles on one XCD
-// (160).
+// NT = 2 (390 with a minimum MFMA per sub-block and one token tile), 62% busy by
+// the counters, the matrix cores 37%; the waits are the barrier and the start of
+// each tile.  Gate and up of an 8B-class model, 28672 x 4096, 512 tokens in one
+// launch: 161 us (747 TOP/s); two launches of the one-tile kernel before, 244.
+// Q6_K: the row decode is 330 instructions, a tile 80: with a multiply-add per
+// scale group and output instead (430 per tile), 4096 x 14336 and 14336 x 4096,
+// 512 tokens took 242 and 213 us, now 164 and 163 (367 TOP/s).  Measured and
+// dropped: four token tiles (spills at two waves per SIMD: 189 us); each row
+// tile's token tiles on one XCD (160).
 typedef _Float16 rh_v8h __attribute__((ext_vector_type(8)));
 typedef float rh_v16f __attribute__((ext_vector_type(16)));
 typedef float rh_v4f __attribute__((ext_vector_type(4)));

@@ -1255,17 +1255,17 @@ static int gemm_kq_enqueue(const GemmMat *ms, int n, const BatchXq &b, int T, in
     // Q4_K: 64 tokens per workgroup where two such workgroups per CU remain (the
     // row decode is shared by two token tiles), 32 where three quarters of the CUs
     // get one, else K split over a workgroup's waves.  Measured, us: 28672 x 4096,
-    // 512 tokens: 173 with 64 tokens, 211 with 32; 4096 x 4096, 512 tokens (256 or
-    // 512 workgroups): 34 either way; 14336 x 4096, 37 tokens (112 or 224): 29 and
-    // 21.6, K split 27; 1024 x 4096, 512 tokens (128 with 32 tokens): K split 15.1,
-    // 20.5 with 32; 4096 x 4096, 64 tokens: 10.4 and 19.6.
+    // 512 tokens: 173 with 64 tokens, 207 with 32; 4096 x 4096, 512 tokens (256 or
+    // 512 workgroups): 35 either way; 14336 x 4096, 37 tokens (112 or 224): 30 and
+    // 22, K split 26; 1024 x 4096, 512 tokens (128 with 32 tokens): K split 14.9,
+    // 21.6 with 32; 4096 x 4096, 64 tokens: 10.6 and 20.8.
     // Q6_K: 32 tokens per workgroup where they give three quarters of the CUs
     // one, 64 once a CU would get a second, else K split.  us with 32 tokens, 64,
-    // K split: 14336 x 4096, 512 tokens (1792 or 896 workgroups) 223, 163, 338;
-    // 100 tokens (448 or 224) 69, 51, 89; 37 tokens (224 or 112) 42, 47, 51; 4096 x
-    // 14336, 512 tokens (512 or 256) 231, 164, 298; 256 tokens (256 or 128) 132,
-    // 150, 155; 150 tokens (160 or 96) 129, 148, 118; 1024 x 4096, 512 tokens (128
-    // or 64) 40, 47, 28.
+    // K split: 14336 x 4096, 512 tokens (1792 or 896 workgroups) 227, 165, 327;
+    // 100 tokens (448 or 224) 69, 50, 82; 37 tokens (224 or 112) 42, 47, 48; 4096 x
+    // 14336, 512 tokens (512 or 256) 239, 164, 281; 256 tokens (256 or 128) 135,
+    // 150, 141; 150 tokens (160 or 96) 129, 147, 105; 1024 x 4096, 512 tokens (128
+    // or 64) 41, 47, 26.
     // Up to 32 tokens a 64-token workgroup would only add padding.
     const int64_t wg1 = (int64_t)tiles * ((T + 31) / 32), wg2 = (int64_t)tiles * ((T + 63) / 64);
     const bool two = wg2 < wg1 && (q4 ? wg2 >= 2 * g.n_cu : wg1 > g.n_cu);
