@@ -1563,9 +1563,11 @@ __global__ __launch_bounds__(64 * C4_WAVES) void attn_exact_chain4_kernel(AttnEx
 // the next launch.
 //
 // The code (58 KB) starts at a multiple of 64 KB: its time depends on where it
-// lies, and without that on every kernel before it.  The same instructions took
-// 33.2 us per layer of an 8B model at 4096 positions at one place and 33.9 at
-// another (16 tokens through 6 layers 9.26, 9.33 or 9.39 ms; 9.26 so aligned).
+// lies, and without that on the size of every kernel before it.  The same
+// instructions at other places (offset in 64 KB), tok/s of the 8B-shape decode at
+// 4096 positions: 0x7900 385.8, 0x200 384.1, 0 383.6, 0xcf00 383.3, 0x8000 382.5,
+// 0xe000 381.6.  0 is not the best of them but the one that can be asked for;
+// gpt-oss-20b, whose full layers run the 64-wide form, is fastest there.
 template <int HD>
 __global__ __launch_bounds__(64 * C4_WAVES) __attribute__((aligned(65536))) void attn_exact_stream_kernel(
     AttnExactArgs A0) {

@@ -37,8 +37,8 @@ def test_expert_lists_use_no_scratch(kernels):
 
 
 def test_streamed_attention_code_starts_at_64_kb(tmp_path):
-    """Where the streamed attention's 58 KB of code lie changes its time by 2%,
-    so the place is fixed."""
+    """Where the streamed attention's 58 KB of code lie changes a decode's time
+    by up to 1%, so the place is fixed."""
     shutil.copy(os.path.join(ROOT, "rustyllm_amd", "librusty_hip.so"), tmp_path / "lib.so")
     subprocess.run([f"{LLVM}/llvm-objdump", "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
     obj = next(f for f in os.listdir(tmp_path) if f.endswith("gfx950"))
